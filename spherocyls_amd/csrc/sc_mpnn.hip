@@ -58,7 +58,6 @@ constexpr int kKo = 80;       // [h, 1, 0..]
 constexpr int kNo = 16;       // output width (3 used)
 constexpr int kEdgeFeat = 5;
 constexpr int kNodeFeat = 4;
-constexpr int kChunk = 2048;  // rows per weight-gradient partial
 // largest warm-start displacement per component (particle radii are ~0.5)
 constexpr float kCapXY = 1.0f;
 constexpr float kCapPhi = 0.5f;
@@ -165,53 +164,127 @@ __global__ void __launch_bounds__(256) k_gemm_nt(const bf16* __restrict__ A, int
 }
 
 // Partial weight gradients: P[chunk][K][N] = A[rows of chunk]^T . D[rows of
-// chunk], A row-major [M][lda] (K columns), D row-major [M][ldd] (N = NTN*16
-// columns).  One workgroup per chunk of kChunk rows; its four wavefronts share
-// the (K/16) x NTN output tiles.
-template <int NTN>
+// chunk], A row-major [M][lda] (K = KT*16 columns), D row-major [M][ldd] (N =
+// NTN*16 columns).  One workgroup per chunk of `chunk` rows (a multiple of
+// 32); its four wavefronts share the KT x NTN output tiles.
+//
+// The reduction runs down the rows, along which the operands are strided, so
+// a lane that loaded its own operand would read 16 two-byte values per MFMA
+// from 16 rows.  Instead a thread reads two neighbouring columns (4 bytes) of
+// 8 rows, a wavefront 256 contiguous bytes of each row, and packs them into
+// the two 16-byte operands those columns need; operands go through LDS
+// ([8 rows][column], read back as one ds_read_b128 per operand) in two buffers,
+// so a stage's loads are in flight while the previous stage multiplies.  What
+// bounds it is reading A and D once (416 B a row for the 144 x 64 maps).
+// 128000 edges, 144 x 64: 31 us (1.7 TB/s); 420 us with two-byte loads and 2048
+// rows per chunk (63 workgroups).
+template <int KT, int NTN>
 __global__ void __launch_bounds__(256) k_gemm_tn(const bf16* __restrict__ A, int lda,
-                                                  const bf16* __restrict__ D, int ldd, int M, int K,
-                                                  float* __restrict__ P) {
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int m_begin = blockIdx.x * kChunk;
-  const int m_end = min(M, m_begin + kChunk);
-  const int KT = K / 16;
-  const int ntiles = KT * NTN;
-  float* Pc = P + (size_t)blockIdx.x * K * NTN * 16;
-  const int kq = 4 * (lane >> 4);
-  for (int tile = wave; tile < ntiles; tile += 4) {
-    const int kt = tile / NTN, nt = tile % NTN;
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    // the reduction runs over rows m, 32 per MFMA: lane group g takes rows
-    // m0 + 8 g .. m0 + 8 g + 7 (rows past the chunk contribute zeros)
-    for (int m0 = m_begin; m0 < m_end; m0 += 32) {
-      s16x8 a, b;
+                                                  const bf16* __restrict__ D, int ldd, int M,
+                                                  int chunk, float* __restrict__ P) {
+  constexpr int kCols = (KT + NTN) * 16, kPairs = kCols / 2;
+  constexpr int kTasks = kPairs * 4;                // column pairs x groups of 8 rows
+  constexpr int kPer = (kTasks + 255) / 256;        // tasks per thread
+  constexpr int kTiles = KT * NTN, kAcc = (kTiles + 3) / 4;
+  __shared__ s16x8 s_op[2][4 * kCols];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m_begin = blockIdx.x * chunk, m_end = min(M, m_begin + chunk);
+  uint32_t raw[kPer][8];
+  auto load = [&](int m0) {
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int q = tid + 256 * k;
+      const int col = 2 * (q % kPairs), mg = q / kPairs;
+      const bool inA = col < KT * 16;
+      const bf16* base = inA ? A + col : D + (col - KT * 16);
+      const int ld = inA ? lda : ldd;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const int m = m0 + 2 * kq + i;
-        const bool ok = m < m_end;
-        // A operand = A^T tile: row (lane % 16) of the K block, column m
-        a[i] = ok ? (short)A[(size_t)m * lda + kt * 16 + (lane & 15)] : (short)0;
-        // B operand = D tile: row m, column (lane % 16) of the N block
-        b[i] = ok ? (short)D[(size_t)m * ldd + nt * 16 + (lane & 15)] : (short)0;
+        const int m = m0 + 8 * mg + i;
+        raw[k][i] = q < kTasks && m < m_end
+                        ? *reinterpret_cast<const uint32_t*>(base + (size_t)m * ld)
+                        : 0u;
       }
-      acc = mfma32(a, b, acc);
     }
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int q = tid + 256 * k;
+      if (q >= kTasks) continue;
+      const int col = 2 * (q % kPairs), mg = q / kPairs;
+      s16x8 lo, hi;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        lo[i] = (short)(raw[k][i] & 0xffffu);
+        hi[i] = (short)(raw[k][i] >> 16);
+      }
+      s_op[buf][mg * kCols + col] = lo;
+      s_op[buf][mg * kCols + col + 1] = hi;
+    }
+  };
+  f32x4 acc[kAcc];
+#pragma unroll
+  for (int t = 0; t < kAcc; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  load(m_begin);
+  int buf = 0;
+  for (int m0 = m_begin; m0 < m_end; m0 += 32, buf ^= 1) {
+    // the other buffer is still being read by slower wavefronts; this one was
+    // last read a stage earlier, before the previous barrier
+    store(buf);
+    __syncthreads();
+    if (m0 + 32 < m_end) load(m0 + 32);
+    const s16x8* op = s_op[buf] + (lane >> 4) * kCols + (lane & 15);
+#pragma unroll
+    for (int t = 0; t < kAcc; ++t) {
+      const int tile = wave + 4 * t;
+      if (tile < kTiles)
+        acc[t] = mfma32(op[(tile / NTN) * 16], op[(KT + tile % NTN) * 16], acc[t]);
+    }
+  }
+  float* Pc = P + (size_t)blockIdx.x * kTiles * 256;
+  const int kq = 4 * (lane >> 4);
+#pragma unroll
+  for (int t = 0; t < kAcc; ++t) {
+    const int tile = wave + 4 * t;
+    if (tile >= kTiles) continue;
+    const int kt = tile / NTN, nt = tile % NTN;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      Pc[(size_t)(kt * 16 + kq + i) * (NTN * 16) + nt * 16 + (lane & 15)] = acc[i];
+      Pc[(size_t)(kt * 16 + kq + i) * (NTN * 16) + nt * 16 + (lane & 15)] = acc[t][i];
   }
 }
 
-// G[i] (+)= sum over chunks of P[chunk][i], chunks in order.
-__global__ void k_sum_partials(const float* __restrict__ P, int nchunks, int size,
-                               float* __restrict__ G, int accumulate) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= size) return;
-  float s = accumulate ? G[i] : 0.0f;
-  for (int c = 0; c < nchunks; ++c) s += P[(size_t)c * size + i];
-  G[i] = s;
+// Rows per partial of a weight gradient over M rows: 256, so that a few tens of
+// thousands of rows already give every CU a workgroup, doubled while there
+// would be more than 512 partials (each K x N floats, written and read back).
+inline int chunk_rows(int M) {
+  int c = 256;
+  while ((M + c - 1) / c > 512) c *= 2;
+  return c;
+}
+constexpr int kMaxChunks = 512;
+
+// G[i] = sum over chunks of P[chunk][i].  A workgroup takes 32 elements; its 8
+// groups of 32 threads each sum a contiguous eighth of the chunks in order,
+// and the eight sums are added in order.  (One thread per element walks all
+// chunks in one dependent chain: 17 us for 63 chunks of 9216 elements.)
+__global__ void __launch_bounds__(256) k_sum_partials(const float* __restrict__ P, int nchunks,
+                                                       int size, float* __restrict__ G) {
+  __shared__ float s[256];
+  const int t = threadIdx.x, part = t >> 5, i = blockIdx.x * 32 + (t & 31);
+  const int per = (nchunks + 7) / 8, c0 = part * per, c1 = min(nchunks, c0 + per);
+  float v = 0.0f;
+  if (i < size)
+#pragma unroll 8
+    for (int c = c0; c < c1; ++c) v += P[(size_t)c * size + i];
+  s[t] = v;
+  __syncthreads();
+  if (t < 32 && i < size) {
+    float sum = s[t];
+    for (int k = 1; k < 8; ++k) sum += s[t + 32 * k];
+    G[i] = sum;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -751,8 +824,7 @@ void ensure_capacity(sc_mpnn* m, int n, int e) {
   realloc_dev(m, m->d_deg, nc + 1);
   realloc_dev(m, m->d_scan, (size_t)nc / 1024 + 2);
   if (!m->d_flag) m->d_flag = m->template dalloc<int>(1);
-  const size_t chunks = (size_t)std::max(nc, ec) / kChunk + 1;
-  m->pcap = chunks * kKe * kH;
+  m->pcap = (size_t)std::min(std::max(nc, ec) / 256 + 1, kMaxChunks) * kKe * kH;
   realloc_dev(m, m->P, m->pcap);
   realloc_dev(m, m->part, (size_t)blocks(nc) + 1);
   m->ncap = nc;
@@ -781,16 +853,15 @@ void gemm_nt(sc_mpnn* m, const bf16* A, int lda, const bf16* Bt, int ldb, int M,
                      A, lda, Bt, ldb, M, K, C, ldc, Hin, Hout, ldh);
 }
 
-template <int NTN>
-void gemm_tn(sc_mpnn* m, const bf16* A, int lda, const bf16* D, int ldd, int M, int K,
-             float* Gout) {
-  const int size = K * NTN * 16;
+template <int KT, int NTN>
+void gemm_tn(sc_mpnn* m, const bf16* A, const bf16* D, int M, float* Gout) {
+  const int size = KT * NTN * 256;
   if (M <= 0) return;
-  const int chunks = (M + kChunk - 1) / kChunk;
-  hipLaunchKernelGGL((k_gemm_tn<NTN>), dim3(chunks), dim3(256), 0, m->stream, A, lda, D, ldd, M, K,
-                     m->P);
-  hipLaunchKernelGGL(k_sum_partials, dim3(blocks((size_t)size)), dim3(256), 0, m->stream, m->P,
-                     chunks, size, Gout, 0);
+  const int chunk = chunk_rows(M), chunks = (M + chunk - 1) / chunk;
+  hipLaunchKernelGGL((k_gemm_tn<KT, NTN>), dim3(chunks), dim3(256), 0, m->stream, A, KT * 16, D,
+                     NTN * 16, M, chunk, m->P);
+  hipLaunchKernelGGL(k_sum_partials, dim3(blocks((size_t)size, 32)), dim3(256), 0, m->stream, m->P,
+                     chunks, size, Gout);
 }
 
 void forward(sc_mpnn* m) {
@@ -823,12 +894,12 @@ float backward(sc_mpnn* m) {
   const int nb = blocks(n);
   hipLaunchKernelGGL(k_loss, dim3(nb), dim3(256), 0, st, m->Y, m->T, n, m->dY, m->part);
   float* dloss = m->P;  // scratch for the reduced loss
-  hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(1), 0, st, m->part, nb, 1, dloss, 0);
+  hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, st, m->part, nb, 1, dloss);
   float loss = 0.0f;
   MPCK(hipMemcpyAsync(&loss, dloss, sizeof(float), hipMemcpyDeviceToHost, st));
   MPCK(hipStreamSynchronize(st));
   // decoder
-  gemm_tn<1>(m, m->Hin, kKo, m->dY, kNo, n, kKo, m->G + L.wo);
+  gemm_tn<kKo / 16, kNo / 16>(m, m->Hin, m->dY, n, m->G + L.wo);
   gemm_nt<5, kEpiStore>(m, m->dY, kNo, m->Wn + L.wo, kNo, n, kNo, m->dA, kKo);
   // gradient of the last hidden state: the h columns of dHin
   hipLaunchKernelGGL(k_take_cols, dim3(blocks((size_t)n * kH)), dim3(256), 0, st, m->dA, kKo, n,
@@ -839,12 +910,12 @@ float backward(sc_mpnn* m) {
     // node update: U = Uin . Wu, h_{l+1} = h_l + silu(U)
     hipLaunchKernelGGL(k_act_grad, dim3(blocks((size_t)n * kH)), dim3(256), 0, st, dH, kH, 0,
                        m->U[l], n, m->dPre);
-    gemm_tn<4>(m, m->Uin[l], kKu, m->dPre, kH, n, kKu, m->G + L.wu[l]);
+    gemm_tn<kKu / 16, kH / 16>(m, m->Uin[l], m->dPre, n, m->G + L.wu[l]);
     gemm_nt<9, kEpiStore>(m, m->dPre, kH, m->Wn + L.wu[l], kH, n, kH, m->dA, kKu);
     if (e > 0) {
       hipLaunchKernelGGL(k_edge_grad, dim3(blocks((size_t)e * kH)), dim3(256), 0, st, m->dA,
                          m->Z[l], m->dst, e, m->dPre);
-      gemm_tn<4>(m, m->Ein[l], kKe, m->dPre, kH, e, kKe, m->G + L.wm[l]);
+      gemm_tn<kKe / 16, kH / 16>(m, m->Ein[l], m->dPre, e, m->G + L.wm[l]);
       gemm_nt<9, kEpiStore>(m, m->dPre, kH, m->Wn + L.wm[l], kH, e, kH, m->dEin, kKe);
     } else {
       MPCK(hipMemsetAsync(m->G + L.wm[l], 0, sizeof(float) * kKe * kH, st));
@@ -856,7 +927,7 @@ float backward(sc_mpnn* m) {
   // encoder
   hipLaunchKernelGGL(k_act_grad, dim3(blocks((size_t)n * kH)), dim3(256), 0, st, dH, kH, 0, m->Ze,
                      n, m->dZe);
-  gemm_tn<4>(m, m->X, kKx, m->dZe, kH, n, kKx, m->G + L.we);
+  gemm_tn<kKx / 16, kH / 16>(m, m->X, m->dZe, n, m->G + L.we);
   return loss;
 }
 
