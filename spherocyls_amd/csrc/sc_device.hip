@@ -78,68 +78,6 @@ size_t tile_lds_bytes(int cap, int groups, int nthr) {
   return off;
 }
 
-// Minimiser decision for a packing from its reduced sums: the FIRE step
-// (velocity mixing or retreat, time step and mixing factor, convergence) or
-// the gradient-descent stop test.  S is the state the force pass evaluated.
-__device__ PackScal decide(const ReduceArgs& a, const PackInfo& P, const PackScal& S,
-                           const double* tot) {
-#pragma clang fp contract(off)
-  PackScal S2 = S;
-  const double frms = sqrt(tot[kSumR2] / (3.0 * P.n));
-  if (a.do_fire) {
-    const FireParams& fp = a.fire;
-    S2.frms = frms;
-    // Convergence is judged on FP64 pair forces only: a packing still on FP32
-    // pair math whose residual falls below max(switch_frms, ftol) moves to FP64
-    // and keeps iterating.
-    const bool fp32 = S.prec == kFP32;
-    if (!fp32 && frms < fp.ftol) {
-      S2.converged = 1;
-      S2.iters = S.step;
-    } else if (S.step >= (int)fp.max_iter) {
-      S2.converged = 2;
-      S2.iters = S.step;
-    } else {
-      double P_ = tot[kSumP], G_ = tot[kSumG], V_ = tot[kSumV];
-      double dt = S.fire_dt, alpha = S.fire_alpha, npos = S.fire_npos;
-      S2.fire_dt_old = dt;
-      if (P_ >= 0) {
-        S2.fire_mix = 1;
-        S2.fire_c_keep = 1.0 - alpha;
-        S2.fire_c_force = (G_ > 0) ? alpha * sqrt(V_ / G_) : 0.0;
-        npos += 1;
-        if (npos > fp.n_min) {
-          dt = fmin(dt * fp.f_inc, fp.dt_max);
-          alpha = alpha * fp.f_alpha;
-        }
-      } else {
-        S2.fire_mix = 0;
-        S2.fire_c_keep = 0;
-        S2.fire_c_force = 0;
-        dt = dt * fp.f_dec;
-        alpha = fp.alpha0;
-        npos = 0;
-      }
-      S2.fire_dt = dt;
-      S2.fire_dt_new = dt;
-      S2.fire_alpha = alpha;
-      S2.fire_npos = npos;
-      S2.step = S.step + 1;
-      if (fp32 && frms < fmax(fp.switch_frms, fp.ftol)) S2.prec = kFP64;
-    }
-  } else if (a.do_gd) {
-    // gradient-descent passes always record energy: E = tot[kSeE] / (2N)
-    S2.frms = frms;
-    if (tot[kSeE] * P.inv_2n <= a.fire.emin || S.step >= (int)a.fire.max_iter) {
-      S2.converged = 1;
-      S2.iters = S.step;
-    } else {
-      S2.step = S.step + 1;
-    }
-  }
-  return S2;
-}
-
 // Finalisation of the reduced sums of packing pk (one thread): stress/energy
 // records, and the minimiser decision into scal_next.
 __device__ void finalize_pack(const ReduceArgs& a, int pk, const PackInfo& P, const PackScal& S,
@@ -161,13 +99,17 @@ __device__ void finalize_pack(const ReduceArgs& a, int pk, const PackInfo& P, co
   ps[kSumG] = tot[kSumG];
   ps[kSumV] = tot[kSumV];
   ps[kSumR2] = tot[kSumR2];
-  if (a.do_fire || a.do_gd) a.scal_next[pk] = decide(a, P, S, tot);
+  if (a.do_fire || a.do_gd) {
+    const MinStep m = minimiser_step(a.fire, a.do_fire, P.n, P.inv_2n, S, tot[kSumR2], tot[kSumP],
+                                     tot[kSumG], tot[kSumV], tot[kSeE], true);
+    advance(a.scal_next[pk], S, m, a.do_fire);
+  }
 }
 
 // Sum packing pk's workgroup partials in workgroup order: thread t takes
 // partials t, t + nthr, ..., then the fixed-order block sum.  Every thread
 // calls it; the totals are in s_red[0 .. kNSum) afterwards.
-__device__ void reduce_partials(const ReduceArgs& a, int pk, double* s_red) {
+__device__ __forceinline__ void reduce_partials(const ReduceArgs& a, int pk, double* s_red) {
 #pragma clang fp contract(off)
   const int tid = threadIdx.x, nthr = blockDim.x;
   const int2 rg = a.ranges[pk];
@@ -310,7 +252,7 @@ __global__ void __launch_bounds__(256) k_tile(TileArgs a) {
     double ph = a.sphi[g];
     double Ai = a.b.A[g];
     double sn, cs;
-    sincos(ph, &sn, &cs);
+    rod_sincos(ph, &sn, &cs);
     L.x[dst] = a.sx[g];
     L.y[dst] = a.sy[g];
     L.nx[dst] = Ai * cs;
@@ -640,8 +582,7 @@ __global__ void k_bin_all(Bank b, const int* pack_of, const PackInfo* packs, con
 // rebuild flag when a particle leaves its skin/2 box around the build position.
 __global__ void __launch_bounds__(256) k_update(UpdateArgs u) {
 #pragma clang fp contract(off)
-  __shared__ double s_red[4 * kNSum];
-  __shared__ PackScal s_dec;
+  __shared__ double s_red[16];
   const Bank& b = u.b;
   const int tid = threadIdx.x;
   const int lin = blockIdx.x * blockDim.x + tid;
@@ -659,7 +600,7 @@ __global__ void __launch_bounds__(256) k_update(UpdateArgs u) {
     const int w = (ub.y - P.poff) >> 8, nw = (P.n + 255) >> 8, ncell = P.rows * P.cols;
     for (int c = w * 256 + tid; c < ncell; c += nw * 256) u.cnt_clear[P.coff + c] = 0;
   }
-  const PackScal S0 = u.red.scal[pk];
+  const PackScal& S0 = u.red.scal[pk];
   const bool lead = ub.y == P.poff;  // the packing's first workgroup stores the decision
   // A finished packing is left as it is: no move, no store, no binning.  Its
   // force passes return at once, and the buckets of every packing are filled
@@ -687,20 +628,71 @@ __global__ void __launch_bounds__(256) k_update(UpdateArgs u) {
     xbg = u.xb[gl];
     ybg = u.yb[gl];
   }
+  MinStep S;
   if (u.fused) {
-    reduce_partials(u.red, pk, s_red);
-    if (tid == 0) {
-      double fin[kNSum];
-      for (int i = 0; i < kNSum; ++i) fin[i] = s_red[i];
-      if (lead) finalize_pack(u.red, pk, P, S0, fin, records_se(u.red, S0));
-      s_dec = decide(u.red, P, S0, fin);
+    // The sums the decision needs (FIRE's four, or the energy), one barrier, and
+    // the decision by every thread for itself: what bounds the kernel is this
+    // serial chain, not its 30 words a particle.  With all 13 sums by shuffles
+    // and the decision by one thread it took 13.8 us for 16k particles and 30 us
+    // for 256 packings of 1024, against 6.8 and 14.5.
+    const bool fire = u.mode != 0;
+    const int2 rg = u.red.ranges[pk];
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+    for (int t = rg.x + tid; t < rg.x + rg.y; t += 256) {
+      const double* tp = u.red.part + (size_t)t * kNSum;
+      if (fire) {
+        s0 += tp[kSumR2];
+        s1 += tp[kSumP];
+        s2 += tp[kSumG];
+        s3 += tp[kSumV];
+      } else {
+        s0 += tp[kSeE];
+      }
     }
-  } else if (tid == 0) {
-    s_dec = u.red.scal_next[pk];
+    s0 = wave_sum(s0);
+    if (fire) {
+      s1 = wave_sum(s1);
+      s2 = wave_sum(s2);
+      s3 = wave_sum(s3);
+    }
+    if ((tid & 63) == 63) {
+      double* r = s_red + (tid >> 6) * 4;
+      r[0] = s0;
+      r[1] = s1;
+      r[2] = s2;
+      r[3] = s3;
+    }
+    __syncthreads();
+    s0 = s_red[0] + s_red[4] + s_red[8] + s_red[12];
+    if (fire) {
+      s1 = s_red[1] + s_red[5] + s_red[9] + s_red[13];
+      s2 = s_red[2] + s_red[6] + s_red[10] + s_red[14];
+      s3 = s_red[3] + s_red[7] + s_red[11] + s_red[15];
+    }
+    S = minimiser_step(u.red.fire, fire, P.n, P.inv_2n, S0, s0, s1, s2, s3, s0, false);
+    if (lead && tid == 0) {
+      advance(u.red.scal_next[pk], S0, S, fire);
+      double* ps = u.red.pack_sum + (size_t)pk * kNSum;
+      if (fire) {
+        ps[kSumR2] = s0;
+        ps[kSumP] = s1;
+        ps[kSumG] = s2;
+        ps[kSumV] = s3;
+      } else {
+        ps[kSeE] = s0 * P.inv_2n;
+      }
+    }
+  } else {
+    const PackScal& N = u.red.scal_next[pk];
+    S.end = N.converged;
+    S.mix = N.fire_mix;
+    S.c_keep = N.fire_c_keep;
+    S.c_force = N.fire_c_force;
+    S.dt_old = N.fire_dt_old;
+    S.dt = N.fire_dt_new;
   }
-  __syncthreads();
-  const PackScal S = s_dec;
-  if (S.converged) return;  // converged at the state just evaluated
+  if (S.end) return;  // finished at the state just evaluated
+  const double Lx = S0.Lx, Ly = S0.Ly;
   int bin_c = -1;
   if (own) {
     if (u.mode == 0) {
@@ -709,20 +701,20 @@ __global__ void __launch_bounds__(256) k_update(UpdateArgs u) {
       y += dt * Fy;
       p += dt * Tq / Ig;
     } else {
-      double sq = sqrt(Ig);
-      double gx = Fx, gy = Fy, gp = Tq / sq;
+      const double isq = 1.0 / sqrt(Ig);
+      double gx = Fx, gy = Fy, gp = Tq * isq;
       double ux, uy, up;
-      if (S.fire_mix) {
-        ux = S.fire_c_keep * vx + S.fire_c_force * gx;
-        uy = S.fire_c_keep * vy + S.fire_c_force * gy;
-        up = S.fire_c_keep * vp + S.fire_c_force * gp;
+      if (S.mix) {
+        ux = S.c_keep * vx + S.c_force * gx;
+        uy = S.c_keep * vy + S.c_force * gy;
+        up = S.c_keep * vp + S.c_force * gp;
       } else {
-        x -= 0.5 * S.fire_dt_old * vx;
-        y -= 0.5 * S.fire_dt_old * vy;
-        p -= 0.5 * S.fire_dt_old * vp / sq;
+        x -= 0.5 * S.dt_old * vx;
+        y -= 0.5 * S.dt_old * vy;
+        p -= 0.5 * S.dt_old * vp * isq;
         ux = uy = up = 0.0;
       }
-      double dtn = S.fire_dt_new;
+      const double dtn = S.dt;
       ux += dtn * gx;
       uy += dtn * gy;
       up += dtn * gp;
@@ -738,21 +730,21 @@ __global__ void __launch_bounds__(256) k_update(UpdateArgs u) {
       }
       x += mx;
       y += my;
-      p += dtn * up / sq;
+      p += dtn * up * isq;
     }
-    bool okx = wrap_coord(x, S.Lx), oky = wrap_coord(y, S.Ly);
+    bool okx = wrap_coord(x, Lx), oky = wrap_coord(y, Ly);
     if (!okx || !oky || !isfinite(p)) atomicOr(u.err, kErrNonFinite);
     b.x[g] = x;
     b.y[g] = y;
     b.phi[g] = p;
     double sn, cs;
-    sincos(p, &sn, &cs);
+    rod_sincos(p, &sn, &cs);
     b.nx[g] = Ag * cs;
     b.ny[g] = Ag * sn;
-    bin_c = cell_of(x, y, S.Lx, S.Ly, P);
+    bin_c = cell_of(x, y, Lx, Ly, P);
     if (u.flag_out) {
       const double hs = 0.5 * P.pad;  // list skin = the packing's cell padding
-      if (fabs(min_image(x - xbg, S.Lx)) >= hs || fabs(min_image(y - ybg, S.Ly)) >= hs)
+      if (fabs(min_image(x - xbg, Lx)) >= hs || fabs(min_image(y - ybg, Ly)) >= hs)
         u.flag_out[pk] = 1;
     }
   }
@@ -763,7 +755,7 @@ __global__ void __launch_bounds__(256) k_update(UpdateArgs u) {
 // convergence (or max_iter), in one launch.  An iteration is the force pass,
 // the reduction and decision, and the update of the two-launch path (k_list
 // force pass, k_update), with the same formulas and the same FIRE state
-// machine (decide); only the order of the sums differs.  Nothing of an
+// machine (minimiser_step); only the order of the sums differs.  Nothing of an
 // iteration touches global memory: the packing's coordinates, segment vectors,
 // radii, half lengths, ids, rows and forces live in LDS, and each particle's
 // angle, velocity and build position in the registers of the thread that
@@ -952,10 +944,9 @@ __global__ void __launch_bounds__(kSmallThreads) k_fire_small(SmallFireArgs a) {
         tot[kSumG] += s_part[w * kFire + 2];
         tot[kSumV] += s_part[w * kFire + 3];
       }
-      ReduceArgs ra{};
-      ra.fire = fp;
-      ra.do_fire = 1;
-      s_S = decide(ra, P, S, tot);
+      const MinStep m = minimiser_step(fp, true, n, P.inv_2n, S, tot[kSumR2], tot[kSumP],
+                                       tot[kSumG], tot[kSumV], 0.0, true);
+      advance(s_S, S, m, true);
       s_rebuild = 0;  // every thread read it before the barriers above
     }
     __syncthreads();  // decision visible
@@ -998,7 +989,7 @@ __global__ void __launch_bounds__(kSmallThreads) k_fire_small(SmallFireArgs a) {
         s_stop = 1;
       }
       double sn, cs;
-      sincos(phi, &sn, &cs);
+      rod_sincos(phi, &sn, &cs);
       s_x[tid] = x;
       s_y[tid] = y;
       s_nx[tid] = Au * cs;

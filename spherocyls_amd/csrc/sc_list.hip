@@ -330,14 +330,9 @@ __global__ void __launch_bounds__(256)
       }
       if (k0 >= n) break;
     }
-    if (LANES > 1) {
-#pragma unroll
-      for (int off = LANES >> 1; off > 0; off >>= 1) {
-        Fx += __shfl_xor(Fx, off);
-        Fy += __shfl_xor(Fy, off);
-        Tq += __shfl_xor(Tq, off);
-      }
-    }
+    Fx = group_sum(Fx, LANES);
+    Fy = group_sum(Fy, LANES);
+    Tq = group_sum(Tq, LANES);
     // ---- per-particle epilogue (lane 0)
     const double half_skin = 0.5 * P.pad;
     // build position of the row (written above by this lane when it rebuilt
@@ -404,7 +399,7 @@ __global__ void __launch_bounds__(256)
       a.py[g] = qy;
       a.pphi[g] = qp;
       double sn, cs;
-      sincos(qp, &sn, &cs);
+      rod_sincos(qp, &sn, &cs);
       a.pnx[g] = Ai * cs;
       a.pny[g] = Ai * sn;
       a.v0x[g] = v0x;
@@ -479,7 +474,7 @@ __global__ void __launch_bounds__(256)
       a.b.y[g] = y1;
       a.b.phi[g] = p1;
       double sn, cs;
-      sincos(p1, &sn, &cs);
+      rod_sincos(p1, &sn, &cs);
       a.b.nx[g] = Ai * cs;
       a.b.ny[g] = Ai * sn;
       bin_into(g, x1, y1, Lbx, Lby, P, a.cnt_fill, a.slot_fill, a.err);
@@ -493,12 +488,10 @@ __global__ void __launch_bounds__(256)
 
   // ---- scalar advance (corrector: one thread per packing)
   if (MODE == kModeCorr && g == P.poff && lane == 0) {
-    // copied word by word and updated in place: the struct never lives in
-    // registers across the kernel (it would spill)
-    const int* src = reinterpret_cast<const int*>(&a.scal[pk]);
-    int* dst = reinterpret_cast<int*>(&a.scal_next[pk]);
-    for (int w = 0; w < (int)(sizeof(PackScal) / sizeof(int)); ++w) dst[w] = src[w];
-    PackScal& S2 = a.scal_next[pk];
+    // read again here, so that the struct is not live across the kernel, and in
+    // one piece: copied word by word, this thread waited for memory 30 times
+    // (2.3 of 9.6 us of the pass at N = 512)
+    PackScal S2 = a.scal[pk];
     S2.step = S2.step + 1;
     if (box_pure) {
       S2.Lx = L_new_x;
@@ -517,12 +510,20 @@ __global__ void __launch_bounds__(256)
       S2.Lx = L_new_x;
       S2.Ly = L_new_y;
     }
+    a.scal_next[pk] = S2;
   }
 
   if constexpr (kSums) {
     if (!do_sum) return;
-    block_sum<kNSum>(acc, s_red, nthr);
-    if (tid < kNSum) a.part[(size_t)bslot * kNSum + tid] = s_red[tid];
+    if constexpr (SE) {
+      block_sum<kNSum>(acc, s_red, nthr);
+      if (tid < kNSum) a.part[(size_t)bslot * kNSum + tid] = s_red[tid];
+    } else {  // the residual and FIRE's sums
+      double v[4] = {acc[kSumP], acc[kSumG], acc[kSumV], acc[kSumR2]};
+      static_assert(kSumP == 9 && kSumG == 10 && kSumV == 11 && kSumR2 == 12, "last four sums");
+      block_sum<4>(v, s_red, nthr);
+      if (tid < 4) a.part[(size_t)bslot * kNSum + kSumP + tid] = s_red[tid];
+    }
   }
 }
 
@@ -550,7 +551,7 @@ __global__ void k_segvec(Bank b, int ntot) {
   int g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= ntot) return;
   double sn, cs;
-  sincos(b.phi[g], &sn, &cs);
+  rod_sincos(b.phi[g], &sn, &cs);
   b.nx[g] = b.A[g] * cs;
   b.ny[g] = b.A[g] * sn;
 }

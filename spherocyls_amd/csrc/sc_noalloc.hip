@@ -160,7 +160,7 @@ __global__ void k_na_prepare(unsigned char* base, int n, const double* x, const 
   at<double>(base, kLay.x)[g] = x[g];
   at<double>(base, kLay.y)[g] = y[g];
   double sn, cs;
-  sincos(phi[g], &sn, &cs);
+  rod_sincos(phi[g], &sn, &cs);
   at<double>(base, kLay.nx)[g] = A[g] * cs;
   at<double>(base, kLay.ny)[g] = A[g] * sn;
   at<int>(base, kLay.id)[g] = g;

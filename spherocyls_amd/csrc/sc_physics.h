@@ -87,6 +87,41 @@ __device__ __forceinline__ bool segments_cross(T ddx, T ddy, T nxA, T nyA, T nxB
          ((gp > T(0) && gm < T(0)) || (gp < T(0) && gm > T(0)));
 }
 
+// Division x / d with a reciprocal that several quotients share.  r =
+// reciprocal(d) is the hardware estimate after two Newton steps; the quotient's
+// residual is corrected once by fused multiply-adds, which rounds it
+// correctly (Markstein) as the compiler's own division sequence does, in 3
+// instructions instead of 11 and without its scaling for operands near the
+// ends of the exponent range, which lengths and forces do not come near.
+// d = 0 gives NaN, also for x != 0: used only where x = 0 then (a disc's
+// squared half length), or d > 0.  The pair math is a chain of dependent FP64
+// operations (a division is 70 cycles of latency, this 20): 262k particles
+// sheared by 100 steps, 7.97 -> 7.59 ms together with root() below.
+__device__ __forceinline__ double reciprocal(double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  r = fma(fma(-d, r, 1.0), r, r);
+  return fma(fma(-d, r, 1.0), r, r);
+}
+__device__ __forceinline__ double over(double x, double d, double r) {
+  const double q = x * r;
+  return fma(fma(-d, q, x), r, q);
+}
+
+// sqrt(v) for v > 0 away from the ends of the exponent range, and a reciprocal
+// of it for over(): the compiler's sequence without its scaling.
+__device__ __forceinline__ double root(double v, double& rinv) {
+  const double y = __builtin_amdgcn_rsq(v);
+  double g = v * y, h = 0.5 * y;
+  const double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  g = fma(fma(-g, g, v), h, g);
+  g = fma(fma(-g, g, v), h, g);
+  rinv = h + h;
+  rinv = fma(fma(-g, rinv, 1.0), rinv, rinv);
+  return g;
+}
+
 // Segment-segment closest approach and harmonic contact force, following
 // calc_force_pair (src/cpp/strain_dynamics.cpp:38-64) term by term.  Returns
 // false when |D| >= sigma (or D is NaN).  FP64: no contraction, so the rounding
@@ -103,10 +138,10 @@ __device__ __forceinline__ bool pair_contact_f64(double ddx, double ddy, double 
   double det = a * c - b * b;
   double tu = (b * d - a * e) / det;
   double t = fmin(fmax(tu, -1.0), 1.0);
-  double s = -(b * t + d) / a;
+  double s = over(-(b * t + d), a, reciprocal(a));
   double sabs = fabs(s);
   s = fmin(fmax(s, -1.0), 1.0);
-  if (sabs > 1.0) t = fmin(fmax(-(b * s + e) / c, -1.0), 1.0);
+  if (sabs > 1.0) t = fmin(fmax(over(-(b * s + e), c, reciprocal(c)), -1.0), 1.0);
   double Dx = ddx + s * nxA - t * nxB;
   double Dy = ddy + s * nyA - t * nyB;
   double d2 = Dx * Dx + Dy * Dy;
@@ -126,10 +161,11 @@ __device__ __forceinline__ bool pair_contact_f64(double ddx, double ddy, double 
     o.dV = 1.0 / sig;
     return true;
   }
-  double dist = sqrt(d2);
-  double dV = (1.0 - dist / sig) / sig;
-  double fx = Dx * dV / dist;
-  double fy = Dy * dV / dist;
+  double rd, rs = reciprocal(sig);
+  double dist = root(d2, rd);
+  double dV = over(1.0 - over(dist, sig, rs), sig, rs);
+  double fx = over(Dx * dV, dist, rd);
+  double fy = over(Dy * dV, dist, rd);
   o.fx = fx;
   o.fy = fy;
   o.tp = s * nxA * fy - s * nyA * fx;
@@ -163,10 +199,19 @@ __device__ __forceinline__ bool contact_point(T Dx, T Dy, T s, T t, T nxA, T nyA
     o.dV = T(1) / sig;
     return true;
   }
-  T dist = sqrt(d2);
-  T dV = (T(1) - dist / sig) / sig;
-  T fx = Dx * dV / dist;
-  T fy = Dy * dV / dist;
+  T dist, dV, fx, fy;
+  if constexpr (sizeof(T) == sizeof(double)) {
+    double rd, rs = reciprocal(sig);
+    dist = root(d2, rd);
+    dV = over(1.0 - over(dist, sig, rs), sig, rs);
+    fx = over(Dx * dV, dist, rd);
+    fy = over(Dy * dV, dist, rd);
+  } else {
+    dist = sqrt(d2);
+    dV = (T(1) - dist / sig) / sig;
+    fx = Dx * dV / dist;
+    fy = Dy * dV / dist;
+  }
   o.fx = fx;
   o.fy = fy;
   o.tp = s * nxA * fy - s * nyA * fx;
@@ -247,45 +292,38 @@ __device__ __forceinline__ void pair_contacts_2p(double ddx, double ddy, double 
     t3 = t2;
   } else {
     const double tu = (b * d - a * e) / det;
+    const double ra = reciprocal(a), rc = reciprocal(c);
     t1 = clamp1(tu);
-    s1 = -(b * t1 + d) / a;
-    double sarg = fabs(s1);
+    s1 = over(-(b * t1 + d), a, ra);
+    const double sarg = fabs(s1);
     s1 = clamp1(s1);
     crossed = fabs(tu) < 1.0 && sarg < 1.0 && segments_cross(ddx, ddy, nxA, nyA, nxB, nyB);
-    if (sarg >= 1.0) {
-      t1 = clamp1(-(b * s1 + e) / c);
-      s2 = -s1;
-      t2 = -(b * s2 + e) / c;
-      double targ = fabs(t2);
-      t2 = clamp1(t2);
-      if (targ > 1.0) {
-        s2 = clamp1(-(b * t2 + d) / a);
-        s3 = s2;
-        t3 = t2;
-      } else {
-        t3 = b < 0.0 ? -s1 : s1;
-        s3 = -(b * t3 + d) / a;
-        sarg = fabs(s3);
-        s3 = clamp1(s3);
-        if (sarg >= 1.0) t3 = clamp1(-(b * s3 + e) / c);
-      }
-    } else {
-      t2 = -t1;
-      s2 = -(b * t2 + d) / a;
-      sarg = fabs(s2);
-      s2 = clamp1(s2);
-      if (sarg > 1.0) {
-        t2 = clamp1(-(b * s2 + e) / c);
-        s3 = s2;
-        t3 = t2;
-      } else {
-        s3 = b < 0.0 ? -t1 : t1;
-        t3 = -(b * s3 + e) / c;
-        double targ = fabs(t3);
-        t3 = clamp1(t3);
-        if (targ >= 1.0) s3 = clamp1(-(b * t3 + d) / a);
-      }
+    // The rod whose end (u1 = +-1) fixed the first contact, A if s1 was clamped
+    // and else B (whose t1 was): its parameters are u, the other rod's v.  The
+    // two cases mirror each other, so both run the same instructions.
+    const bool endA = sarg >= 1.0;
+    if (endA) t1 = clamp1(over(-(b * s1 + e), c, rc));
+    const double u1 = endA ? s1 : t1;
+    const double nu = endA ? d : e, du = endA ? a : c, ru = endA ? ra : rc;
+    const double nv = endA ? e : d, dv = endA ? c : a, rv = endA ? rc : ra;
+    double u2 = -u1;
+    double v2 = over(-(b * u2 + nv), dv, rv);
+    const bool beyond = fabs(v2) > 1.0;
+    v2 = clamp1(v2);
+    // one division serves u2 (the second contact beyond v's end) or u3
+    double v3 = b < 0.0 ? -u1 : u1;
+    const double uq = over(-(b * (beyond ? v2 : v3) + nu), du, ru);
+    double u3 = clamp1(uq);
+    if (beyond) {
+      u2 = u3;
+      v3 = v2;
+    } else if (fabs(uq) >= 1.0) {
+      v3 = clamp1(over(-(b * u3 + nv), dv, rv));
     }
+    s2 = endA ? u2 : v2;
+    t2 = endA ? v2 : u2;
+    s3 = endA ? u3 : v3;
+    t3 = endA ? v3 : u3;
   }
   h0 = contact_point<T>(T(ddx + s1 * nxA - t1 * nxB), T(ddy + s1 * nyA - t1 * nyB), T(s1), T(t1),
                         T(nxA), T(nyA), T(nxB), T(nyB), T(sig), crossed, T(ddx), T(ddy), o0);
@@ -365,6 +403,27 @@ __device__ __forceinline__ void add_contact_sums(const PairOut<double>& r, doubl
   acc[kSeCPyx] += r.fx * (cya - cyb);
 }
 
+// Sine and cosine of a rod's angle.  The test makes the library's reduction
+// for huge arguments unreachable, so its code, constants and registers leave
+// every kernel that moves particles (moving a particle of a one-launch FIRE:
+// 3100 -> 1200 cycles); values are the library's.  An angle of 2^20 or more (a
+// rod that turned 166 thousand times) first loses its whole turns, by multiples
+// of 2 pi held in two words: within 1e-12 up to 1e19, where the angle's own
+// last bit is many turns, and finite beyond.
+__device__ __forceinline__ void rod_sincos(double x, double* sn, double* cs) {
+  double r = x;
+  for (int i = 0; i < 24 && !(fabs(r) < 1048576.0); ++i) {
+    const double k = rint(r * 0.15915494309189535);
+    r = fma(-k, 2.4492935982947064e-16, fma(-k, 6.283185307179586, r));
+  }
+  if (fabs(r) < 1048576.0) {
+    sincos(r, sn, cs);
+  } else {  // not finite
+    *sn = r - r;
+    *cs = 1.0 + *sn;
+  }
+}
+
 // Minimum image in sheared coordinates (src/cpp/strain_dynamics.cpp:28-29).
 __device__ __forceinline__ double min_image(double d, double L) {
 #pragma clang fp contract(off)
@@ -374,6 +433,7 @@ __device__ __forceinline__ double min_image(double d, double L) {
 // Wrap rule of find_cells (src/cpp/spherocyl_box.cpp:279-286); bounded so a
 // runaway coordinate cannot spin.  Returns false for a non-finite coordinate.
 __device__ __forceinline__ bool wrap_coord(double& v, double L) {
+  if (v >= 0.0 && v <= L) return true;
   if (!isfinite(v)) return false;
   int guard = 0;
   while (v > L && guard < 8) { v -= L; ++guard; }
@@ -515,27 +575,176 @@ __device__ __forceinline__ void pair_into(double xi, double yi, double nxi, doub
   }
 }
 
+// What a minimiser does after a force pass, from its packing's sums: the FIRE
+// step (velocity mixing or retreat, time step and mixing factor, convergence)
+// or the gradient-descent stop test.  Cheap enough that every wavefront that
+// moves particles takes it for itself.
+struct MinStep {
+  double dt_old, dt, alpha, npos;  // FIRE: time step before and after, mixing factor, uphill count
+  double c_keep, c_force;          // FIRE: velocity = c_keep v + c_force g (mix), or a retreat
+  double frms;                     // set where it can end the run (or with `residual`)
+  int mix, prec;
+  int end;                         // 0: go on, 1: converged, 2: FIRE at max_iter
+};
+
+// S: the scalars the force pass evaluated; R2, Pw, G, V: FIRE's sums; E: the
+// gradient descent's energy sum.  residual: frms is wanted in any case.
+__device__ __forceinline__ MinStep minimiser_step(const FireParams& fp, bool do_fire, int n,
+                                                  double inv_2n, const PackScal& S, double R2,
+                                                  double Pw, double G, double V, double E,
+                                                  bool residual) {
+#pragma clang fp contract(off)
+  MinStep m;
+  const int step = S.step;
+  const bool last = step >= (int)fp.max_iter;
+  double dt = S.fire_dt, alpha = S.fire_alpha, npos = S.fire_npos;
+  m.dt_old = dt;
+  m.c_keep = m.c_force = m.frms = 0.0;
+  m.mix = m.end = 0;
+  m.prec = S.prec;
+  if (do_fire) {
+    // Convergence is judged on FP64 pair forces only: a packing still on FP32
+    // pair math whose residual falls below max(switch_frms, ftol) moves to FP64
+    // and keeps iterating.  The root is taken only where F_rms may be below a
+    // limit (its square times 3 N, with room for rounding and underflow).
+    const bool fp32 = m.prec == kFP32;
+    const double lim = fp32 ? fmax(fp.switch_frms, fp.ftol) : fp.ftol;
+    if (residual || last || R2 <= lim * lim * (3.0 * n) * (1.0 + 1e-9) + 1e-300) {
+      m.frms = sqrt(R2 / (3.0 * n));
+      if (!fp32 && m.frms < fp.ftol) m.end = 1;
+      else if (last) m.end = 2;
+      else if (fp32 && m.frms < lim) m.prec = kFP64;
+    }
+    if (Pw >= 0) {
+      m.mix = 1;
+      m.c_keep = 1.0 - alpha;
+      m.c_force = (G > 0) ? alpha * sqrt(V / G) : 0.0;
+      npos += 1;
+      if (npos > fp.n_min) {
+        dt = fmin(dt * fp.f_inc, fp.dt_max);
+        alpha = alpha * fp.f_alpha;
+      }
+    } else {
+      dt = dt * fp.f_dec;
+      alpha = fp.alpha0;
+      npos = 0;
+    }
+  } else {
+    // gradient-descent passes always record energy: E / (2N)
+    if (residual) m.frms = sqrt(R2 / (3.0 * n));
+    if (E * inv_2n <= fp.emin || last) m.end = 1;
+  }
+  m.dt = dt;
+  m.alpha = alpha;
+  m.npos = npos;
+  return m;
+}
+
+// The scalars after that step (the storing thread).
+__device__ __forceinline__ void advance(PackScal& S1, const PackScal& S0, const MinStep& m,
+                                        bool do_fire) {
+  S1 = S0;
+  if (m.end) {
+    S1.frms = m.frms;
+    S1.converged = m.end;
+    S1.iters = S0.step;
+    return;
+  }
+  S1.step = S0.step + 1;
+  if (!do_fire) return;
+  S1.fire_dt = m.dt;
+  S1.fire_alpha = m.alpha;
+  S1.fire_npos = m.npos;
+  S1.prec = m.prec;
+  // read by the update kernel when k_reduce took the decision
+  S1.fire_mix = m.mix;
+  S1.fire_c_keep = m.c_keep;
+  S1.fire_c_force = m.c_force;
+  S1.fire_dt_old = m.dt_old;
+  S1.fire_dt_new = m.dt;
+}
+
 // ---------------------------------------------------------------------------
 // block reduction helpers (fixed order -> deterministic)
 // ---------------------------------------------------------------------------
+// Sum over the wavefront's 64 lanes, valid in lane 63.  Data-parallel-primitive
+// moves (rows of 16 lanes, then the row broadcasts) cost VALU issue only; the
+// same tree by shuffles is six LDS round trips.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+  const long long u = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)u, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), CTRL, ROWS, 0xf, false);
+  return v + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double wave_sum(double v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr:1
+  v = dpp_add<0x112, 0xf>(v);  // row_shr:2
+  v = dpp_add<0x114, 0xf>(v);  // row_shr:4
+  v = dpp_add<0x118, 0xf>(v);  // row_shr:8
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v = dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
+// Sum over the L lanes (1, 2, 4 or 8, aligned) that share a particle, in all of
+// them, as the tree lane ^ 4, ^ 2, ^ 1.  Data-parallel-primitive moves instead
+// of shuffles, which are LDS round trips: lanes four apart by row shifts (a
+// half row's lower bank takes the upper one's values and the other way), then
+// quad permutes.
+__device__ __forceinline__ int dpp_xor4(int v) {
+  const int up = __builtin_amdgcn_update_dpp(v, v, 0x104, 0xf, 0x5, false);   // row_shl:4
+  return __builtin_amdgcn_update_dpp(up, v, 0x114, 0xf, 0xa, false);          // row_shr:4
+}
+template <int CTRL>
+__device__ __forceinline__ int dpp_quad(int v) {
+  return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false);
+}
+__device__ __forceinline__ double group_sum(double v, int L) {
+  auto join = [](int lo, int hi) {
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+  };
+  if (L >= 8) {
+    const long long u = __double_as_longlong(v);
+    v += join(dpp_xor4((int)u), dpp_xor4((int)(u >> 32)));
+  }
+  if (L >= 4) {  // lanes 2 3 0 1
+    const long long u = __double_as_longlong(v);
+    v += join(dpp_quad<0x4e>((int)u), dpp_quad<0x4e>((int)(u >> 32)));
+  }
+  if (L >= 2) {  // lanes 1 0 3 2
+    const long long u = __double_as_longlong(v);
+    v += join(dpp_quad<0xb1>((int)u), dpp_quad<0xb1>((int)(u >> 32)));
+  }
+  return v;
+}
+
+// The value in lane 63, as a scalar.
+__device__ __forceinline__ double last_lane(double v) {
+  const long long u = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)u, 63);
+  const int hi = __builtin_amdgcn_readlane((int)(u >> 32), 63);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// Sums of v over the workgroup in wavefront order, in s_red[0 .. NV) for every
+// thread.
 template <int NV>
 __device__ __forceinline__ void block_sum(double (&v)[NV], double* s_red, int nthr) {
   const int tid = threadIdx.x;
+  const int w = tid >> 6, nw = nthr >> 6;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    double x = v[i];
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
-    v[i] = x;
+    const double x = wave_sum(v[i]);
+    if ((tid & 63) == 63) s_red[w * NV + i] = x;
   }
-  const int w = tid >> 6, nw = nthr >> 6;
-  if ((tid & 63) == 0)
-#pragma unroll
-    for (int i = 0; i < NV; ++i) s_red[w * NV + i] = v[i];
-  __syncthreads();
-  if (tid < NV) {
-    double x = 0;
-    for (int k = 0; k < nw; ++k) x += s_red[k * NV + tid];
-    s_red[tid] = x;  // each slot tid is read (k = 0) before this write by the same thread
+  if (nw > 1) {
+    __syncthreads();
+    if (tid < NV) {
+      double x = 0;
+      for (int k = 0; k < nw; ++k) x += s_red[k * NV + tid];
+      s_red[tid] = x;  // each slot tid is read (k = 0) before this write by the same thread
+    }
   }
   __syncthreads();
 }
