@@ -118,16 +118,18 @@ int sc_set_contact_model(sc_system* s, int model);
  * are identical; graphs cut launch overhead for small systems.  Event timing
  * (sc_timing_enable) always launches eagerly. */
 int sc_set_graphs(sc_system* s, int enable);
-/* FIRE of small packings in one launch (no reference counterpart; a launch
- * choice like sc_set_graphs).  On the list path, once every packing that
- * sc_fire_minimize still advances holds at most max_particles particles
- * (0 <= max_particles <= 256; default 256, 0 = never), one workgroup per
- * packing runs the remaining iterations inside a single kernel: same
- * iteration, decisions and stop rule, sums in another order (results agree
- * to rounding, not bit for bit).  A launch runs at most steps_per_launch
- * iterations (0: the default, 50000) and the packings still running are
- * launched again, so no single kernel runs long.  With event timing on, that
- * kernel is counted under SC_KERNEL_FIRE_FORCE. */
+/* Many steps in one launch (no reference counterpart; a launch choice like
+ * sc_set_graphs).  max_particles > 0 (at most 256; the default) lets teams of
+ * workgroups that stay resident run FIRE iterations, gradient-descent steps and
+ * the sheared steps of a single packing on the list path, wherever the
+ * workgroups of all packings still running fit the GPU together (a single
+ * packing of about 60 thousand particles does); 0 launches kernels for every
+ * step.  Same steps, decisions and stop rules, sums in another order: results
+ * agree to rounding, not bit for bit.  A launch of a minimiser runs at most
+ * steps_per_launch iterations (0: the default, 50000) and the packings still
+ * running are launched again, so no single kernel runs long.  With event timing
+ * on, a minimiser's launch is counted under SC_KERNEL_FIRE_FORCE; sheared steps
+ * are then launched one by one. */
 int sc_set_small_fire(sc_system* s, int max_particles, int steps_per_launch);
 int sc_get_contact_model(const sc_system* s, int* model);
 /* Force-pass implementation (no reference counterpart; both give the same

@@ -33,7 +33,14 @@ HIP_FLAGS = [
 ]
 CXX_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-I", os.path.join(ROOT, "include")]
 
-HIP_SOURCES = ["sc_device.hip", "sc_list.hip", "sc_api.hip", "sc_mpnn.hip", "sc_noalloc.hip"]
+HIP_SOURCES = ["sc_device.hip", "sc_list.hip", "sc_api.hip", "sc_mpnn.hip", "sc_noalloc.hip",
+               "sc_team.hip"]
+# The team kernel is one loop around a whole step: hoisting what is invariant in
+# it (addresses of LDS arrays, constants of the sine) into registers held across
+# the loop makes it spill, so that motion is off there.
+EXTRA_HIP_FLAGS = {
+    "sc_team.hip": ["-mllvm", "-disable-machine-licm", "-mllvm", "-sink-insts-to-avoid-spills"],
+}
 CXX_SOURCES = [os.path.join(CSRC, "sc_configgen.cpp")]
 HOST_LIB_SOURCES = ["spherocyl_box.cpp", "dat_file.cpp"]
 DRIVERS = {
@@ -61,7 +68,8 @@ def build(verbose: bool = False) -> str:
     objs = []
     for src in HIP_SOURCES:
         obj = os.path.join(BUILD, src.replace(".hip", ".o"))
-        _run([HIPCC, *HIP_FLAGS, "-c", os.path.join(CSRC, src), "-o", obj], verbose)
+        _run([HIPCC, *HIP_FLAGS, *EXTRA_HIP_FLAGS.get(src, []), "-c", os.path.join(CSRC, src),
+              "-o", obj], verbose)
         objs.append(obj)
     host_srcs = list(CXX_SOURCES)
     host_srcs += [os.path.join(HOST, f) for f in HOST_LIB_SOURCES

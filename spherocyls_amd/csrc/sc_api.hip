@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -26,8 +27,6 @@ __global__ void k_segvec(Bank b, int ntot);
 __global__ void k_bin_all(Bank b, const int* pack_of, const PackInfo* packs, const PackScal* scal,
                           int* cnt, int* slot, int* err, int ntot, int wrap_angles);
 __global__ void k_update(UpdateArgs u);
-template <bool TWO_POINT, bool MIXED>
-__global__ void k_fire_small(SmallFireArgs a);
 __global__ void k_affine(Bank b, const int* pack_of, const double* scale, int ntot, int y_only);
 __global__ void k_scan_cells(const PackInfo* packs, const int* cnt, int* cstart);
 __global__ void k_sort_cells(const int* cstart, int* cnt, int* slot, const int* id, int* perm,
@@ -40,6 +39,12 @@ __global__ void k_to_caller(Bank b, const int* pack_of, const PackInfo* packs, i
 __global__ void k_from_caller(Bank b, const int* pack_of, const PackInfo* packs, const double* i0,
                               const double* i1, const double* i2, int ntot);
 size_t tile_lds_bytes(int cap, int groups, int nthr);
+// sc_team.hip
+template <int MODE, bool TWO_POINT, bool MIXED, int SHAPE>
+__global__ void k_team(TeamArgs a);
+__global__ void k_team_clear(TeamArgs a);
+__global__ void k_team_records(TeamArgs a, int team, double* out);
+size_t team_lds_bytes(int shape, int cell_words);
 constexpr int kExport = 64;
 }  // namespace sc
 
@@ -117,9 +122,15 @@ struct sc_system {
   int prec = SC_PREC_FP64;
   int contact_model = SC_CONTACT_CLOSEST;
   bool use_graphs = true;
-  int small_max = kSmallMax;  // FIRE of packings up to this size in one launch (0: never)
-  int small_steps = 50000;    // ... for at most this many iterations per launch
-  int* d_small_idx = nullptr;
+  int small_max = kSmallMax;  // 0: no teams, launches for every step
+  int small_steps = 50000;    // minimiser iterations of a team launch, at most
+  // teams (sc_team.hip): exchange words and the launch's seats
+  unsigned long long *d_team_pos = nullptr, *d_team_sums = nullptr, *d_team_flags = nullptr;
+  TeamSeat* d_team_seats = nullptr;
+  int* d_team_status = nullptr;
+  int team_seat_cap = 0;
+  double* d_team_se = nullptr;
+  size_t team_se_cap = 0;
   int ncells = 0, ntiles = 0, npblocks = 0;
   std::vector<int4> tiles;
   std::vector<int2> pblocks, tile_ranges, list_ranges;
@@ -814,36 +825,171 @@ void launch_update(sc_system* s, const PassSpec& ps, const FireParams& fp, int m
   s->cur_scal = 1 - s->cur_scal;
 }
 
-// FIRE of the packings in `active` in one launch of k_fire_small (one
-// workgroup per packing; every packing holds at most s->small_max <= kSmallMax
-// particles), to convergence or for at most s->small_steps iterations.  Positions, velocities, forces and the
-// per-packing scalars are written back in place; the rows of the list path no
-// longer match the moved particles, so every row is rebuilt by the next pass.
-void run_small_fire(sc_system* s, const std::vector<int>& active, const FireParams& fp) {
-  if (!s->d_small_idx) s->d_small_idx = s->dalloc<int>(s->npack);
-  HIPCK(hipMemcpyAsync(s->d_small_idx, active.data(), sizeof(int) * active.size(),
+// ---- teams: many steps in one launch (sc_team.hip) -------------------------
+
+using TeamFn = void (*)(TeamArgs);
+TeamFn team_kernel(int mode, bool two_point, bool mixed, int shape) {
+#define SC_TEAM_ROW(M, H)                                     \
+  {{&k_team<M, false, false, H>, &k_team<M, false, true, H>}, \
+   {&k_team<M, true, false, H>, &k_team<M, true, true, H>}}
+#define SC_TEAM_SHAPE(H)                                                          \
+  {SC_TEAM_ROW(kTeamFire, H), SC_TEAM_ROW(kTeamGd, H), SC_TEAM_ROW(kTeamHeun, H), \
+   {{&k_team<kTeamHeunSe, false, false, H>, nullptr},                             \
+    {&k_team<kTeamHeunSe, true, false, H>, nullptr}}}
+  // [shape][mode][contact model][pair precision]
+  static const TeamFn table[kTeamShapes][4][2][2] = {SC_TEAM_SHAPE(0), SC_TEAM_SHAPE(1)};
+#undef SC_TEAM_SHAPE
+#undef SC_TEAM_ROW
+  return table[shape][mode][two_point ? 1 : 0][mixed ? 1 : 0];
+}
+
+// A device runs one team launch of this process at a time: two launches that
+// each hold part of the CUs would wait for each other.  Held from the launch
+// to its end.
+constexpr int kMaxDevices = 64;
+std::mutex g_team_mu[kMaxDevices];
+
+struct TeamPlan {
+  int shape = 0;
+  std::vector<TeamSeat> seats;
+  size_t lds = 0;
+};
+
+// Seats for the packings in `want`: members of at most kTeamOwn[shape]
+// particles, of equal size within a packing, in the smallest shape whose
+// workgroups are all resident at once.  False when they do not fit.
+bool team_plan(sc_system* s, int mode, const std::vector<int>& want, TeamPlan& plan) {
+  if (s->path != SC_PATH_LIST || s->device >= kMaxDevices || want.empty()) return false;
+  long particles = 0;
+  int cell_words = 0;
+  for (int k : want) {
+    particles += s->packs[k].n;
+    cell_words = std::max(cell_words, (s->packs[k].rows * s->packs[k].cols + 31) / 32);
+  }
+  int cu = 0;
+  HIPCK(hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, s->device));
+  // Up to 128 particles one member of shape 1 is as fast as two of 64 (two-point
+  // FIRE of 128: 7.86 us an iteration either way) and waits for nobody; above,
+  // smaller members have fewer pairs each (N = 700: 64 a member 8.7 us).
+  int most = 0;
+  for (int k : want) most = std::max(most, s->packs[k].n);
+  for (int shape = most <= kTeamOwn[1] ? 1 : 0; shape < kTeamShapes; ++shape) {
+    const int own = kTeamOwn[shape];
+    const size_t lds = team_lds_bytes(shape, cell_words);
+    if (particles > (long)own * 4 * cu || lds + 1024 > (size_t)s->lds_max) continue;
+    TeamFn fn = team_kernel(mode, s->contact_model == SC_CONTACT_TWO_POINT,
+                            s->prec == SC_PREC_MIXED, shape);
+    HIPCK(hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    int per_cu = 0;
+    HIPCK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kTeamThreads, lds));
+    const long room = (long)per_cu * cu;
+    plan = TeamPlan{};
+    plan.shape = shape;
+    plan.lds = lds;
+    bool fits = true;
+    for (int k : want) {
+      const PackInfo& P = s->packs[k];
+      const int team = (P.n + own - 1) / own, per = (P.n + team - 1) / team;
+      // a rebuild's hit masks, 64 particles each, share the rows' LDS
+      fits = (long)plan.seats.size() + team <= room &&
+             P.n + 64 * 8 <= 64 * own * (kTeamRow + 2) / 4;
+      if (!fits) break;
+      const int base = (int)plan.seats.size();
+      int at = 0;
+      for (int m = 0; m < team; ++m) {
+        const int c = std::min(per, P.n - at);
+        plan.seats.push_back(TeamSeat{k, P.poff + at, c, m, team, base, per, 0});
+        at += c;
+      }
+    }
+    if (fits) return true;
+  }
+  return false;
+}
+
+// One team launch of at most max_steps iterations or steps, waited for.
+// Returns the launch's status bits (TeamStatus); the scalars are advanced in
+// place, and rows and cells no longer match the moved particles.
+int run_team(sc_system* s, int mode, const TeamPlan& plan, const FireParams* fp, int max_steps,
+             int se_every = 0, int step0 = 0, int nrec = 0) {
+  const int nseats = (int)plan.seats.size();
+  if (!s->d_team_pos) {
+    s->d_team_pos = s->dalloc<unsigned long long>((size_t)16 * s->ntot);
+  }
+  if (nseats > s->team_seat_cap) {
+    s->dfree(s->d_team_sums);
+    s->dfree(s->d_team_flags);
+    s->dfree(s->d_team_seats);
+    s->dfree(s->d_team_status);
+    s->d_team_status = s->dalloc<int>(nseats);
+    s->d_team_sums = s->dalloc<unsigned long long>((size_t)12 * kTeamUpdWaves * nseats);
+    s->d_team_flags = s->dalloc<unsigned long long>((size_t)kTeamFlagSlots * nseats);
+    s->d_team_seats = s->dalloc<TeamSeat>(nseats);
+    s->team_seat_cap = nseats;
+  }
+  HIPCK(hipMemcpyAsync(s->d_team_seats, plan.seats.data(), sizeof(TeamSeat) * nseats,
                        hipMemcpyHostToDevice, s->stream));
-  SmallFireArgs a{};
+  TeamArgs a{};
   a.b = s->B();
   a.packs = s->d_packs;
   a.scal = s->d_scal[s->cur_scal];
-  a.pack_idx = s->d_small_idx;
+  a.seats = s->d_team_seats;
+  a.pos = s->d_team_pos;
+  a.sums = s->d_team_sums;
+  a.flags = s->d_team_flags;
+  a.status = s->d_team_status;
   a.err = s->d_err;
-  a.fire = fp;
-  // a launch stops after s->small_steps iterations (50000 by default, about
-  // half a second), so no single kernel runs long; the minimiser's loop
-  // launches again for packings still running, whose rows are rebuilt from
-  // the state reached
-  a.max_steps = s->small_steps;
-  const bool tp = s->contact_model == SC_CONTACT_TWO_POINT;
-  const bool mixed = s->prec == SC_PREC_MIXED;
-  auto kern = tp ? (mixed ? &k_fire_small<true, true> : &k_fire_small<true, false>)
-                 : (mixed ? &k_fire_small<false, true> : &k_fire_small<false, false>);
-  {
-    KernelTimer t(s, SC_KERNEL_FIRE_FORCE);
-    hipLaunchKernelGGL(kern, dim3((unsigned)active.size()), dim3(kSmallThreads), 0, s->stream,
-                       a);
+  if (fp) a.fire = *fp;
+  a.gamma_window = s->gamma_window;
+  a.ntot = s->ntot;
+  a.nseats = nseats;
+  a.max_steps = max_steps;
+  if (nrec > 0) {  // records of the states before the launch's steps, step 0 excepted
+    const size_t need = (size_t)nrec * nseats * kNSe;
+    if (need > s->team_se_cap) {
+      s->dfree(s->d_team_se);
+      s->d_team_se = s->dalloc<double>(need);
+      s->team_se_cap = need;
+    }
+    a.se_part = s->d_team_se;
   }
+  a.se_every = std::max(se_every, 1);
+  a.se_first = step0 > 0 ? 1 : 0;
+  a.step0 = step0;
+  TeamFn fn = team_kernel(mode, s->contact_model == SC_CONTACT_TWO_POINT,
+                          s->prec == SC_PREC_MIXED, plan.shape);
+  std::vector<int> words(nseats);
+  {
+    std::lock_guard<std::mutex> lk(g_team_mu[s->device]);
+    hipLaunchKernelGGL(k_team_clear, dim3(std::min(1024, grid_for(16 * s->ntot, 256))), dim3(256),
+                       0, s->stream, a);
+    {
+      KernelTimer t(s, mode >= kTeamHeun ? SC_KERNEL_PREDICT : SC_KERNEL_FIRE_FORCE);
+      hipLaunchKernelGGL(fn, dim3(nseats), dim3(kTeamThreads), plan.lds, s->stream, a);
+    }
+    if (nrec > 0)
+      hipLaunchKernelGGL(k_team_records, dim3(nrec), dim3(64), 0, s->stream, a, nseats,
+                         s->d_se_ring + ((size_t)(step0 + se_every - 1) / se_every -
+                                         (step0 > 0 ? 1 : 0)) * kNSe);
+    HIPCK(hipMemcpyAsync(words.data(), s->d_team_status, sizeof(int) * nseats,
+                         hipMemcpyDeviceToHost, s->stream));
+    HIPCK(hipMemcpyAsync(s->scal.data(), s->d_scal[s->cur_scal], sizeof(PackScal) * s->npack,
+                         hipMemcpyDeviceToHost, s->stream));
+    HIPCK(hipStreamSynchronize(s->stream));
+  }
+  int status = 0;
+  for (int w : words) status |= w;
+  force_rebuild(s);
+  if (status & kTeamStalled) throw StatusError{SC_ERR_HIP, "a team of workgroups stalled"};
+  return status;
+}
+
+// Cells and rows for the launches per step after a team launch.
+void leave_team(sc_system* s) {
+  s->cur_buf = 0;
+  bin_all_sized(s, 0, 0);
+  clear_other_buffers(s);
   force_rebuild(s);
 }
 
@@ -1327,6 +1473,32 @@ int sc_strain_steps(sc_system* s, int nsteps, int se_every, double* se_out) {
   // timing; the steps left over run eagerly.
   const int resort_every = 1000;  // locality only: cells are exact every pass
   int st = 0;
+  // A packing whose workgroups fit the GPU at once steps as a team, a launch up
+  // to the next locality re-sort.  (Packings of a batch that gave up a launch at
+  // different steps could not go on together; records of mixed-precision runs
+  // are FP64 passes of their own.)
+  const bool se = se_every > 0 && se_every < nsteps;  // records before the last step's
+  const int mode = se ? kTeamHeunSe : kTeamHeun;
+  const std::vector<int> only{0};
+  TeamPlan plan;
+  if (s->npack == 1 && s->small_max > 0 && !s->timing && nsteps > 1 &&
+      !(se && s->prec == SC_PREC_MIXED) && team_plan(s, mode, only, plan)) {
+    while (st < nsteps) {
+      const int upto = std::min(nsteps, st + 2 * resort_every);
+      // states st .. upto - 1 that are recorded (never state 0)
+      const int recs = se ? (upto - 1) / se_every - (st > 0 ? (st - 1) / se_every : 0) : 0;
+      const int status = run_team(s, mode, plan, nullptr, upto - st, se_every, st, recs);
+      st = s->scal[0].step;
+      if (status) break;
+      if (st < nsteps) {
+        leave_team(s);
+        resort(s);
+        int e = check_errors(s);
+        if (e != SC_OK) return e;
+      }
+    }
+    leave_team(s);
+  }
   if (s->use_graphs && !s->timing && se_every == 0 && s->ntot <= kGraphMaxParticles) {
     const int chunk = 48;
     GraphExec g(s);
@@ -1490,8 +1662,17 @@ int sc_gd_steps(sc_system* s, int nmax, double emin, int* steps_done) {
   fp.max_iter = nmax;
   // nmax updates need nmax + 1 checked force passes; chunks never launch more
   const int chunk = std::min(64, nmax + 1);
+  std::vector<int> every;
+  for (int k = 0; k < s->npack; ++k) every.push_back(k);
+  TeamPlan plan;
+  bool teams = s->small_max > 0 && team_plan(s, kTeamGd, every, plan);
   while (true) {
-    for (int m = 0; m < chunk; ++m) {
+    if (teams) {
+      if (run_team(s, kTeamGd, plan, &fp, s->small_steps)) {
+        teams = false;
+        leave_team(s);
+      }
+    } else for (int m = 0; m < chunk; ++m) {
       PassSpec ps;
       ps.mode = kModeForces;
       ps.do_gd = 1;
@@ -1623,23 +1804,26 @@ int sc_fire_minimize(sc_system* s, const double* params, double switch_frms, int
       alloc_pblocks(s);
     }
   };
-  // Once every packing still running is small, one launch runs them to the
-  // end (k_fire_small): the tail of a batch then costs no launches per
-  // iteration, and a small system never launches per iteration at all.  List
-  // path only: its rows hold as many partners as the list kernels' (64) and
-  // are chosen by a rule no wider than theirs, so the one-launch path stops
-  // with SC_ERR_LIST_OVERFLOW only where the two-launch path would.
+  // Once the workgroups of all packings still running fit the GPU together,
+  // they run as teams, many iterations in one launch.  List path only: a
+  // team's rows hold as many partners as the list kernels' (64) and are chosen
+  // by a rule no wider than theirs, so it stops with SC_ERR_LIST_OVERFLOW only
+  // where they would.
   std::vector<int> active;
   for (int k = 0; k < s->npack; ++k) active.push_back(k);
-  auto all_small = [&]() {
-    if (s->small_max <= 0 || s->path != SC_PATH_LIST || active.empty()) return false;
-    for (int k : active)
-      if (s->packs[k].n > s->small_max) return false;
-    return true;
-  };
+  bool teams = s->small_max > 0, was_team = false;
+  TeamPlan plan;
   while (true) {
-    if (all_small()) {
-      run_small_fire(s, active, fp);
+    const bool team = teams && team_plan(s, kTeamFire, active, plan);
+    if (was_team && !team) leave_team(s);
+    was_team = team;
+    if (team) {
+      // CUs left idle by finished packings: back to the host for a new plan
+      // before long
+      int steps = s->small_steps;
+      if (active.size() > 1) steps = std::min(steps, 128);
+      const int st = run_team(s, kTeamFire, plan, &fp, steps);
+      if (st & (kTeamAbsent | kTeamOver)) teams = false;
     } else if (graph) {
       if (!g.exec) g.capture([&]() { iterations(chunk); });
       g.launch();
@@ -1669,7 +1853,7 @@ int sc_fire_minimize(sc_system* s, const double* params, double switch_frms, int
     for (int k = 0; k < s->npack; ++k)
       if (!s->scal[k].converged) active.push_back(k);
     if (active.empty()) break;
-    if (s->path == SC_PATH_LIST && 2 * (int)active.size() <= last_active) {
+    if (!team && s->path == SC_PATH_LIST && 2 * (int)active.size() <= last_active) {
       if (g.exec) {  // the captured launches name the old lists
         HIPCK(hipGraphExecDestroy(g.exec));
         g.exec = nullptr;

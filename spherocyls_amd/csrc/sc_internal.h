@@ -193,21 +193,49 @@ struct UpdateArgs {
   int fused;               // 1: reduce and decide here; 0: k_reduce already wrote red.scal_next
 };
 
-// FIRE of small packings in one launch: one workgroup of kSmallThreads per
-// packing of at most kSmallMax particles holds the packing in LDS and runs
-// every iteration (force pass, reduction, decision, update, list rebuild)
-// itself, so an iteration costs no launch and no global round trip.
+// Largest argument of sc_set_small_fire.
 constexpr int kSmallMax = 256;
-constexpr int kSmallThreads = 512;
-constexpr int kSmallRow = kNbrCap;  // partners a particle's LDS row holds
-struct SmallFireArgs {
+
+// Teams of workgroups that run many steps in one launch (sc_team.hip).
+constexpr int kTeamThreads = 512;
+constexpr int kTeamRow = kNbrCap;   // partners a particle's LDS row holds
+// Launch shapes: own particles of a member, and own + halo particles its LDS holds.
+constexpr int kTeamShapes = 2;
+constexpr int kTeamUpdWaves = 2;  // wavefronts that hold own particles, at most
+constexpr int kTeamOwn[kTeamShapes] = {64, 128}, kTeamCap[kTeamShapes] = {512, 768};
+enum TeamMode : int { kTeamFire = 0, kTeamGd = 1, kTeamHeun = 2, kTeamHeunSe = 3 };
+// bits of a member's flag word
+enum TeamFlag : int { kFlagRebuild = 1, kFlagStop = 2, kFlagOver = 4, kFlagFast = 8 };
+constexpr int kTeamFlagSlots = 6;  // four of pass flags, two of rebuild flags
+// launch status: a member never came up (nothing was written); a wait ran out
+// later; a member's halo or a row did not fit (the state reached is written
+// back); a particle outran the rebuild of a Heun launch (nothing was written)
+enum TeamStatus : int { kTeamAbsent = 1, kTeamStalled = 2, kTeamOver = 4, kTeamFast = 8 };
+// One workgroup: particles first .. first + count - 1 of the packing; member
+// `member` of its team of `team`, whose members are seats base .. base + team - 1.
+struct TeamSeat {
+  int pack, first, count, member, team, base;
+  int most;  // particles of the team's largest member
+  int pad0;
+};
+struct TeamArgs {
   Bank b;
   const PackInfo* packs;
-  PackScal* scal;          // read at the start, written at the end (in place)
-  const int* pack_idx;     // workgroup -> packing
+  PackScal* scal;            // read at the start, written at the end (in place)
+  const TeamSeat* seats;
+  unsigned long long* pos;   // [4][ntot][4] exchanged positions
+  unsigned long long* sums;  // [3][nseats][kTeamUpdWaves][4]
+  unsigned long long* flags; // [kTeamFlagSlots][nseats]
+  int* status;               // [nseats]: TeamStatus bits at a team's first seat
   int* err;
   FireParams fire;
-  int max_steps;           // iterations per launch: the host launches again for packings left
+  double gamma_window;
+  int ntot, nseats;
+  int max_steps;             // iterations (Heun: steps) of this launch
+  // kTeamHeunSe: a record where (step0 + steps) % se_every == 0, before the
+  // first step only with se_first; partial sums [record][member][kNSe]
+  int se_every, se_first, step0;
+  double* se_part;
 };
 
 // Device view of a system's current state, for other device code of this

@@ -1,0 +1,892 @@
+// Many steps in one launch: teams of workgroups.
+//
+// A step of a packing of a few hundred to a few ten thousand particles is two
+// small kernels whose time is launch gaps and chains of dependent loads, not
+// bandwidth or arithmetic (N = 16384: force pass 9.5 us and update 13.8 us per
+// FIRE iteration for 0.6 us of memory traffic).  Here the workgroups of a
+// packing (its team) stay resident and run the steps themselves.  Each member
+// owns a run of consecutive particles of the cell-sorted bank and keeps their
+// state in registers and LDS; the particles around them (its halo) are copied
+// into LDS once per force pass, so the pair loop reads LDS only.
+//
+// Exchange between members.  Every XCD has its own L2, so members exchange
+// through 8-byte words written and read with relaxed agent-scope atomics
+// (write-through stores, loads that bypass the caches); no fence, which would
+// write back and invalidate a whole L2, is needed:
+//   * positions: a record of 4 words per particle in one of four buffers.  A
+//     word no position can have (kEmpty, a NaN with a payload no operation
+//     yields) marks a word not written yet, so a reader polls the data
+//     itself: one trip instead of flag-then-data.  A member waits for its
+//     halo only, not for the whole team;
+//   * sums (minimisers): four words per member and update wavefront in one of
+//     three slots, empty-marked like the positions; every member adds up all
+//     sums in the same order and takes the same decision;
+//   * flags (Heun): one word per member and pass, (sequence number << 8 |
+//     bits), in four slots; a reader waits for the pass's number.
+// Rebuilds.  Rows hold while no particle has moved half the skin from its
+// position at the last rebuild.  Minimisers evaluate a pass on the old rows
+// and a member that has moved too far says so in place of its sums: the team
+// then rebuilds from the same positions and repeats the pass, so the common
+// pass has no exchange for it.  Heun steps have no team-wide exchange to
+// carry that: a member asks at 0.6 of the limit, all read the flags one pass
+// late, when they have long arrived, and a particle that reached the limit
+// before the rebuild makes the launch give up with nothing written (the host
+// then takes these steps with the launches per step).
+// Buffer reuse.  Positions of a pass are marked empty once every member is
+// known to have read them: in a minimiser when all sums of the pass are in, in
+// Heun two passes later, when all flags of the pass in between are in.  The
+// marks are waited for before the member's next sums or flags go out, which
+// everyone who will poll the buffer's next positions reads first.  Sum slots
+// follow the same rule with the sums themselves.
+//
+// Every wait is bounded.  The first pass of a launch doubles as the roll call:
+// a member that never becomes resident (another kernel holds the CUs) makes the
+// others leave without having written anything, and the host goes on with the
+// launches per step.  The host launches at most as many workgroups as are
+// resident at once.
+//
+// Measured, all-gather of 4 words by G workgroups over all XCDs: 1.05 us (G = 2),
+// 1.5 (16), 1.8 (64), 2.0 (128), 2.8 (256); an empty kernel in a captured graph
+// takes 1.65 us.  Against the launches per step, two-point FIRE iterations of
+// 16384 particles 19.5 -> 13.5 us, of 700 15.7 -> 10.1; sheared steps of 16384
+// 21.6 -> 14.6 us, of 512 14.9 -> 11.8; descent of 1000 16.6 -> 9.3.
+#include <hip/hip_runtime.h>
+
+#include "sc_internal.h"
+#include "sc_physics.h"
+
+namespace sc {
+
+namespace {
+
+typedef unsigned long long u64;
+constexpr u64 kEmpty = 0x7ff8deadbeef0001ull;
+// In place of a sum: the rows no longer hold; a coordinate is not finite.
+constexpr u64 kNeedMark = 0x7ff8deadbeef0002ull, kStopMark = 0x7ff8deadbeef0003ull;
+constexpr int kBufs = 4;  // position buffers
+constexpr int kWaves = kTeamThreads / 64;
+constexpr int kRowStride = kTeamRow + 2;  // odd word stride: rows start in different banks
+
+__device__ __forceinline__ u64 word_load(const u64* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void word_store(u64* p, u64 v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ u64 bits_of(double v) { return (u64)__double_as_longlong(v); }
+__device__ __forceinline__ double from_bits(u64 v) { return __longlong_as_double((long long)v); }
+
+// All of this wavefront's stores have reached the coherence point.
+__device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// The value, opaque to the optimiser: addresses formed from it are computed
+// where they are used instead of being hoisted out of the step loop, where the
+// two dozen arrays' addresses would fill the registers the pair math needs.
+__device__ __forceinline__ int opaque(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// A wait that ends: over() is true once `limit` ticks (100 MHz) have passed
+// since its first call, or, after 0.1 ms, when a member of the team has
+// reported that it gave up.  (The clock is not read while words arrive at the
+// first look.)
+struct Wait {
+  u64 t0 = 0;
+  __device__ __forceinline__ bool over(u64 limit, const int* status) {
+    const u64 t = wall_clock64();
+    if (t0 == 0) {
+      t0 = t;
+      return false;
+    }
+    return t - t0 > limit ||
+           (t - t0 > 10000 &&
+            (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) &
+             (kTeamAbsent | kTeamStalled)));
+  }
+};
+
+// LDS of a member of up to OWN particles, OWN + halo <= CAP.  Compile-time sizes
+// put every array at a constant offset, so an access is one index register and
+// an immediate.  The cell marks of a rebuild follow (dynamic, by the packing's
+// grid).
+template <int OWN, int CAP>
+struct TeamLds {
+  double x[CAP], y[CAP], nx[CAP], ny[CAP], R[CAP], A[CAP];  // own particles, then the halo
+  double fx[OWN], fy[OWN], tq[OWN];                         // own particles: forces
+  double phi[OWN], vx[OWN], vy[OWN], vp[OWN];  // ... angle; FIRE velocity, Heun predictor velocity
+  double xb[OWN], yb[OWN];                     // ... position at the last rebuild
+  double m[OWN];                               // ... FIRE 1 / sqrt(I), GD and Heun I
+  double ox[OWN], oy[OWN], op[OWN], rc[OWN];   // ... Heun: state the step starts from, RC
+  int id[CAP];
+  int halo[CAP];                               // storage index of halo entry e
+  union {
+    unsigned short row[OWN * kRowStride];      // partners (local indices)
+    u64 hit[OWN * kRowStride / 4];             // rebuild: halo hit masks, 64 particles each
+  };
+  unsigned cells[4];                           // rebuild: marked cells (dynamic)
+};
+
+}  // namespace
+
+// Bytes of dynamic LDS of a launch of shape `shape` over grids of up to
+// cell_words * 32 cells.
+size_t team_lds_bytes(int shape, int cell_words) {
+  const size_t fixed = shape == 0 ? sizeof(TeamLds<kTeamOwn[0], kTeamCap[0]>)
+                                  : sizeof(TeamLds<kTeamOwn[1], kTeamCap[1]>);
+  return fixed + (size_t)cell_words * sizeof(unsigned);
+}
+
+// Empty marks for every word a launch polls, zero flags.
+__global__ void k_team_clear(TeamArgs a) {
+  const size_t np = (size_t)kBufs * a.ntot * 4, ns = (size_t)3 * a.nseats * 4 * kTeamUpdWaves,
+               nf = (size_t)kTeamFlagSlots * a.nseats;
+  const size_t stride = (size_t)gridDim.x * blockDim.x;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < np + ns + nf; i += stride) {
+    if (i < np) a.pos[i] = kEmpty;
+    else if (i < np + ns) a.sums[i - np] = kEmpty;
+    else a.flags[i - np - ns] = 0;
+  }
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < a.nseats; i += (int)stride) a.status[i] = 0;
+}
+
+// Stress and energy records of a launch (one packing): a workgroup adds up a
+// record's partial sums in member order and normalises them as k_reduce does.
+__global__ void __launch_bounds__(64) k_team_records(TeamArgs a, int team, double* out) {
+  const int r = blockIdx.x, t = threadIdx.x;
+  if (t >= kNSe) return;
+  const PackInfo& P = a.packs[0];
+  const PackScal& S = a.scal[0];
+  double v = 0.0;
+  for (int m = 0; m < team; ++m) v += a.se_part[((size_t)r * team + m) * kNSe + t];
+  if (t == kSeE) v *= P.inv_2n;
+  else if (t != kSeNc) v /= S.Lx * S.Ly;
+  out[(size_t)r * kNSe + t] = v;
+}
+
+// MODE kTeamFire / kTeamGd: minimiser iterations (force pass, sums and
+// decision, update) until the packing has finished or a.max_steps have run.
+// MODE kTeamHeun / kTeamHeunSe: a.max_steps sheared Heun steps (predictor and
+// corrector passes); kTeamHeunSe also records stress and energy, FP64 only.
+// The formulas, the rows' selection rule and the FIRE state machine are those
+// of k_list and k_update; sums run in another order.
+template <int MODE, bool TWO_POINT, bool MIXED, int SHAPE>
+__global__ void __launch_bounds__(kTeamThreads) __attribute__((amdgpu_waves_per_eu(4)))
+k_team(TeamArgs a) {
+#pragma clang fp contract(off)
+  constexpr bool kHeun = MODE == kTeamHeun || MODE == kTeamHeunSe;
+  constexpr bool kFire = MODE == kTeamFire, kGd = MODE == kTeamGd;
+  constexpr int kSums = kFire ? 4 : 1;  // words of a published sum
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  __shared__ double s_part[kWaves * kNSe];
+  __shared__ int s_count[kWaves];
+  // Raised and read in phases separated by barriers, so that all threads leave
+  // a loop together: s_need (own particles ask for a rebuild), s_bits (flags
+  // gathered from the team), s_fail (a wait ran out), s_over (halo or row
+  // overflow), s_next (what the minimiser does next).
+  __shared__ int s_need, s_bits, s_fail, s_over, s_next;
+  enum : int { kGoOn = 0, kDone = 1, kAgain = 2 };
+  // Per-packing scalars of iteration k in slot k & 1: thread 0 writes the next
+  // iteration's while others still read this one's.
+  __shared__ PackScal s_S[2];
+  const int tid0 = threadIdx.x, lane64 = tid0 & 63, wave = tid0 >> 6;
+  int tid = tid0;
+  const TeamSeat seat = a.seats[blockIdx.x];
+  const int pk = seat.pack, T = seat.team, me = seat.member;
+  const PackInfo P = a.packs[pk];
+  if (!kHeun && a.scal[pk].converged) return;  // the whole team
+  const Bank& b = a.b;
+  const int own = seat.count, first = seat.first;
+  const int cell_words = (P.rows * P.cols + 31) >> 5;
+  constexpr int kCap = kTeamCap[SHAPE];
+  TeamLds<kTeamOwn[SHAPE], kCap>& l = *reinterpret_cast<TeamLds<kTeamOwn[SHAPE], kCap>*>(lds_raw);
+  int* const status = a.status + seat.base;  // the team's
+  u64* const flags = a.flags + seat.base;    // [slot][member]: slots nseats apart
+  u64* const sums = a.sums + (size_t)seat.base * 4 * kTeamUpdWaves;
+
+  // force mapping: L lanes per own particle; update mapping: thread t moves
+  // own particle t (the first wavefronts)
+  int L = 1, lg = 0;
+  while (L < 8 && own * 2 * L <= kTeamThreads) {
+    L *= 2;
+    ++lg;
+  }
+  const int lane = tid & (L - 1), p0 = tid >> lg;
+  const bool act = p0 < own;
+  const int glane = lane64 & ~(L - 1);  // first lane of the particle's group in the wavefront
+  const bool upd = tid < own;
+  const int nuw = (seat.most + 63) >> 6;  // update wavefronts of the team's largest member
+  const int nsum = T > 1 ? T * nuw : 1;   // published sums
+  int gu = first + (upd ? tid : 0);
+
+  if (upd) {
+    l.x[tid] = b.x[gu];
+    l.y[tid] = b.y[gu];
+    l.nx[tid] = b.nx[gu];
+    l.ny[tid] = b.ny[gu];
+    l.R[tid] = b.R[gu];
+    l.A[tid] = b.A[gu];
+    l.id[tid] = b.id[gu];
+    l.phi[tid] = b.phi[gu];
+    l.m[tid] = kFire ? 1.0 / sqrt(b.I[gu]) : b.I[gu];
+    if (kFire) {
+      l.vx[tid] = b.vx[gu];
+      l.vy[tid] = b.vy[gu];
+      l.vp[tid] = b.vpsi[gu];
+    }
+    if (kHeun) l.rc[tid] = b.RC[gu];
+  }
+  if (tid == 0) {
+    s_need = s_bits = s_fail = s_over = s_next = 0;
+    s_S[0] = a.scal[pk];
+  }
+  const double Lx = a.scal[pk].Lx, Ly = a.scal[pk].Ly;
+  const double le_ratio = Lx / Ly;
+  const double skin = P.pad, sx = fmax(1.5, 1.0 + 0.5 * Lx / Ly) * P.pad, hs = 0.5 * P.pad;
+  double gam = a.scal[pk].gamma, gam_eval = gam, center = gam;
+  const double window = kHeun ? a.gamma_window : 0.0;
+  const u64 kRollCall = 20000000ull, kStall = 500000000ull;  // 0.2 s, 5 s
+
+  auto record_of = [&](int j, int g) {
+    return a.pos + ((size_t)(j & (kBufs - 1)) * a.ntot + g) * 4;
+  };
+  // publish an own particle's position as pass j's
+  auto publish = [&](int j, double px, double py, double pnx, double pny) {
+    if (T > 1) {
+      u64* r = record_of(j, gu);
+      word_store(r, bits_of(px));
+      word_store(r + 1, bits_of(py));
+      word_store(r + 2, bits_of(pnx));
+      word_store(r + 3, bits_of(pny));
+    }
+  };
+  auto mark_empty = [&](int j) {
+    if (T > 1 && upd) {
+      u64* r = record_of(j, gu);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) word_store(r + k, kEmpty);
+    }
+  };
+  // halo entries' positions of pass j into LDS
+  auto fetch_halo = [&](int j, int H, u64 limit) {
+    for (int e = tid; e < H; e += kTeamThreads) {
+      const u64* r = record_of(j, l.halo[e]);
+      u64 w[4];
+      Wait wait;
+      while (true) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[k] = word_load(r + k);
+        if (w[0] != kEmpty && w[1] != kEmpty && w[2] != kEmpty && w[3] != kEmpty) break;
+        if (wait.over(limit, status)) {
+          s_fail = 1;
+          break;
+        }
+      }
+      l.x[own + e] = from_bits(w[0]);
+      l.y[own + e] = from_bits(w[1]);
+      l.nx[own + e] = from_bits(w[2]);
+      l.ny[own + e] = from_bits(w[3]);
+    }
+  };
+  // every member's flag word numbered seq in slot `slot`, ORed into s_bits
+  auto gather_flags = [&](int slot, unsigned seq, u64 limit) {
+    const u64* f = flags + (size_t)slot * a.nseats;
+    for (int m = tid; m < T; m += kTeamThreads) {
+      u64 v;
+      Wait wait;
+      while (((v = word_load(f + m)) >> 8) != seq)
+        if (wait.over(limit, status)) {
+          s_fail = 1;
+          break;
+        }
+      if ((v >> 8) == seq && (v & 0xff)) atomicOr(&s_bits, (int)(v & 0xff));
+    }
+  };
+  auto put_flag = [&](int slot, unsigned seq, int bits) {  // one thread
+    word_store(flags + (size_t)slot * a.nseats + me, ((u64)seq << 8) | (u64)bits);
+  };
+  // a member that comes up after the others have left at the roll call finds
+  // their report and leaves as absent too
+  auto give_up = [&](int why) {
+    if (why == kTeamStalled &&
+        (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kTeamAbsent))
+      return;
+    atomicOr(status, why);
+  };
+
+  int H = 0;    // halo entries
+  int cnt = 0;  // row length of the force mapping's particle (same in its L lanes)
+  int steps = 0, pass = 0, xch = 0, nrec = 0;
+  unsigned rebuilds = 0;
+  bool build = true;       // this pass starts with new rows (uniform over the team)
+  bool was_built = false;  // Heun: the previous pass did
+  bool predicted = false;  // Heun: the positions are a step's predicted ones
+  if (upd) publish(0, l.x[tid], l.y[tid], l.nx[tid], l.ny[tid]);
+  if (kHeun && T > 1 && tid == 0) put_flag(0, 1, 0);
+  __syncthreads();
+
+  while (true) {
+    tid = opaque(tid0);
+    gu = first + (upd ? tid : 0);
+    const int p = opaque(p0);
+    const u64 limit = pass == 0 ? kRollCall : kStall;
+    // ---- positions of this pass
+    if (T > 1) {
+      if (kHeun && pass > 0) gather_flags((pass - 1) & 3, (unsigned)pass, kStall);
+      if (!build) fetch_halo(pass, H, limit);
+    }
+    __syncthreads();
+    if (s_fail) {
+      if (tid == 0) give_up(pass == 0 ? kTeamAbsent : kTeamStalled);
+      return;
+    }
+    if (kHeun) {
+      const int bits = T > 1 ? s_bits : s_need;
+      if (bits & kFlagStop) break;  // a non-finite coordinate: the error word says so
+      if (T > 1) {
+        if ((bits & kFlagFast) && !was_built) {
+          if (tid == 0) give_up(kTeamFast);
+          return;
+        }
+        build = build || ((bits & kFlagRebuild) && !was_built);
+        if (pass >= 2) mark_empty(pass - 2);
+      } else {
+        build = build || (bits & kFlagRebuild);
+      }
+    } else if (T == 1) {
+      build = build || (s_need & kFlagRebuild);
+    }
+    // ---- halo and rows from the positions of this pass
+    const bool built = build;
+    if (build) {
+      center = gam_eval;
+      const double glo = gam_eval - window, ghi = gam_eval + window;
+      __syncthreads();  // s_need and s_bits read by all
+      if (tid == 0) s_need = s_bits = 0;
+      if (upd) {
+        l.xb[tid] = l.x[tid];
+        l.yb[tid] = l.y[tid];
+      }
+      H = 0;
+      if (T > 1) {
+        // cells within one of an own particle's
+        for (int w = tid; w < cell_words; w += kTeamThreads) l.cells[w] = 0;
+        __syncthreads();
+        if (upd) {
+          double xw = l.x[tid], yw = l.y[tid];
+          wrap_coord(xw, Lx);
+          wrap_coord(yw, Ly);
+          int col, row;
+          cell_col_row(xw, yw, Lx, Ly, P, col, row);
+          for (int d = -1; d <= 1; ++d)
+            for (int e = -1; e <= 1; ++e) {
+              const int c = (row + d + P.rows) % P.rows * P.cols + (col + e + P.cols) % P.cols;
+              atomicOr(&l.cells[c >> 5], 1u << (c & 31));
+            }
+        }
+        __syncthreads();
+        // wavefront w looks at its eighth of the packing, 64 particles at a
+        // time; the words of kAhead looks are in flight together
+        constexpr int kAhead = 8;
+        const int per = (P.n + 64 * kWaves - 1) / (64 * kWaves);
+        int mine = 0;
+        for (int k0 = 0; k0 < per; k0 += kAhead) {
+          u64 wx[kAhead], wy[kAhead];
+          Wait wait;
+          while (true) {
+            bool all = true;
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+              const int i = (wave * per + k0 + k) * 64 + lane64;
+              const u64* r = record_of(pass, P.poff + min(i, P.n - 1));
+              wx[k] = word_load(r);
+              wy[k] = word_load(r + 1);
+            }
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) all = all && wx[k] != kEmpty && wy[k] != kEmpty;
+            if (all) break;
+            if (wait.over(limit, status)) {
+              s_fail = 1;
+              break;
+            }
+          }
+#pragma unroll
+          for (int k = 0; k < kAhead; ++k) {
+            if (k0 + k >= per) break;
+            const int i = (wave * per + k0 + k) * 64 + lane64, g = P.poff + i;
+            double xw = from_bits(wx[k]), yw = from_bits(wy[k]);
+            wrap_coord(xw, Lx);
+            wrap_coord(yw, Ly);
+            int col, row;
+            cell_col_row(xw, yw, Lx, Ly, P, col, row);
+            const int c = row * P.cols + col;
+            const bool hit = i < P.n && (g < first || g >= first + own) &&
+                             ((l.cells[c >> 5] >> (c & 31)) & 1u);
+            const u64 m = __ballot(hit);
+            if (lane64 == 0) l.hit[wave * per + k0 + k] = m;
+            mine += __popcll(m);
+          }
+        }
+        if (lane64 == 0) s_count[wave] = mine;
+        __syncthreads();
+        int at = 0;
+        for (int w = 0; w < kWaves; ++w) {
+          if (w < wave) at += s_count[w];
+          H += s_count[w];
+        }
+        if (own + H <= kCap) {
+          for (int k = 0; k < per; ++k) {
+            const u64 m = l.hit[wave * per + k];
+            if ((m >> lane64) & 1ull)
+              l.halo[at + __popcll(m & ((1ull << lane64) - 1ull))] =
+                  P.poff + (wave * per + k) * 64 + lane64;
+            at += __popcll(m);
+          }
+        } else {
+          H = 0;
+          if (tid == 0) s_over = 1;
+        }
+        __syncthreads();
+        fetch_halo(pass, H, limit);
+        for (int e = tid; e < H; e += kTeamThreads) {
+          const int g = l.halo[e];
+          l.R[own + e] = b.R[g];
+          l.A[own + e] = b.A[g];
+          l.id[own + e] = b.id[g];
+        }
+      }
+      __syncthreads();
+      // rows: the list kernels' selection rule, a ballot placing the hits in
+      // increasing local index
+      cnt = 0;
+      {
+        const int pp = act ? p : 0, M = own + H;
+        const double xp = l.x[pp], yp = l.y[pp], reach_p = l.R[pp] + l.A[pp];
+        for (int base = 0; base < M; base += L) {
+          const int q = base + lane;
+          bool hit = false;
+          if (act && q < M && q != p) {
+            const double reach = reach_p + l.R[q] + l.A[q];
+            const double dy = min_image(yp - l.y[q], Ly);
+            if (fabs(dy) < reach + skin) {
+              const double dx = min_image(xp - l.x[q], Lx);
+              hit = fabs(dx + glo * dy) < reach + sx || fabs(dx + ghi * dy) < reach + sx;
+            }
+          }
+          const u64 hits = (__ballot(hit) >> glane) & ((1ull << L) - 1ull);
+          const int pos = cnt + __popcll(hits & ((1ull << lane) - 1ull));
+          if (hit && pos < kTeamRow) l.row[p * kRowStride + pos] = (unsigned short)q;
+          cnt += __popcll(hits);
+        }
+        if (cnt > kTeamRow) s_over = 2;
+      }
+      __syncthreads();
+      // the team goes on only if every member's halo and rows fit
+      bool over = s_over != 0;
+      if (T > 1) {
+        ++rebuilds;
+        if (tid == 0) put_flag(4 + (rebuilds & 1), rebuilds, over ? kFlagOver : 0);
+        gather_flags(4 + (rebuilds & 1), rebuilds, kStall);
+        __syncthreads();
+        over = (s_bits & kFlagOver) != 0;
+        if (s_fail) {
+          if (tid == 0) give_up(pass == 0 ? kTeamAbsent : kTeamStalled);
+          return;
+        }
+      }
+      if (over) {
+        if (tid == 0) atomicOr(status, kTeamOver);
+        break;  // the state of this pass is written back
+      }
+      build = false;
+    }
+
+    // ---- forces (force mapping): the bounding-circle hits of the particle's
+    // row as a bit mask, the same in its L lanes, which then take them in turn,
+    // so a wavefront runs the pair math (two-point: about 470 FP64
+    // instructions) as often as its busiest particle has L hits
+    const bool fp64 = !MIXED || s_S[kHeun ? 0 : steps & 1].prec == kFP64;
+    const bool record = MODE == kTeamHeunSe && !predicted && (steps > 0 || a.se_first) &&
+                        (a.step0 + steps) % a.se_every == 0;
+    double Fx = 0.0, Fy = 0.0, Tq = 0.0;
+    double acc[kNSum] = {};
+    if (act) {
+      const double xp = l.x[p], yp = l.y[p], nxp = l.nx[p], nyp = l.ny[p];
+      const double Rp = l.R[p], Ap = l.A[p], reach_p = Rp + Ap;
+      const int idp = l.id[p];
+      const unsigned short* row = l.row + p * kRowStride;
+      u64 mask = 0;
+      for (int base = 0; base < cnt; base += L) {
+        bool hit = false;
+        if (base + lane < cnt) {
+          const int q = row[base + lane];
+          double dx = min_image(xp - l.x[q], Lx);
+          const double dy = min_image(yp - l.y[q], Ly);
+          dx += gam_eval * dy;
+          const double reach = reach_p + l.R[q] + l.A[q];
+          hit = dx * dx + dy * dy < reach * reach * (1.0 + 1e-10);
+        }
+        mask |= ((__ballot(hit) >> glane) & ((1ull << L) - 1ull)) << base;
+      }
+      for (int k = 0; k < lane; ++k) mask &= mask - 1;  // this lane's first hit
+      while (mask) {
+        const int q = row[__ffsll((long long)mask) - 1];
+        pair_into<kGd || MODE == kTeamHeunSe, TWO_POINT>(
+            xp, yp, nxp, nyp, Rp, Ap, idp, l.x[q], l.y[q], l.nx[q], l.ny[q], l.R[q], l.A[q],
+            l.id[q], Lx, Ly, gam_eval, fp64, kGd || record, Fx, Fy, Tq, acc);
+        for (int k = 0; k < L; ++k) mask &= mask - 1;  // its next one
+      }
+    }
+    Fx = group_sum(Fx, L);
+    Fy = group_sum(Fy, L);
+    Tq = group_sum(Tq, L);
+    if (act && lane == 0) {
+      l.fx[p] = Fx;
+      l.fy[p] = Fy;
+      l.tq[p] = Tq;
+    }
+    if (kGd) {  // energy of this wavefront's pairs
+      const double e = wave_sum(acc[kSeE]);
+      if (lane64 == 63) s_part[wave] = e;
+    }
+    if (MODE == kTeamHeunSe && record) {
+#pragma unroll
+      for (int k = 0; k < kNSe; ++k) {
+        const double v = wave_sum(acc[k]);
+        if (lane64 == 63) s_part[wave * kNSe + k] = v;
+      }
+    }
+    __syncthreads();  // forces visible to the update mapping
+    tid = opaque(tid0);
+    if (MODE == kTeamHeunSe && record) {
+      if (tid < kNSe) {
+        double v = 0.0;
+        for (int w = 0; w < kWaves; ++w) v += s_part[w * kNSe + tid];
+        a.se_part[((size_t)nrec * T + me) * kNSe + tid] = v;
+      }
+      ++nrec;
+    }
+    double x = 0.0, y = 0.0, phi = 0.0;  // the particle's new state (update mapping)
+    bool moved = kHeun;                  // uniform over a wavefront
+    if (kHeun) {
+      // ---- predictor or corrector (sheared steps, as k_list)
+      if (tid == 0) s_bits = s_need = 0;
+      const double dt = P.dt, gd = P.strain_rate;
+      if (upd) {
+        const double fx = l.fx[tid], fy = l.fy[tid], tq = l.tq[tid], Iu = l.m[tid];
+        const double iso = gd * iso_rot_seg(l.rc[tid], l.nx[tid], l.ny[tid], l.A[tid]);
+        if (!predicted) {
+          const double ox = l.x[tid], oy = l.y[tid], op = l.phi[tid];
+          const double vx = fx - gam * fy, vy = fy, vp = tq / Iu - iso;
+          l.ox[tid] = ox;
+          l.oy[tid] = oy;
+          l.op[tid] = op;
+          l.vx[tid] = vx;
+          l.vy[tid] = vy;
+          l.vp[tid] = vp;
+          x = ox + dt * vx;
+          y = oy + dt * vy;
+          phi = op + dt * vp;
+        } else {
+          x = l.ox[tid] + 0.5 * dt * (l.vx[tid] + (fx - gam_eval * fy));
+          y = l.oy[tid] + 0.5 * dt * (l.vy[tid] + fy);
+          phi = l.op[tid] + 0.5 * dt * (l.vp[tid] + (tq / Iu - iso));
+        }
+      }
+      if (!predicted) {
+        gam_eval = gam + dt * gd;  // the corrector's strain
+        build = fabs(gam_eval - center) >= window;
+      } else {
+        double g2 = gam + gd * dt;
+        if (g2 >= 0.5 * le_ratio) {
+          if (upd) {
+            if (y < 0) y += Ly;
+            else if (y > Ly) y -= Ly;
+            x += le_ratio * y;
+            if (x < 0) x += Lx;
+            else {
+              int guard = 0;
+              while (x > Lx && guard++ < 8) x -= Lx;
+            }
+          }
+          g2 -= le_ratio;
+          build = true;
+        }
+        if (tid == 0) {
+          double gt = s_S[0].gamma_total + gd * dt;
+          if (build && le_ratio == 1.0) gt = (double)(int)(gt + 1) + g2;
+          s_S[0].gamma = g2;
+          s_S[0].gamma_total = gt;
+          s_S[0].step = s_S[0].step + 1;
+        }
+        gam = gam_eval = g2;
+        build = build || fabs(gam - center) >= window;
+        ++steps;
+      }
+      predicted = !predicted;
+      __syncthreads();  // s_need cleared
+    }
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+    if (!kHeun && wave < nuw) {
+      // ---- sums and decision: every update wavefront of every member publishes
+      // its sums, adds up all of them in the same order and decides the same
+      if (kGd) {
+        if (wave == 0 && lane64 < kWaves) s0 = s_part[lane64];
+      } else if (upd) {
+        const double fx = l.fx[tid], fy = l.fy[tid], tq = l.tq[tid], gp = tq * l.m[tid];
+        const double vx = l.vx[tid], vy = l.vy[tid], vp = l.vp[tid];
+        const double f2 = fx * fx + fy * fy;
+        s0 = f2 + tq * tq;
+        s1 = fx * vx + fy * vy + gp * vp;
+        s2 = f2 + gp * gp;
+        s3 = vx * vx + vy * vy + vp * vp;
+      }
+      s0 = wave_sum(s0);
+      if (kFire) {
+        s1 = wave_sum(s1);
+        s2 = wave_sum(s2);
+        s3 = wave_sum(s3);
+      }
+      if (T == 1 && kFire && lane64 == 63) {  // two update wavefronts of one member: through LDS
+        s_part[wave * 4] = s0;
+        s_part[wave * 4 + 1] = s1;
+        s_part[wave * 4 + 2] = s2;
+        s_part[wave * 4 + 3] = s3;
+      }
+    }
+    if (T == 1 && kFire && nuw > 1) __syncthreads();
+    if (!kHeun && wave < nuw) {
+      if (T == 1 && nuw > 1) {
+        if (kFire) {
+          // (lane 63 carries the totals)
+          s0 = s_part[0] + s_part[4];
+          s1 = s_part[1] + s_part[5];
+          s2 = s_part[2] + s_part[6];
+          s3 = s_part[3] + s_part[7];
+        } else {
+          s0 = 0.0;
+          for (int w = 0; w < kWaves; ++w) s0 += s_part[w];
+        }
+      }
+      const int need = s_need;
+      bool again = false, stop = (need & kFlagStop) != 0;
+      if (nsum > 1) {
+        u64* const cur = sums + (size_t)(xch % 3) * a.nseats * 4 * kTeamUpdWaves;
+        stores_done();  // empty marks of the last pass
+        if (lane64 == 63) {
+          u64* w = cur + (me * nuw + wave) * 4;
+          word_store(w, stop ? kStopMark : (need & kFlagRebuild) ? kNeedMark : bits_of(s0));
+          if (kFire) {
+            word_store(w + 1, bits_of(s1));
+            word_store(w + 2, bits_of(s2));
+            word_store(w + 3, bits_of(s3));
+          }
+        }
+        s0 = s1 = s2 = s3 = 0.0;
+        constexpr int kAhead = 4;  // sums of 256 wavefronts in flight
+        for (int k0 = 0; k0 < nsum; k0 += 64 * kAhead) {
+          u64 v[kAhead][kSums];
+          Wait wait;
+          while (true) {
+            bool all = true;
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+              const u64* w = cur + min(k0 + 64 * k + lane64, nsum - 1) * 4;
+#pragma unroll
+              for (int i = 0; i < kSums; ++i) v[k][i] = word_load(w + i);
+            }
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k)
+#pragma unroll
+              for (int i = 0; i < kSums; ++i) all = all && v[k][i] != kEmpty;
+            if (all) break;
+            if (wait.over(kStall, status)) {
+              s_fail = 1;
+              break;
+            }
+          }
+#pragma unroll
+          for (int k = 0; k < kAhead; ++k) {
+            if (k0 + 64 * k + lane64 >= nsum) break;
+            again = again || v[k][0] == kNeedMark;
+            stop = stop || v[k][0] == kStopMark;
+            s0 += from_bits(v[k][0]);
+            if (kFire) {
+              s1 += from_bits(v[k][1]);
+              s2 += from_bits(v[k][2]);
+              s3 += from_bits(v[k][3]);
+            }
+          }
+        }
+        again = __any(again);
+        stop = __any(stop);
+        s0 = wave_sum(s0);
+        if (kFire) {
+          s1 = wave_sum(s1);
+          s2 = wave_sum(s2);
+          s3 = wave_sum(s3);
+        }
+      }
+      if (stop || again) {
+        if (tid == 0) s_next = stop ? kDone : kAgain;
+      } else {
+        mark_empty(pass);  // all have read this pass's positions
+        const PackScal& S0 = s_S[steps & 1];
+        const MinStep S =
+            minimiser_step(a.fire, kFire, P.n, P.inv_2n, S0, last_lane(s0), last_lane(s1),
+                           last_lane(s2), last_lane(s3), last_lane(s0), false);
+        moved = S.end == 0;
+        if (tid == 0) {
+          advance(s_S[(steps + 1) & 1], S0, S, kFire);
+          s_next = S.end ? kDone : kGoOn;
+        }
+        // ---- update (update mapping); nothing moves once finished
+        if (upd && moved) {
+          const double fx = l.fx[tid], fy = l.fy[tid], tq = l.tq[tid];
+          x = l.x[tid];
+          y = l.y[tid];
+          phi = l.phi[tid];
+          if (kGd) {
+            x += P.dt * fx;
+            y += P.dt * fy;
+            phi += P.dt * tq / l.m[tid];
+          } else {
+            const double isq = l.m[tid], gp = tq * isq;
+            const double vx = l.vx[tid], vy = l.vy[tid], vp = l.vp[tid];
+            double ux, uy, up;
+            if (S.mix) {
+              ux = S.c_keep * vx + S.c_force * fx;
+              uy = S.c_keep * vy + S.c_force * fy;
+              up = S.c_keep * vp + S.c_force * gp;
+            } else {
+              x -= 0.5 * S.dt_old * vx;
+              y -= 0.5 * S.dt_old * vy;
+              phi -= 0.5 * S.dt_old * vp * isq;
+              ux = uy = up = 0.0;
+            }
+            const double dt = S.dt;
+            ux += dt * fx;
+            uy += dt * fy;
+            up += dt * gp;
+            l.vx[tid] = ux;
+            l.vy[tid] = uy;
+            l.vp[tid] = up;
+            double mx = dt * ux, my = dt * uy;
+            const double m2 = mx * mx + my * my;
+            if (m2 > a.fire.max_move * a.fire.max_move) {
+              const double sc = a.fire.max_move / sqrt(m2);
+              mx *= sc;
+              my *= sc;
+            }
+            x += mx;
+            y += my;
+            phi += dt * up * isq;
+          }
+        }
+      }
+      // the sum slot after next (its sums have been read by all: those of the
+      // exchange before this one are in)
+      if (nsum > 1 && lane64 < 4)
+        word_store(sums + ((size_t)((xch + 2) % 3) * a.nseats * kTeamUpdWaves + me * nuw + wave) * 4 +
+                       lane64,
+                   kEmpty);
+    }
+    // ---- the new positions
+    if (upd && moved) {
+      double wx = x, wy = y;
+      const bool okx = wrap_coord(wx, Lx), oky = wrap_coord(wy, Ly);
+      int need = 0;
+      if (!okx || !oky || !isfinite(phi)) {
+        atomicOr(a.err, kErrNonFinite);
+        need = kFlagStop;
+      }
+      if (!(kHeun && predicted)) {  // a predicted state stays unwrapped
+        x = wx;
+        y = wy;
+      }
+      double sn, cs;
+      rod_sincos(phi, &sn, &cs);
+      const double nx = l.A[tid] * cs, ny = l.A[tid] * sn;
+      if (kHeun) stores_done();  // empty marks of this pass
+      publish(pass + 1, x, y, nx, ny);
+      l.x[tid] = x;
+      l.y[tid] = y;
+      l.nx[tid] = nx;
+      l.ny[tid] = ny;
+      l.phi[tid] = phi;
+      const double dx = fabs(min_image(x - l.xb[tid], Lx)), dy = fabs(min_image(y - l.yb[tid], Ly));
+      const bool late = kHeun && T > 1;  // the answer comes one pass late
+      if (fmax(dx, dy) >= (late ? 0.6 * hs : hs)) need |= kFlagRebuild;
+      if (late && fmax(dx, dy) >= hs) need |= kFlagFast;
+      if (need) atomicOr(&s_need, need);
+    }
+    ++xch;
+    __syncthreads();  // new coordinates, s_need, s_next and s_fail visible
+    if (!kHeun) {
+      if (s_fail) {
+        if (tid == 0) give_up(pass == 0 ? kTeamAbsent : kTeamStalled);
+        return;
+      }
+      const int next = s_next;
+      if (next == kAgain) {  // the same positions with new rows
+        build = true;
+        continue;
+      }
+      ++steps;
+      if (next == kDone) break;  // finished at the state just evaluated
+    }
+    was_built = built;
+    ++pass;
+    if (steps == a.max_steps && !predicted) break;
+    if (kHeun && T > 1 && tid == 0) put_flag(pass & 3, (unsigned)pass + 1, s_need);
+  }
+  if (kHeun && T > 1 && pass > 0 && !s_over && steps == a.max_steps) {
+    // the last evaluated pass had valid rows on every member
+    gather_flags((pass - 1) & 3, (unsigned)pass, kStall);
+    __syncthreads();
+    if (s_fail || ((s_bits & kFlagFast) && !was_built)) {
+      if (tid == 0) give_up(s_fail ? kTeamStalled : kTeamFast);
+      return;
+    }
+  }
+  __syncthreads();
+  if (upd) {
+    const bool back = kHeun && predicted;  // left inside a step: to its start
+    const double x = back ? l.ox[tid] : l.x[tid], y = back ? l.oy[tid] : l.y[tid];
+    const double phi = back ? l.op[tid] : l.phi[tid];
+    double sn, cs;
+    rod_sincos(phi, &sn, &cs);
+    b.x[gu] = x;
+    b.y[gu] = y;
+    b.phi[gu] = phi;
+    b.nx[gu] = l.A[tid] * cs;
+    b.ny[gu] = l.A[tid] * sn;
+    if (kFire) {
+      b.vx[gu] = l.vx[tid];
+      b.vy[gu] = l.vy[tid];
+      b.vpsi[gu] = l.vp[tid];
+    }
+    b.fx[gu] = l.fx[tid];
+    b.fy[gu] = l.fy[tid];
+    b.tau[gu] = l.tq[tid];
+  }
+  if (me == 0 && tid == 0) a.scal[pk] = s_S[kHeun ? 0 : steps & 1];
+}
+
+#define SC_TEAM_INST(M, H)                                      \
+  template __global__ void k_team<M, false, false, H>(TeamArgs); \
+  template __global__ void k_team<M, true, false, H>(TeamArgs);  \
+  template __global__ void k_team<M, false, true, H>(TeamArgs);  \
+  template __global__ void k_team<M, true, true, H>(TeamArgs);
+#define SC_TEAM_INST_SHAPE(H)                                              \
+  SC_TEAM_INST(kTeamFire, H)                                               \
+  SC_TEAM_INST(kTeamGd, H)                                                 \
+  SC_TEAM_INST(kTeamHeun, H)                                               \
+  template __global__ void k_team<kTeamHeunSe, false, false, H>(TeamArgs); \
+  template __global__ void k_team<kTeamHeunSe, true, false, H>(TeamArgs);
+SC_TEAM_INST_SHAPE(0)
+SC_TEAM_INST_SHAPE(1)
+#undef SC_TEAM_INST_SHAPE
+#undef SC_TEAM_INST
+
+}  // namespace sc

@@ -343,9 +343,10 @@ class System:
         self._ck(self.lib.sc_set_graphs(self.h, int(bool(enable))))
 
     def set_small_fire(self, max_particles, steps_per_launch=0):
-        """FIRE of packings of at most max_particles (<= 256; 0: never) in one
-        launch once every running packing is that small, at most
-        steps_per_launch iterations per launch (0: the default, 50000)."""
+        """Teams of workgroups that run many steps in one launch, where they fit
+        the GPU (max_particles > 0, at most 256), or launches for every step
+        (0); at most steps_per_launch minimiser iterations per launch (0: the
+        default, 50000)."""
         self._ck(self.lib.sc_set_small_fire(self.h, int(max_particles), int(steps_per_launch)))
 
     def contact_model(self):
