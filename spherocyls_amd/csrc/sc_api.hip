@@ -1105,6 +1105,7 @@ int sc_system_create(sc_system** out, int device, int npack, const int* offsets,
       }
       s->filled[k] = filled;
       P.pad = pad[k];
+      P.reach = 2.0 * (s->Rmax[k] + s->Amax[k]);
       cell_grid(L[k], L[k], s->Rmax[k], s->Amax[k], P.pad, P.rows, P.cols);
       PackScal& S = s->scal[k];
       S.Lx = S.Ly = L[k];
@@ -1132,7 +1133,7 @@ int sc_system_create(sc_system** out, int device, int npack, const int* offsets,
     s->d_nbr = s->dalloc<int>((size_t)kNbrCap * ntot);
     s->d_nbr_n = s->dalloc<int>(ntot);
     HIPCK(hipMemsetAsync(s->d_nbr_n, 0, sizeof(int) * ntot, s->stream));
-    s->d_list_center = s->dalloc<double>(npack);
+    s->d_list_center = s->dalloc<double>((size_t)3 * npack);
     for (int i = 0; i < 3; ++i) {
       s->d_flag[i] = s->dalloc<int>(npack);
       HIPCK(hipMemsetAsync(s->d_flag[i], 0, sizeof(int) * npack, s->stream));
@@ -1549,6 +1550,7 @@ int sc_resize_steps(sc_system* s, int nsteps, int shrink, int corrected_image, i
     int st2 = reconfigure_if_needed(s, &Lm);
     if (st2 != SC_OK) return st2;
   }
+  force_rebuild(s);  // rows kept over box changes are valid for resize passes only
   force_pass(s, false, se_every);
   copy_se_out(s, nrec, se_out);
   int e = check_errors(s);

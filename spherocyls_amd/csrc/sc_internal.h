@@ -46,6 +46,7 @@ struct PackInfo {
   double dt, strain_rate, resize_rate;
   double resize_scale;   // (1 - resize_rate)^dt, the box scale of one resize step
   double inv_2n;         // 1 / (2N), energy normalisation
+  double reach;          // 2 (Rmax + Amax): contact distance of the largest pair
 };
 
 // Mutable per-packing scalars, double-buffered: a kernel that advances a
@@ -144,7 +145,7 @@ struct ListArgs {
   int* nbr;                // [kNbrCap][ntot] partner indices
   int* nbr_n;              // [ntot]
   double *xb, *yb;         // positions at the last list build
-  double* list_center;     // [npack] strain at the last list build
+  double* list_center;     // [npack][3] strain and box (Lx, Ly) at the last list build
   const int* flag_in;      // [npack] rebuild before evaluating
   int* flag_out;           // [npack] raised for the next force pass
   int* flag_clear;         // [npack] zeroed here (written by the pass after next)

@@ -56,7 +56,7 @@ constexpr Layout make_layout() {
   l.pblocks = o; o = up256(o + sizeof(int2) * kNaMaxBlocks);
   l.ranges = o; o = up256(o + sizeof(int2));
   l.words = o; o = up256(o + sizeof(int) * 4);  // [0] rebuild flag, [1] error bits
-  l.center = o; o = up256(o + sizeof(double));
+  l.center = o; o = up256(o + 3 * sizeof(double));
   l.pack_sum = o; o = up256(o + sizeof(double) * kNSum);
   l.part = o; o = up256(o + sizeof(double) * kNSum * kNaMaxBlocks);
   l.cnt = o; o = up256(o + sizeof(int) * kNaMaxCells);
