@@ -160,7 +160,8 @@ struct sc_system {
   int* d_perm = nullptr;
   Bank bank[2]{};
   int cur_bank = 0;
-  double *d_px = nullptr, *d_py = nullptr, *d_pphi = nullptr, *d_pnx = nullptr, *d_pny = nullptr;
+  Pos d_px, d_py, d_pnx, d_pny;
+  double* d_pphi = nullptr;
   double *d_v0x = nullptr, *d_v0y = nullptr, *d_v0t = nullptr;
   int* d_pack_of = nullptr;
   double* d_tile_part = nullptr;
@@ -384,11 +385,20 @@ void alloc_pblocks(sc_system* s) {
   s->d_list_part = s->dalloc<double>((size_t)s->npblocks * kNSum);
 }
 
+void alloc_positions(sc_system* s, Pos& x, Pos& y, Pos& nx, Pos& ny) {
+  x.p = s->dalloc<double>(4 * (size_t)s->ntot);
+  y.p = x.p + 1;
+  nx.p = x.p + 2;
+  ny.p = x.p + 3;
+}
+
 Bank alloc_bank(sc_system* s) {
   Bank b{};
   size_t n = s->ntot;
-  for (double** p : {&b.x, &b.y, &b.phi, &b.R, &b.A, &b.I, &b.RC, &b.fx, &b.fy, &b.tau, &b.vx,
-                     &b.vy, &b.vpsi, &b.nx, &b.ny})
+  alloc_positions(s, b.x, b.y, b.nx, b.ny);
+  b.R.p = s->dalloc<double>(2 * n);
+  b.A.p = b.R.p + 1;
+  for (double** p : {&b.phi, &b.I, &b.RC, &b.fx, &b.fy, &b.tau, &b.vx, &b.vy, &b.vpsi})
     *p = s->dalloc<double>(n);
   b.id = s->dalloc<int>(n);
   for (double* p : {b.fx, b.fy, b.tau, b.vx, b.vy, b.vpsi})
@@ -1122,8 +1132,8 @@ int sc_system_create(sc_system** out, int device, int npack, const int* offsets,
     HIPCK(hipMemsetAsync(s->d_err, 0, sizeof(int), s->stream));
     s->bank[0] = alloc_bank(s);
     s->bank[1] = alloc_bank(s);
-    for (double** p : {&s->d_px, &s->d_py, &s->d_pphi, &s->d_pnx, &s->d_pny, &s->d_v0x, &s->d_v0y,
-                       &s->d_v0t, &s->d_xb, &s->d_yb})
+    alloc_positions(s, s->d_px, s->d_py, s->d_pnx, s->d_pny);
+    for (double** p : {&s->d_pphi, &s->d_v0x, &s->d_v0y, &s->d_v0t, &s->d_xb, &s->d_yb})
       *p = s->dalloc<double>(ntot);
     s->d_pack_of = s->dalloc<int>(ntot);
     s->d_perm = s->dalloc<int>(ntot);
@@ -1150,13 +1160,19 @@ int sc_system_create(sc_system** out, int device, int npack, const int* offsets,
 
     Bank& b = s->bank[0];
     auto up = [&](double* d, const std::vector<double>& h) {
-      HIPCK(hipMemcpyAsync(d, h.data(), sizeof(double) * ntot, hipMemcpyHostToDevice, s->stream));
+      HIPCK(hipMemcpyAsync(d, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice,
+                           s->stream));
     };
-    up(b.x, hx);
-    up(b.y, hy);
+    std::vector<double> pos(4 * (size_t)ntot), size(2 * (size_t)ntot);
+    for (int i = 0; i < ntot; ++i) {
+      pos[4 * (size_t)i] = hx[i];
+      pos[4 * (size_t)i + 1] = hy[i];
+      size[2 * (size_t)i] = hR[i];
+      size[2 * (size_t)i + 1] = hA[i];
+    }
+    up(b.x.p, pos);
+    up(b.R.p, size);
     up(b.phi, hp);
-    up(b.R, hR);
-    up(b.A, hA);
     up(b.I, hI);
     up(b.RC, hRC);
     HIPCK(hipMemcpyAsync(b.id, hid.data(), sizeof(int) * ntot, hipMemcpyHostToDevice, s->stream));

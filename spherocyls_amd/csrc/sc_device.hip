@@ -614,7 +614,8 @@ __global__ void __launch_bounds__(256) k_update(UpdateArgs u) {
   const int g = ub.y + tid;
   const bool own = g < P.poff + P.n;
   const int gl = own ? g : P.poff;
-  double x = b.x[gl], y = b.y[gl], p = b.phi[gl];
+  const double2 xy = load2(b.x, gl);
+  double x = xy.x, y = xy.y, p = b.phi[gl];
   const double Fx = b.fx[gl], Fy = b.fy[gl], Tq = b.tau[gl], Ig = b.I[gl];
   const double Ag = b.A[gl];
   double vx = 0.0, vy = 0.0, vp = 0.0;
@@ -734,13 +735,11 @@ __global__ void __launch_bounds__(256) k_update(UpdateArgs u) {
     }
     bool okx = wrap_coord(x, Lx), oky = wrap_coord(y, Ly);
     if (!okx || !oky || !isfinite(p)) atomicOr(u.err, kErrNonFinite);
-    b.x[g] = x;
-    b.y[g] = y;
+    store2(b.x, g, x, y);
     b.phi[g] = p;
     double sn, cs;
     rod_sincos(p, &sn, &cs);
-    b.nx[g] = Ag * cs;
-    b.ny[g] = Ag * sn;
+    store2(b.nx, g, Ag * cs, Ag * sn);
     bin_c = cell_of(x, y, Lx, Ly, P);
     if (u.flag_out) {
       const double hs = 0.5 * P.pad;  // list skin = the packing's cell padding
@@ -843,19 +842,19 @@ __global__ void k_gather(Bank src, Bank dst, const int* perm, int ntot, int with
   // after a bucket overflow the permutation has holes (the overflow is reported
   // to the host); keep every read in bounds regardless
   if (s < 0 || s >= ntot) s = d;
-  dst.x[d] = src.x[s];
-  dst.y[d] = src.y[s];
+  const double2 xy = load2(src.x, s);
+  store2(dst.x, d, xy.x, xy.y);
   dst.phi[d] = src.phi[s];
-  dst.R[d] = src.R[s];
-  dst.A[d] = src.A[s];
+  const double2 ra = load2(src.R, s);
+  store2(dst.R, d, ra.x, ra.y);
   dst.I[d] = src.I[s];
   dst.RC[d] = src.RC[s];
   dst.fx[d] = src.fx[s];
   dst.fy[d] = src.fy[s];
   dst.tau[d] = src.tau[s];
   dst.id[d] = src.id[s];
-  dst.nx[d] = src.nx[s];
-  dst.ny[d] = src.ny[s];
+  const double2 n = load2(src.nx, s);
+  store2(dst.nx, d, n.x, n.y);
   if (with_velocity) {
     dst.vx[d] = src.vx[s];
     dst.vy[d] = src.vy[s];

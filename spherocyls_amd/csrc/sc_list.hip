@@ -77,9 +77,10 @@ __device__ __forceinline__ void row_from_bucket(const ListArgs& a, const int* sl
   for (int k = 0; k < W; ++k) {
     const int q = val[k];
     if (k < m && q != g) {
-      const double reach = reach_i + a.b.R[q] + a.b.A[q];
-      const double dy = min_image(yi - a.ey[q], Ly);
-      const double dx = min_image(xi - a.ex[q], Lx);
+      const double2 xy = load2(a.ex, q), ra = load2(a.b.R, q);
+      const double reach = reach_i + ra.x + ra.y;
+      const double dy = min_image(yi - xy.y, Ly);
+      const double dx = min_image(xi - xy.x, Lx);
       const double flo = dx + glo * dy, fhi = dx + ghi * dy;
       if (fabs(dy) < reach + s && (fabs(flo) < reach + sx || fabs(fhi) < reach + sx)) {
         if (n < kNbrCap) a.nbr[(size_t)n * a.ntot + g] = q;
@@ -260,9 +261,10 @@ __global__ void __launch_bounds__(256)
   for (int i = 0; i < (kSums ? kNSum : 1); ++i) acc[i] = 0.0;
 
   if (active) {
-    const double xi = a.ex[g], yi = a.ey[g];
-    const double nxi = a.enx[g], nyi = a.eny[g];
-    const double Ri = a.b.R[g], Ai = a.b.A[g];
+    const double2 xyi = load2(a.ex, g), ni = load2(a.enx, g), rai = load2(a.b.R, g);
+    const double xi = xyi.x, yi = xyi.y;
+    const double nxi = ni.x, nyi = ni.y;
+    const double Ri = rai.x, Ai = rai.y;
     const int idi = a.b.id[g];
     const double reach_i = Ri + Ai;
 
@@ -311,9 +313,10 @@ __global__ void __launch_bounds__(256)
         double xq[kGather], yq[kGather], Sq[kGather];
 #pragma unroll
         for (int j = 0; j < kGather; ++j) {
-          xq[j] = a.ex[qs[j]];
-          yq[j] = a.ey[qs[j]];
-          Sq[j] = a.b.R[qs[j]] + a.b.A[qs[j]];
+          const double2 xy = load2(a.ex, qs[j]), ra = load2(a.b.R, qs[j]);
+          xq[j] = xy.x;
+          yq[j] = xy.y;
+          Sq[j] = ra.x + ra.y;
         }
 #pragma unroll
         for (int j = 0; j < kGather; ++j) {
@@ -329,9 +332,10 @@ __global__ void __launch_bounds__(256)
       }
       for (int h = 0; h < nh; ++h) {
         const int q = s_hit[h * nthr + tid];
-        pair_into<kSums && SE, TWO_POINT>(xi, yi, nxi, nyi, Ri, Ai, idi, a.ex[q], a.ey[q], a.enx[q],
-                                    a.eny[q], a.b.R[q], a.b.A[q], a.b.id[q], Lx, Ly, gam, fp64,
-                                    do_se, Fx, Fy, Tq, acc);
+        const double2 xy = load2(a.ex, q), nq = load2(a.enx, q), ra = load2(a.b.R, q);
+        pair_into<kSums && SE, TWO_POINT>(xi, yi, nxi, nyi, Ri, Ai, idi, xy.x, xy.y, nq.x, nq.y,
+                                          ra.x, ra.y, a.b.id[q], Lx, Ly, gam, fp64, do_se, Fx, Fy,
+                                          Tq, acc);
       }
       if (k0 >= n) break;
     }
@@ -420,13 +424,11 @@ __global__ void __launch_bounds__(256)
           qy /= P.resize_scale;
         }
       }
-      a.px[g] = qx;
-      a.py[g] = qy;
+      store2(a.px, g, qx, qy);
       a.pphi[g] = qp;
       double sn, cs;
       rod_sincos(qp, &sn, &cs);
-      a.pnx[g] = Ai * cs;
-      a.pny[g] = Ai * sn;
+      store2(a.pnx, g, Ai * cs, Ai * sn);
       a.v0x[g] = v0x;
       a.v0y[g] = v0y;
       a.v0t[g] = v0t;
@@ -444,14 +446,15 @@ __global__ void __launch_bounds__(256)
                                 fabs(min_image(qy - ybi, Lby)) >= half_skin) ||
               fabs(gnext - center) >= a.gamma_window || box_pure;
     } else {  // kModeCorr
-      double x1 = a.b.x[g], y1 = a.b.y[g], p1 = a.b.phi[g];
+      const double2 xy0 = load2(a.b.x, g);
+      double x1 = xy0.x, y1 = xy0.y, p1 = a.b.phi[g];
       double Lbx = Lx, Lby = Ly;
       bool remap = false;
       if (box_pure) {
         // pure_heun_corr_2p (src/cuda/2point_dynamics.cu:2141-2166): the
         // predicted state plus half the change of the force part
-        x1 = a.px[g] + 0.5 * dt * (Fx - a.v0x[g]);
-        y1 = a.py[g] + 0.5 * dt * (Fy - a.v0y[g]);
+        x1 = xi + 0.5 * dt * (Fx - a.v0x[g]);  // (the pass evaluated px, py)
+        y1 = yi + 0.5 * dt * (Fy - a.v0y[g]);
         p1 = a.pphi[g] + 0.5 * dt * (Tq / a.b.I[g] - a.v0t[g]);
         Lbx = L_new_x;
         Lby = L_new_y;
@@ -496,13 +499,11 @@ __global__ void __launch_bounds__(256)
       }
       bool okx = wrap_coord(x1, Lbx), oky = wrap_coord(y1, Lby);
       if (!okx || !oky || !isfinite(p1)) atomicOr(a.err, kErrNonFinite);
-      a.b.x[g] = x1;
-      a.b.y[g] = y1;
+      store2(a.b.x, g, x1, y1);
       a.b.phi[g] = p1;
       double sn, cs;
       rod_sincos(p1, &sn, &cs);
-      a.b.nx[g] = Ai * cs;
-      a.b.ny[g] = Ai * sn;
+      store2(a.b.nx, g, Ai * cs, Ai * sn);
       bin_into(g, x1, y1, Lbx, Lby, P, a.cnt_fill, a.slot_fill, a.err);
       double gnext = box_pure || box_resize ? S.gamma : S.gamma + gd * dt;
       if (remap) gnext -= le_ratio;

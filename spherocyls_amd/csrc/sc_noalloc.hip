@@ -43,7 +43,7 @@ constexpr int kNaMaxBlocks = (kNaMaxN + kNaBlock - 1) / kNaBlock;
 // Byte layout of the scratch array (each region 256-byte aligned).
 struct Layout {
   size_t info, scal, pblocks, ranges, words, center, pack_sum, part, cnt, slot;
-  size_t x, y, nx, ny, xb, yb, id, pack_of, nbr_n, nbr, total;
+  size_t pos, size, xb, yb, id, pack_of, nbr_n, nbr, total;
 };
 
 constexpr size_t up256(size_t v) { return (v + 255) / 256 * 256; }
@@ -61,10 +61,8 @@ constexpr Layout make_layout() {
   l.part = o; o = up256(o + sizeof(double) * kNSum * kNaMaxBlocks);
   l.cnt = o; o = up256(o + sizeof(int) * kNaMaxCells);
   l.slot = o; o = up256(o + sizeof(int) * kNaMaxCells * kCapMin);
-  l.x = o; o = up256(o + sizeof(double) * kNaMaxN);
-  l.y = o; o = up256(o + sizeof(double) * kNaMaxN);
-  l.nx = o; o = up256(o + sizeof(double) * kNaMaxN);
-  l.ny = o; o = up256(o + sizeof(double) * kNaMaxN);
+  l.pos = o; o = up256(o + 4 * sizeof(double) * kNaMaxN);   // records (x, y, nx, ny)
+  l.size = o; o = up256(o + 2 * sizeof(double) * kNaMaxN);  // records (R, A)
   l.xb = o; o = up256(o + sizeof(double) * kNaMaxN);
   l.yb = o; o = up256(o + sizeof(double) * kNaMaxN);
   l.id = o; o = up256(o + sizeof(int) * kNaMaxN);
@@ -152,17 +150,20 @@ __global__ void __launch_bounds__(256) k_na_setup(unsigned char* base, int n, do
 // Copy of the caller's positions (binning wraps them), segment vectors, the
 // identity ids and packing map, and zeroed bucket counts of the grid.
 __global__ void k_na_prepare(unsigned char* base, int n, const double* x, const double* y,
-                             const double* phi, const double* A) {
+                             const double* phi, const double* R, const double* A) {
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   const PackInfo& P = *at<PackInfo>(base, kLay.info);
   if (g < P.rows * P.cols) at<int>(base, kLay.cnt)[g] = 0;
   if (g >= n) return;
-  at<double>(base, kLay.x)[g] = x[g];
-  at<double>(base, kLay.y)[g] = y[g];
+  double* pos = at<double>(base, kLay.pos) + 4 * (size_t)g;
+  pos[0] = x[g];
+  pos[1] = y[g];
   double sn, cs;
   rod_sincos(phi[g], &sn, &cs);
-  at<double>(base, kLay.nx)[g] = A[g] * cs;
-  at<double>(base, kLay.ny)[g] = A[g] * sn;
+  pos[2] = A[g] * cs;
+  pos[3] = A[g] * sn;
+  at<double>(base, kLay.size)[2 * g] = R[g];
+  at<double>(base, kLay.size)[2 * g + 1] = A[g];
   at<int>(base, kLay.id)[g] = g;
   at<int>(base, kLay.pack_of)[g] = 0;
 }
@@ -222,15 +223,16 @@ extern "C" int sc_calc_se_noalloc(int n, double L, double gamma, double pad, int
     hipLaunchKernelGGL(k_na_setup, dim3(1), dim3(256), 0, sm, base, n, L, gamma, pad, A, R,
                        nblocks);
     const int nprep = (std::max(n, kNaMaxCells) + 255) / 256;
-    hipLaunchKernelGGL(k_na_prepare, dim3(nprep), dim3(256), 0, sm, base, n, x, y, phi, A);
+    hipLaunchKernelGGL(k_na_prepare, dim3(nprep), dim3(256), 0, sm, base, n, x, y, phi, R,
+                       A);
     Bank b{};
-    b.x = at<double>(base, kLay.x);
-    b.y = at<double>(base, kLay.y);
+    b.x.p = at<double>(base, kLay.pos);
+    b.y.p = b.x.p + 1;
+    b.nx.p = b.x.p + 2;
+    b.ny.p = b.x.p + 3;
+    b.R.p = at<double>(base, kLay.size);
+    b.A.p = b.R.p + 1;
     b.phi = const_cast<double*>(phi);
-    b.R = const_cast<double*>(R);
-    b.A = const_cast<double*>(A);
-    b.nx = at<double>(base, kLay.nx);
-    b.ny = at<double>(base, kLay.ny);
     b.id = at<int>(base, kLay.id);
     b.fx = fx;
     b.fy = fy;
