@@ -125,7 +125,8 @@ struct sc_system {
   int small_max = kSmallMax;  // 0: no teams, launches for every step
   int small_steps = 50000;    // minimiser iterations of a team launch, at most
   // teams (sc_team.hip): exchange words and the launch's seats
-  unsigned long long *d_team_pos = nullptr, *d_team_sums = nullptr, *d_team_flags = nullptr;
+  unsigned long long *d_team_pos = nullptr, *d_team_sums = nullptr, *d_team_flags = nullptr,
+                     *d_team_chunks = nullptr;
   TeamSeat* d_team_seats = nullptr;
   int* d_team_status = nullptr;
   int team_seat_cap = 0;
@@ -901,9 +902,8 @@ bool team_plan(sc_system* s, int mode, const std::vector<int>& want, TeamPlan& p
     for (int k : want) {
       const PackInfo& P = s->packs[k];
       const int team = (P.n + own - 1) / own, per = (P.n + team - 1) / team;
-      // a rebuild's hit masks, 64 particles each, share the rows' LDS
-      fits = (long)plan.seats.size() + team <= room &&
-             P.n + 64 * 8 <= 64 * own * (kTeamRow + 2) / 4;
+      // (a rebuild keeps a word for every run of 64 particles)
+      fits = (long)plan.seats.size() + team <= room && team * ((per + 63) / 64) <= 8 * own;
       if (!fits) break;
       const int base = (int)plan.seats.size();
       int at = 0;
@@ -930,11 +930,13 @@ int run_team(sc_system* s, int mode, const TeamPlan& plan, const FireParams* fp,
   if (nseats > s->team_seat_cap) {
     s->dfree(s->d_team_sums);
     s->dfree(s->d_team_flags);
+    s->dfree(s->d_team_chunks);
     s->dfree(s->d_team_seats);
     s->dfree(s->d_team_status);
     s->d_team_status = s->dalloc<int>(nseats);
     s->d_team_sums = s->dalloc<unsigned long long>((size_t)12 * kTeamUpdWaves * nseats);
     s->d_team_flags = s->dalloc<unsigned long long>((size_t)kTeamFlagSlots * nseats);
+    s->d_team_chunks = s->dalloc<unsigned long long>((size_t)4 * kTeamUpdWaves * nseats);
     s->d_team_seats = s->dalloc<TeamSeat>(nseats);
     s->team_seat_cap = nseats;
   }
@@ -948,6 +950,7 @@ int run_team(sc_system* s, int mode, const TeamPlan& plan, const FireParams* fp,
   a.pos = s->d_team_pos;
   a.sums = s->d_team_sums;
   a.flags = s->d_team_flags;
+  a.chunks = s->d_team_chunks;
   a.status = s->d_team_status;
   a.err = s->d_err;
   if (fp) a.fire = *fp;

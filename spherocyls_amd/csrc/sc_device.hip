@@ -100,8 +100,8 @@ __device__ void finalize_pack(const ReduceArgs& a, int pk, const PackInfo& P, co
   ps[kSumV] = tot[kSumV];
   ps[kSumR2] = tot[kSumR2];
   if (a.do_fire || a.do_gd) {
-    const MinStep m = minimiser_step(a.fire, a.do_fire, P.n, P.inv_2n, S, tot[kSumR2], tot[kSumP],
-                                     tot[kSumG], tot[kSumV], tot[kSeE], true);
+    const MinStep m = minimiser_step(a.fire, a.do_fire, P.n, P.inv_2n, min_state(S), tot[kSumR2],
+                                     tot[kSumP], tot[kSumG], tot[kSumV], tot[kSeE], true);
     advance(a.scal_next[pk], S, m, a.do_fire);
   }
 }
@@ -670,7 +670,7 @@ __global__ void __launch_bounds__(256) k_update(UpdateArgs u) {
       s2 = s_red[2] + s_red[6] + s_red[10] + s_red[14];
       s3 = s_red[3] + s_red[7] + s_red[11] + s_red[15];
     }
-    S = minimiser_step(u.red.fire, fire, P.n, P.inv_2n, S0, s0, s1, s2, s3, s0, false);
+    S = minimiser_step(u.red.fire, fire, P.n, P.inv_2n, min_state(S0), s0, s1, s2, s3, s0, false);
     if (lead && tid == 0) {
       advance(u.red.scal_next[pk], S0, S, fire);
       double* ps = u.red.pack_sum + (size_t)pk * kNSum;

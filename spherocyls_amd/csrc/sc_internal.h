@@ -253,6 +253,7 @@ struct TeamArgs {
   unsigned long long* pos;   // [4][ntot][4] exchanged positions
   unsigned long long* sums;  // [3][nseats][kTeamUpdWaves][4]
   unsigned long long* flags; // [kTeamFlagSlots][nseats]
+  unsigned long long* chunks;  // [nseats][kTeamUpdWaves][4] where 64 own particles are (rebuilds)
   int* status;               // [nseats]: TeamStatus bits at a team's first seat
   int* err;
   FireParams fire;

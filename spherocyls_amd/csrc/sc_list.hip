@@ -339,9 +339,11 @@ __global__ void __launch_bounds__(256)
       }
       if (k0 >= n) break;
     }
-    Fx = group_sum(Fx, LANES);
-    Fy = group_sum(Fy, LANES);
-    Tq = group_sum(Tq, LANES);
+    double F[3] = {Fx, Fy, Tq};
+    group_sum(F, LANES);
+    Fx = F[0];
+    Fy = F[1];
+    Tq = F[2];
     // ---- per-particle epilogue (lane 0)
     const double half_skin = 0.5 * P.pad;
     // build position of the row (written above by this lane when it rebuilt

@@ -587,22 +587,44 @@ struct MinStep {
   int end;                         // 0: go on, 1: converged, 2: FIRE at max_iter
 };
 
-// S: the scalars the force pass evaluated; R2, Pw, G, V: FIRE's sums; E: the
+// What the step depends on besides the sums.
+struct MinState {
+  double dt, alpha, npos;
+  int step, prec;
+};
+__device__ __forceinline__ MinState min_state(const PackScal& S) {
+  return MinState{S.fire_dt, S.fire_alpha, S.fire_npos, S.step, S.prec};
+}
+
+// S: the state the force pass evaluated; R2, Pw, G, V: FIRE's sums; E: the
 // gradient descent's energy sum.  residual: frms is wanted in any case.
 __device__ __forceinline__ MinStep minimiser_step(const FireParams& fp, bool do_fire, int n,
-                                                  double inv_2n, const PackScal& S, double R2,
+                                                  double inv_2n, const MinState& S, double R2,
                                                   double Pw, double G, double V, double E,
                                                   bool residual) {
 #pragma clang fp contract(off)
   MinStep m;
-  const int step = S.step;
-  const bool last = step >= (int)fp.max_iter;
-  double dt = S.fire_dt, alpha = S.fire_alpha, npos = S.fire_npos;
-  m.dt_old = dt;
+  const bool last = S.step >= (int)fp.max_iter;
+  m.dt_old = m.dt = S.dt;
+  m.alpha = S.alpha;
+  m.npos = S.npos;
   m.c_keep = m.c_force = m.frms = 0.0;
   m.mix = m.end = 0;
   m.prec = S.prec;
   if (do_fire) {
+    // Selects, not branches: every step takes this path and waits for it.
+    const bool up = Pw >= 0;
+    const double root = sqrt(V / G);  // NaN for G = 0, not used then
+    const double npos = S.npos + 1;
+    const bool grow = npos > fp.n_min;
+    const double dt_up = grow ? fmin(S.dt * fp.f_inc, fp.dt_max) : S.dt;
+    const double alpha_up = grow ? S.alpha * fp.f_alpha : S.alpha;
+    m.mix = up ? 1 : 0;
+    m.c_keep = up ? 1.0 - S.alpha : 0.0;
+    m.c_force = up && G > 0 ? S.alpha * root : 0.0;
+    m.npos = up ? npos : 0.0;
+    m.dt = up ? dt_up : S.dt * fp.f_dec;
+    m.alpha = up ? alpha_up : fp.alpha0;
     // Convergence is judged on FP64 pair forces only: a packing still on FP32
     // pair math whose residual falls below max(switch_frms, ftol) moves to FP64
     // and keeps iterating.  The root is taken only where F_rms may be below a
@@ -615,29 +637,17 @@ __device__ __forceinline__ MinStep minimiser_step(const FireParams& fp, bool do_
       else if (last) m.end = 2;
       else if (fp32 && m.frms < lim) m.prec = kFP64;
     }
-    if (Pw >= 0) {
-      m.mix = 1;
-      m.c_keep = 1.0 - alpha;
-      m.c_force = (G > 0) ? alpha * sqrt(V / G) : 0.0;
-      npos += 1;
-      if (npos > fp.n_min) {
-        dt = fmin(dt * fp.f_inc, fp.dt_max);
-        alpha = alpha * fp.f_alpha;
-      }
-    } else {
-      dt = dt * fp.f_dec;
-      alpha = fp.alpha0;
-      npos = 0;
-    }
   } else {
     // gradient-descent passes always record energy: E / (2N)
     if (residual) m.frms = sqrt(R2 / (3.0 * n));
     if (E * inv_2n <= fp.emin || last) m.end = 1;
   }
-  m.dt = dt;
-  m.alpha = alpha;
-  m.npos = npos;
   return m;
+}
+
+// The state after that step.
+__device__ __forceinline__ MinState after(const MinState& S, const MinStep& m) {
+  return m.end ? S : MinState{m.dt, m.alpha, m.npos, S.step + 1, m.prec};
 }
 
 // The scalars after that step (the storing thread).
@@ -687,7 +697,7 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
-// Sum over the L lanes (1, 2, 4 or 8, aligned) that share a particle, in all of
+// Sums over the L lanes (1, 2, 4 or 8, aligned) that share a particle, in all of
 // them, as the tree lane ^ 4, ^ 2, ^ 1.  Data-parallel-primitive moves instead
 // of shuffles, which are LDS round trips: lanes four apart by row shifts (a
 // half row's lower bank takes the upper one's values and the other way), then
@@ -700,31 +710,77 @@ template <int CTRL>
 __device__ __forceinline__ int dpp_quad(int v) {
   return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false);
 }
-__device__ __forceinline__ double group_sum(double v, int L) {
+__device__ __forceinline__ void group_sum(double (&v)[3], int L) {
   auto join = [](int lo, int hi) {
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
   };
-  if (L >= 8) {
-    const long long u = __double_as_longlong(v);
-    v += join(dpp_xor4((int)u), dpp_xor4((int)(u >> 32)));
-  }
-  if (L >= 4) {  // lanes 2 3 0 1
-    const long long u = __double_as_longlong(v);
-    v += join(dpp_quad<0x4e>((int)u), dpp_quad<0x4e>((int)(u >> 32)));
-  }
-  if (L >= 2) {  // lanes 1 0 3 2
-    const long long u = __double_as_longlong(v);
-    v += join(dpp_quad<0xb1>((int)u), dpp_quad<0xb1>((int)(u >> 32)));
-  }
-  return v;
+  if (L >= 8)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const long long u = __double_as_longlong(v[i]);
+      v[i] += join(dpp_xor4((int)u), dpp_xor4((int)(u >> 32)));
+    }
+  if (L >= 4)  // lanes 2 3 0 1
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const long long u = __double_as_longlong(v[i]);
+      v[i] += join(dpp_quad<0x4e>((int)u), dpp_quad<0x4e>((int)(u >> 32)));
+    }
+  if (L >= 2)  // lanes 1 0 3 2
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const long long u = __double_as_longlong(v[i]);
+      v[i] += join(dpp_quad<0xb1>((int)u), dpp_quad<0xb1>((int)(u >> 32)));
+    }
 }
 
-// The value in lane 63, as a scalar.
-__device__ __forceinline__ double last_lane(double v) {
+// The value in lane `lane`, as a scalar.
+__device__ __forceinline__ double lane_value(double v, int lane) {
   const long long u = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)u, 63);
-  const int hi = __builtin_amdgcn_readlane((int)(u >> 32), 63);
+  const int lo = __builtin_amdgcn_readlane((int)u, lane);
+  const int hi = __builtin_amdgcn_readlane((int)(u >> 32), lane);
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// Sum of v over the lanes with this lane's last two bits, valid in lanes 12-15
+// of every row of 16.
+__device__ __forceinline__ double quad_sum(double v) {
+  v = dpp_add<0x114, 0xf>(v);  // row_shr:4
+  v = dpp_add<0x118, 0xf>(v);  // row_shr:8
+  v += __shfl_xor(v, 16);
+  v += __shfl_xor(v, 32);
+  return v;
+}
+// Sums of four values over the wavefront, value i in lanes 12 + i (mod 16): two
+// exchanges within quads leave each lane with one value, so the rest is a
+// single tree instead of four.
+__device__ __forceinline__ double four_sums(double a, double b, double c, double d) {
+  auto quad = [](double v, bool two) {
+    const long long u = __double_as_longlong(v);
+    const int lo = two ? dpp_quad<0x4e>((int)u) : dpp_quad<0xb1>((int)u);
+    const int hi = two ? dpp_quad<0x4e>((int)(u >> 32)) : dpp_quad<0xb1>((int)(u >> 32));
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+  };
+  const bool odd = threadIdx.x & 1, high = threadIdx.x & 2;
+  const double ab = (odd ? b : a) + quad(odd ? a : b, false);
+  const double cd = (odd ? d : c) + quad(odd ? c : d, false);
+  return quad_sum((high ? cd : ab) + quad(high ? ab : cd, true));
+}
+
+// OR of v over the wavefront, valid in lane 63.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned long long dpp_or(unsigned long long v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), CTRL, ROWS, 0xf, false);
+  return v | ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo;
+}
+__device__ __forceinline__ unsigned long long wave_or(unsigned long long v) {
+  v = dpp_or<0x111, 0xf>(v);
+  v = dpp_or<0x112, 0xf>(v);
+  v = dpp_or<0x114, 0xf>(v);
+  v = dpp_or<0x118, 0xf>(v);
+  v = dpp_or<0x142, 0xa>(v);
+  return dpp_or<0x143, 0xc>(v);
 }
 
 // Sums of v over the workgroup in wavefront order, in s_red[0 .. NV) for every

@@ -48,9 +48,15 @@
 // Measured, all-gather of 4 words by G workgroups over all XCDs: 1.05 us (G = 2),
 // 1.5 (16), 1.8 (64), 2.0 (128), 2.8 (256); an empty kernel in a captured graph
 // takes 1.65 us.  Against the launches per step, two-point FIRE iterations of
-// 16384 particles 19.5 -> 13.5 us, of 700 15.7 -> 10.1; sheared steps of 16384
-// 21.6 -> 14.6 us, of 512 14.9 -> 11.8; descent of 1000 16.6 -> 9.3.
+// 16384 particles 19.1 -> 12.1 us, of 700 15.4 -> 9.8; sheared steps of 16384
+// 20.8 -> 14.6 us, of 512 14.3 -> 11.9; descent of 1000 16.4 -> 9.0.
+// Where a FIRE pass of 16384 (11 us, 26k cycles) goes: gathering the sums 7.6k,
+// pair math 3.0k, rebuilds 3.2k (22 in 381 passes; 4.4k when every member looked
+// at every particle), new positions 1.9k, halo 1.7k, row tests 1.3k, sums 0.9k,
+// decision 0.7k (1.8k by one thread on the whole record of scalars).
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "sc_internal.h"
 #include "sc_physics.h"
@@ -122,7 +128,10 @@ struct TeamLds {
   int halo[CAP];                               // storage index of halo entry e
   union {
     unsigned short row[OWN * kRowStride];      // partners (local indices)
-    u64 hit[OWN * kRowStride / 4];             // rebuild: halo hit masks, 64 particles each
+    struct {                                   // rebuild, by runs of 64 particles
+      u64 hit[8 * OWN];                        // particles in the halo
+      int run[8 * OWN], at[8 * OWN];           // runs looked at; their first halo entry
+    } scan;
   };
   unsigned cells[4];                           // rebuild: marked cells (dynamic)
 };
@@ -140,12 +149,14 @@ size_t team_lds_bytes(int shape, int cell_words) {
 // Empty marks for every word a launch polls, zero flags.
 __global__ void k_team_clear(TeamArgs a) {
   const size_t np = (size_t)kBufs * a.ntot * 4, ns = (size_t)3 * a.nseats * 4 * kTeamUpdWaves,
-               nf = (size_t)kTeamFlagSlots * a.nseats;
+               nf = (size_t)kTeamFlagSlots * a.nseats, nc = (size_t)a.nseats * 4 * kTeamUpdWaves;
   const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < np + ns + nf; i += stride) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < np + ns + nf + nc;
+       i += stride) {
     if (i < np) a.pos[i] = kEmpty;
     else if (i < np + ns) a.sums[i - np] = kEmpty;
-    else a.flags[i - np - ns] = 0;
+    else if (i < np + ns + nf) a.flags[i - np - ns] = 0;
+    else a.chunks[i - np - ns - nf] = 0;
   }
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < a.nseats; i += (int)stride) a.status[i] = 0;
 }
@@ -176,7 +187,6 @@ k_team(TeamArgs a) {
 #pragma clang fp contract(off)
   constexpr bool kHeun = MODE == kTeamHeun || MODE == kTeamHeunSe;
   constexpr bool kFire = MODE == kTeamFire, kGd = MODE == kTeamGd;
-  constexpr int kSums = kFire ? 4 : 1;  // words of a published sum
   extern __shared__ __align__(16) unsigned char lds_raw[];
   __shared__ double s_part[kWaves * kNSe];
   __shared__ int s_count[kWaves];
@@ -186,9 +196,13 @@ k_team(TeamArgs a) {
   // overflow), s_next (what the minimiser does next).
   __shared__ int s_need, s_bits, s_fail, s_over, s_next;
   enum : int { kGoOn = 0, kDone = 1, kAgain = 2 };
-  // Per-packing scalars of iteration k in slot k & 1: thread 0 writes the next
+  // A minimiser's state of iteration k in slot k & 1: thread 0 writes the next
   // iteration's while others still read this one's.
-  __shared__ PackScal s_S[2];
+  __shared__ MinState s_m[2];
+  __shared__ double s_frms;
+  __shared__ int s_end;
+  __shared__ PackScal s_S;                  // thread 0's: Heun strain, and what goes back
+  __shared__ u64 s_near[2];                 // rebuild: rows, columns of cells around own particles
   const int tid0 = threadIdx.x, lane64 = tid0 & 63, wave = tid0 >> 6;
   int tid = tid0;
   const TeamSeat seat = a.seats[blockIdx.x];
@@ -200,6 +214,7 @@ k_team(TeamArgs a) {
   const int cell_words = (P.rows * P.cols + 31) >> 5;
   constexpr int kCap = kTeamCap[SHAPE];
   TeamLds<kTeamOwn[SHAPE], kCap>& l = *reinterpret_cast<TeamLds<kTeamOwn[SHAPE], kCap>*>(lds_raw);
+  double* const lpos = reinterpret_cast<double*>(lds_raw);  // l.x, l.y, l.nx, l.ny, kCap each
   int* const status = a.status + seat.base;  // the team's
   u64* const flags = a.flags + seat.base;    // [slot][member]: slots nseats apart
   u64* const sums = a.sums + (size_t)seat.base * 4 * kTeamUpdWaves;
@@ -237,8 +252,9 @@ k_team(TeamArgs a) {
     if (kHeun) l.rc[tid] = b.RC[gu];
   }
   if (tid == 0) {
-    s_need = s_bits = s_fail = s_over = s_next = 0;
-    s_S[0] = a.scal[pk];
+    s_need = s_bits = s_fail = s_over = s_next = s_end = 0;
+    s_S = a.scal[pk];
+    s_m[0] = min_state(s_S);
   }
   const double Lx = a.scal[pk].Lx, Ly = a.scal[pk].Ly;
   const double le_ratio = Lx / Ly;
@@ -250,42 +266,96 @@ k_team(TeamArgs a) {
   auto record_of = [&](int j, int g) {
     return a.pos + ((size_t)(j & (kBufs - 1)) * a.ntot + g) * 4;
   };
-  // publish an own particle's position as pass j's
-  auto publish = [&](int j, double px, double py, double pnx, double pny) {
-    if (T > 1) {
-      u64* r = record_of(j, gu);
-      word_store(r, bits_of(px));
-      word_store(r + 1, bits_of(py));
-      word_store(r + 2, bits_of(pnx));
-      word_store(r + 3, bits_of(pny));
+  // Large teams move records word by word with four lanes to a record, so that
+  // an instruction touches 16 whole records (512 bytes in a row) and not one
+  // word of 64: all members' words are under way at once (469 members' shear of
+  // 60k particles, 100 passes: 1.81 ms the other way, 1.70 this way; 256
+  // members' FIRE 4.21 and 4.13).  Small teams wait for one trip, which the way
+  // through LDS and the further rounds lengthen (16 members' descent 1.34 and
+  // 1.47 ms), and so do 256 members' sheared steps, whose passes wait for
+  // nothing else (1.47 and 1.58 ms).
+  const bool wide = T >= (kHeun ? 384 : 128);
+  // publish this wavefront's own positions, which it has written to LDS, as
+  // pass j's
+  auto publish = [&](int j) {
+    if (T > 1 && !wide) {
+      if (upd) {
+        u64* r = record_of(j, gu);
+        word_store(r, bits_of(l.x[tid]));
+        word_store(r + 1, bits_of(l.y[tid]));
+        word_store(r + 2, bits_of(l.nx[tid]));
+        word_store(r + 3, bits_of(l.ny[tid]));
+      }
+    } else if (T > 1) {
+      // (x, y, nx, ny lie kCap apart in LDS)
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int i = wave * 64 + k * 16 + (lane64 >> 2), w = tid & 3;
+        if (i < own) word_store(record_of(j, first + i) + w, bits_of(lpos[w * kCap + i]));
+      }
     }
   };
-  auto mark_empty = [&](int j) {
-    if (T > 1 && upd) {
-      u64* r = record_of(j, gu);
+  auto mark_empty = [&](int j) {  // the first nuw wavefronts
+    if (T > 1) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) word_store(r + k, kEmpty);
+      for (int k = 0; k < 4; ++k) {
+        const int i = wave * 64 + k * 16 + (lane64 >> 2);
+        if (i < own) word_store(record_of(j, first + i) + (tid & 3), kEmpty);
+      }
     }
   };
   // halo entries' positions of pass j into LDS
   auto fetch_halo = [&](int j, int H, u64 limit) {
-    for (int e = tid; e < H; e += kTeamThreads) {
-      const u64* r = record_of(j, l.halo[e]);
-      u64 w[4];
+    if (!wide) {
+      for (int e = tid; e < H; e += kTeamThreads) {
+        const u64* r = record_of(j, l.halo[e]);
+        u64 v[4];
+        Wait wait;
+        while (true) {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) v[k] = word_load(r + k);
+          if (v[0] != kEmpty && v[1] != kEmpty && v[2] != kEmpty && v[3] != kEmpty) break;
+          if (wait.over(limit, status)) {
+            s_fail = 1;
+            break;
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) lpos[k * kCap + own + e] = from_bits(v[k]);
+      }
+      return;
+    }
+    constexpr int kAhead = 4;
+    const int w = tid & 3, n4 = 4 * H;
+    for (int i0 = tid; i0 < n4; i0 += kAhead * kTeamThreads) {
+      const u64* r[kAhead];
+      u64 v[kAhead];
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k)
+        if (i0 + k * kTeamThreads < n4) r[k] = record_of(j, l.halo[(i0 + k * kTeamThreads) >> 2]) + w;
       Wait wait;
       while (true) {
+        bool all = true;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) w[k] = word_load(r + k);
-        if (w[0] != kEmpty && w[1] != kEmpty && w[2] != kEmpty && w[3] != kEmpty) break;
+        for (int k = 0; k < kAhead; ++k) {
+          v[k] = 0;
+          if (i0 + k * kTeamThreads < n4) v[k] = word_load(r[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) all = all && v[k] != kEmpty;
+        if (all) break;
         if (wait.over(limit, status)) {
           s_fail = 1;
           break;
         }
       }
-      l.x[own + e] = from_bits(w[0]);
-      l.y[own + e] = from_bits(w[1]);
-      l.nx[own + e] = from_bits(w[2]);
-      l.ny[own + e] = from_bits(w[3]);
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) {
+        const int i = i0 + k * kTeamThreads;
+        if (i < n4) lpos[w * kCap + own + (i >> 2)] = from_bits(v[k]);
+      }
     }
   };
   // every member's flag word numbered seq in slot `slot`, ORed into s_bits
@@ -321,7 +391,7 @@ k_team(TeamArgs a) {
   bool build = true;       // this pass starts with new rows (uniform over the team)
   bool was_built = false;  // Heun: the previous pass did
   bool predicted = false;  // Heun: the positions are a step's predicted ones
-  if (upd) publish(0, l.x[tid], l.y[tid], l.nx[tid], l.ny[tid]);
+  if (wave < nuw) publish(0);
   if (kHeun && T > 1 && tid == 0) put_flag(0, 1, 0);
   __syncthreads();
 
@@ -349,7 +419,7 @@ k_team(TeamArgs a) {
           return;
         }
         build = build || ((bits & kFlagRebuild) && !was_built);
-        if (pass >= 2) mark_empty(pass - 2);
+        if (pass >= 2 && wave < nuw) mark_empty(pass - 2);
       } else {
         build = build || (bits & kFlagRebuild);
       }
@@ -369,36 +439,95 @@ k_team(TeamArgs a) {
       }
       H = 0;
       if (T > 1) {
-        // cells within one of an own particle's
+        ++rebuilds;
+        // Cells within one of an own particle's; and for each run of 64 own
+        // particles the rows and columns of cells (modulo 64) it lies in, for
+        // the other members.
         for (int w = tid; w < cell_words; w += kTeamThreads) l.cells[w] = 0;
+        if (tid < 2) s_near[tid] = 0;
         __syncthreads();
-        if (upd) {
-          double xw = l.x[tid], yw = l.y[tid];
-          wrap_coord(xw, Lx);
-          wrap_coord(yw, Ly);
-          int col, row;
-          cell_col_row(xw, yw, Lx, Ly, P, col, row);
-          for (int d = -1; d <= 1; ++d)
-            for (int e = -1; e <= 1; ++e) {
-              const int c = (row + d + P.rows) % P.rows * P.cols + (col + e + P.cols) % P.cols;
-              atomicOr(&l.cells[c >> 5], 1u << (c & 31));
+        if (wave < nuw) {
+          u64 at_row = 0, at_col = 0, near_row = 0, near_col = 0;
+          if (upd) {
+            double xw = l.x[tid], yw = l.y[tid];
+            wrap_coord(xw, Lx);
+            wrap_coord(yw, Ly);
+            int col, row;
+            cell_col_row(xw, yw, Lx, Ly, P, col, row);
+            at_row = 1ull << (row & 63);
+            at_col = 1ull << (col & 63);
+            for (int d = -1; d <= 1; ++d) {
+              const int r = (row + d + P.rows) % P.rows, c = (col + d + P.cols) % P.cols;
+              near_row |= 1ull << (r & 63);
+              near_col |= 1ull << (c & 63);
+              for (int e = -1; e <= 1; ++e) {
+                const int q = r * P.cols + (col + e + P.cols) % P.cols;
+                atomicOr(&l.cells[q >> 5], 1u << (q & 31));
+              }
             }
+          }
+          at_row = wave_or(at_row);
+          at_col = wave_or(at_col);
+          near_row = wave_or(near_row);
+          near_col = wave_or(near_col);
+          if (lane64 == 63) {
+            u64* c = a.chunks + ((size_t)blockIdx.x * kTeamUpdWaves + wave) * 4;
+            word_store(c, at_row);
+            word_store(c + 1, at_col);
+            stores_done();
+            word_store(c + 2, rebuilds);
+            atomicOr(&s_near[0], near_row);
+            atomicOr(&s_near[1], near_col);
+          }
         }
         __syncthreads();
-        // wavefront w looks at its eighth of the packing, 64 particles at a
-        // time; the words of kAhead looks are in flight together
-        constexpr int kAhead = 8;
-        const int per = (P.n + 64 * kWaves - 1) / (64 * kWaves);
-        int mine = 0;
-        for (int k0 = 0; k0 < per; k0 += kAhead) {
+        // the runs of 64 particles that may reach into those cells, in storage
+        // order (s_count: each wavefront's number of them)
+        const u64 near_row = s_near[0], near_col = s_near[1];
+        int nrun = 0;
+        for (int c0 = 0; c0 < T * nuw; c0 += kTeamThreads) {
+          const int c = c0 + tid, m = c / nuw, part = c - m * nuw;
+          bool look = false;
+          if (c < T * nuw && part * 64 < min(seat.most, P.n - m * seat.most)) {
+            const u64* w = a.chunks + ((size_t)(seat.base + m) * kTeamUpdWaves + part) * 4;
+            Wait wait;
+            while (word_load(w + 2) != rebuilds)
+              if (wait.over(limit, status)) {
+                s_fail = 1;
+                break;
+              }
+            look = m != me && (word_load(w) & near_row) && (word_load(w + 1) & near_col);
+          }
+          const u64 looks = __ballot(look);
+          if (lane64 == 0) s_count[wave] = __popcll(looks);
+          __syncthreads();
+          int to = nrun;
+          for (int w = 0; w < kWaves; ++w) {
+            if (w < wave) to += s_count[w];
+            nrun += s_count[w];
+          }
+          if (look) l.scan.run[to + __popcll(looks & ((1ull << lane64) - 1ull))] = c;
+          __syncthreads();
+        }
+        // their particles in marked cells
+        constexpr int kAhead = 4;
+        auto run_at = [&](int k, int& count) {  // first particle of the packing, and how many
+          const int c = l.scan.run[k], m = c / nuw, part = c - m * nuw;
+          count = min(64, min(seat.most, P.n - m * seat.most) - part * 64);
+          return m * seat.most + part * 64;
+        };
+        for (int k0 = wave; k0 < nrun; k0 += kWaves * kAhead) {
           u64 wx[kAhead], wy[kAhead];
           Wait wait;
           while (true) {
             bool all = true;
 #pragma unroll
             for (int k = 0; k < kAhead; ++k) {
-              const int i = (wave * per + k0 + k) * 64 + lane64;
-              const u64* r = record_of(pass, P.poff + min(i, P.n - 1));
+              wx[k] = wy[k] = 0;
+              if (k0 + k * kWaves >= nrun) continue;
+              int count;
+              const int i = run_at(k0 + k * kWaves, count);
+              const u64* r = record_of(pass, P.poff + i + min(lane64, count - 1));
               wx[k] = word_load(r);
               wy[k] = word_load(r + 1);
             }
@@ -412,35 +541,44 @@ k_team(TeamArgs a) {
           }
 #pragma unroll
           for (int k = 0; k < kAhead; ++k) {
-            if (k0 + k >= per) break;
-            const int i = (wave * per + k0 + k) * 64 + lane64, g = P.poff + i;
+            if (k0 + k * kWaves >= nrun) break;
+            int count;
+            run_at(k0 + k * kWaves, count);
             double xw = from_bits(wx[k]), yw = from_bits(wy[k]);
             wrap_coord(xw, Lx);
             wrap_coord(yw, Ly);
             int col, row;
             cell_col_row(xw, yw, Lx, Ly, P, col, row);
             const int c = row * P.cols + col;
-            const bool hit = i < P.n && (g < first || g >= first + own) &&
-                             ((l.cells[c >> 5] >> (c & 31)) & 1u);
-            const u64 m = __ballot(hit);
-            if (lane64 == 0) l.hit[wave * per + k0 + k] = m;
-            mine += __popcll(m);
+            const u64 m = __ballot(lane64 < count && ((l.cells[c >> 5] >> (c & 31)) & 1u));
+            if (lane64 == 0) l.scan.hit[k0 + k * kWaves] = m;
           }
         }
-        if (lane64 == 0) s_count[wave] = mine;
         __syncthreads();
-        int at = 0;
-        for (int w = 0; w < kWaves; ++w) {
-          if (w < wave) at += s_count[w];
-          H += s_count[w];
+        if (wave == 0) {  // first halo entry of each run
+          int at = 0;
+          for (int k0 = 0; k0 < nrun; k0 += 64) {
+            const int k = k0 + lane64, v = k < nrun ? __popcll(l.scan.hit[k]) : 0;
+            int incl = v;
+            for (int off = 1; off < 64; off <<= 1) {
+              const int t = __shfl_up(incl, off);
+              if (lane64 >= off) incl += t;
+            }
+            if (k < nrun) l.scan.at[k] = at + incl - v;
+            at += __shfl(incl, 63);
+          }
+          if (lane64 == 0) s_count[0] = at;
         }
+        __syncthreads();
+        H = s_count[0];
         if (own + H <= kCap) {
-          for (int k = 0; k < per; ++k) {
-            const u64 m = l.hit[wave * per + k];
+          for (int k = wave; k < nrun; k += kWaves) {
+            const u64 m = l.scan.hit[k];
+            int count;
+            const int i = run_at(k, count);
             if ((m >> lane64) & 1ull)
-              l.halo[at + __popcll(m & ((1ull << lane64) - 1ull))] =
-                  P.poff + (wave * per + k) * 64 + lane64;
-            at += __popcll(m);
+              l.halo[l.scan.at[k] + __popcll(m & ((1ull << lane64) - 1ull))] =
+                  P.poff + i + lane64;
           }
         } else {
           H = 0;
@@ -484,7 +622,6 @@ k_team(TeamArgs a) {
       // the team goes on only if every member's halo and rows fit
       bool over = s_over != 0;
       if (T > 1) {
-        ++rebuilds;
         if (tid == 0) put_flag(4 + (rebuilds & 1), rebuilds, over ? kFlagOver : 0);
         gather_flags(4 + (rebuilds & 1), rebuilds, kStall);
         __syncthreads();
@@ -505,7 +642,7 @@ k_team(TeamArgs a) {
     // row as a bit mask, the same in its L lanes, which then take them in turn,
     // so a wavefront runs the pair math (two-point: about 470 FP64
     // instructions) as often as its busiest particle has L hits
-    const bool fp64 = !MIXED || s_S[kHeun ? 0 : steps & 1].prec == kFP64;
+    const bool fp64 = !MIXED || s_m[kHeun ? 0 : steps & 1].prec == kFP64;
     const bool record = MODE == kTeamHeunSe && !predicted && (steps > 0 || a.se_first) &&
                         (a.step0 + steps) % a.se_every == 0;
     double Fx = 0.0, Fy = 0.0, Tq = 0.0;
@@ -537,13 +674,12 @@ k_team(TeamArgs a) {
         for (int k = 0; k < L; ++k) mask &= mask - 1;  // its next one
       }
     }
-    Fx = group_sum(Fx, L);
-    Fy = group_sum(Fy, L);
-    Tq = group_sum(Tq, L);
+    double F[3] = {Fx, Fy, Tq};
+    group_sum(F, L);
     if (act && lane == 0) {
-      l.fx[p] = Fx;
-      l.fy[p] = Fy;
-      l.tq[p] = Tq;
+      l.fx[p] = F[0];
+      l.fy[p] = F[1];
+      l.tq[p] = F[2];
     }
     if (kGd) {  // energy of this wavefront's pairs
       const double e = wave_sum(acc[kSeE]);
@@ -613,11 +749,11 @@ k_team(TeamArgs a) {
           build = true;
         }
         if (tid == 0) {
-          double gt = s_S[0].gamma_total + gd * dt;
+          double gt = s_S.gamma_total + gd * dt;
           if (build && le_ratio == 1.0) gt = (double)(int)(gt + 1) + g2;
-          s_S[0].gamma = g2;
-          s_S[0].gamma_total = gt;
-          s_S[0].step = s_S[0].step + 1;
+          s_S.gamma = g2;
+          s_S.gamma_total = gt;
+          s_S.step = s_S.step + 1;
         }
         gam = gam_eval = g2;
         build = build || fabs(gam - center) >= window;
@@ -641,28 +777,15 @@ k_team(TeamArgs a) {
         s2 = f2 + gp * gp;
         s3 = vx * vx + vy * vy + vp * vp;
       }
-      s0 = wave_sum(s0);
-      if (kFire) {
-        s1 = wave_sum(s1);
-        s2 = wave_sum(s2);
-        s3 = wave_sum(s3);
-      }
-      if (T == 1 && kFire && lane64 == 63) {  // two update wavefronts of one member: through LDS
-        s_part[wave * 4] = s0;
-        s_part[wave * 4 + 1] = s1;
-        s_part[wave * 4 + 2] = s2;
-        s_part[wave * 4 + 3] = s3;
-      }
+      // FIRE: value i of the sums in lanes 12 + i
+      s0 = kFire ? four_sums(s0, s1, s2, s3) : wave_sum(s0);
+      if (T == 1 && kFire && (lane64 >> 2) == 3) s_part[wave * 4 + (lane64 & 3)] = s0;
     }
     if (T == 1 && kFire && nuw > 1) __syncthreads();
     if (!kHeun && wave < nuw) {
-      if (T == 1 && nuw > 1) {
+      if (T == 1 && nuw > 1) {  // two update wavefronts of one member: through LDS
         if (kFire) {
-          // (lane 63 carries the totals)
-          s0 = s_part[0] + s_part[4];
-          s1 = s_part[1] + s_part[5];
-          s2 = s_part[2] + s_part[6];
-          s3 = s_part[3] + s_part[7];
+          s0 = s_part[lane64 & 3] + s_part[4 + (lane64 & 3)];
         } else {
           s0 = 0.0;
           for (int w = 0; w < kWaves; ++w) s0 += s_part[w];
@@ -673,32 +796,27 @@ k_team(TeamArgs a) {
       if (nsum > 1) {
         u64* const cur = sums + (size_t)(xch % 3) * a.nseats * 4 * kTeamUpdWaves;
         stores_done();  // empty marks of the last pass
-        if (lane64 == 63) {
-          u64* w = cur + (me * nuw + wave) * 4;
-          word_store(w, stop ? kStopMark : (need & kFlagRebuild) ? kNeedMark : bits_of(s0));
-          if (kFire) {
-            word_store(w + 1, bits_of(s1));
-            word_store(w + 2, bits_of(s2));
-            word_store(w + 3, bits_of(s3));
-          }
-        }
-        s0 = s1 = s2 = s3 = 0.0;
-        constexpr int kAhead = 4;  // sums of 256 wavefronts in flight
-        for (int k0 = 0; k0 < nsum; k0 += 64 * kAhead) {
-          u64 v[kAhead][kSums];
+        const bool first_word = kFire ? lane64 == 12 : lane64 == 63;
+        if (first_word || (kFire && (lane64 >> 2) == 3))
+          word_store(cur + (me * nuw + wave) * 4 + (kFire ? lane64 & 3 : 0),
+                     !first_word ? bits_of(s0)
+                     : stop      ? kStopMark
+                     : (need & kFlagRebuild) ? kNeedMark : bits_of(s0));
+        // every wavefront's sums, a word to a lane (FIRE: four lanes to a record)
+        constexpr int kRecords = kFire ? 16 : 64;  // of a load
+        s0 = 0.0;
+        auto collect = [&](int k0, auto ahead) {
+          constexpr int kAhead = decltype(ahead)::value;
+          u64 v[kAhead];
+          const int r0 = k0 + (kFire ? lane64 >> 2 : lane64), w = kFire ? lane64 & 3 : 0;
           Wait wait;
           while (true) {
             bool all = true;
 #pragma unroll
-            for (int k = 0; k < kAhead; ++k) {
-              const u64* w = cur + min(k0 + 64 * k + lane64, nsum - 1) * 4;
-#pragma unroll
-              for (int i = 0; i < kSums; ++i) v[k][i] = word_load(w + i);
-            }
-#pragma unroll
             for (int k = 0; k < kAhead; ++k)
+              v[k] = word_load(cur + min(r0 + k * kRecords, nsum - 1) * 4 + w);
 #pragma unroll
-              for (int i = 0; i < kSums; ++i) all = all && v[k][i] != kEmpty;
+            for (int k = 0; k < kAhead; ++k) all = all && v[k] != kEmpty;
             if (all) break;
             if (wait.over(kStall, status)) {
               s_fail = 1;
@@ -706,38 +824,38 @@ k_team(TeamArgs a) {
             }
           }
 #pragma unroll
-          for (int k = 0; k < kAhead; ++k) {
-            if (k0 + 64 * k + lane64 >= nsum) break;
-            again = again || v[k][0] == kNeedMark;
-            stop = stop || v[k][0] == kStopMark;
-            s0 += from_bits(v[k][0]);
-            if (kFire) {
-              s1 += from_bits(v[k][1]);
-              s2 += from_bits(v[k][2]);
-              s3 += from_bits(v[k][3]);
+          for (int k = 0; k < kAhead; ++k)
+            if (r0 + k * kRecords < nsum) {
+              again = again || v[k] == kNeedMark;
+              stop = stop || v[k] == kStopMark;
+              s0 += from_bits(v[k]);
             }
-          }
-        }
+        };
+        if (nsum <= kRecords) collect(0, std::integral_constant<int, 1>{});
+        else if (nsum <= 4 * kRecords) collect(0, std::integral_constant<int, 4>{});
+        else
+          for (int k0 = 0; k0 < nsum; k0 += 16 * kRecords)
+            collect(k0, std::integral_constant<int, 16>{});
         again = __any(again);
         stop = __any(stop);
-        s0 = wave_sum(s0);
-        if (kFire) {
-          s1 = wave_sum(s1);
-          s2 = wave_sum(s2);
-          s3 = wave_sum(s3);
-        }
+        s0 = kFire ? quad_sum(s0) : wave_sum(s0);
       }
       if (stop || again) {
         if (tid == 0) s_next = stop ? kDone : kAgain;
       } else {
         mark_empty(pass);  // all have read this pass's positions
-        const PackScal& S0 = s_S[steps & 1];
+        const MinState S0 = s_m[steps & 1];
         const MinStep S =
-            minimiser_step(a.fire, kFire, P.n, P.inv_2n, S0, last_lane(s0), last_lane(s1),
-                           last_lane(s2), last_lane(s3), last_lane(s0), false);
+            kFire ? minimiser_step(a.fire, true, P.n, P.inv_2n, S0, lane_value(s0, 12),
+                                   lane_value(s0, 13), lane_value(s0, 14), lane_value(s0, 15), 0.0,
+                                   false)
+                  : minimiser_step(a.fire, false, P.n, P.inv_2n, S0, 0.0, 0.0, 0.0, 0.0,
+                                   lane_value(s0, 63), false);
         moved = S.end == 0;
         if (tid == 0) {
-          advance(s_S[(steps + 1) & 1], S0, S, kFire);
+          s_m[(steps + 1) & 1] = after(S0, S);
+          s_end = S.end;
+          s_frms = S.frms;
           s_next = S.end ? kDone : kGoOn;
         }
         // ---- update (update mapping); nothing moves once finished
@@ -806,19 +924,30 @@ k_team(TeamArgs a) {
       }
       double sn, cs;
       rod_sincos(phi, &sn, &cs);
-      const double nx = l.A[tid] * cs, ny = l.A[tid] * sn;
-      if (kHeun) stores_done();  // empty marks of this pass
-      publish(pass + 1, x, y, nx, ny);
+      if (kHeun && !wide) {  // from registers: the others wait for this alone
+        stores_done();       // empty marks of this pass
+        if (T > 1) {
+          u64* r = record_of(pass + 1, gu);
+          word_store(r, bits_of(x));
+          word_store(r + 1, bits_of(y));
+          word_store(r + 2, bits_of(l.A[tid] * cs));
+          word_store(r + 3, bits_of(l.A[tid] * sn));
+        }
+      }
       l.x[tid] = x;
       l.y[tid] = y;
-      l.nx[tid] = nx;
-      l.ny[tid] = ny;
+      l.nx[tid] = l.A[tid] * cs;
+      l.ny[tid] = l.A[tid] * sn;
       l.phi[tid] = phi;
       const double dx = fabs(min_image(x - l.xb[tid], Lx)), dy = fabs(min_image(y - l.yb[tid], Ly));
       const bool late = kHeun && T > 1;  // the answer comes one pass late
       if (fmax(dx, dy) >= (late ? 0.6 * hs : hs)) need |= kFlagRebuild;
       if (late && fmax(dx, dy) >= hs) need |= kFlagFast;
       if (need) atomicOr(&s_need, need);
+    }
+    if (moved && wave < nuw && (!kHeun || wide)) {
+      if (kHeun) stores_done();  // empty marks of this pass
+      publish(pass + 1);
     }
     ++xch;
     __syncthreads();  // new coordinates, s_need, s_next and s_fail visible
@@ -870,7 +999,22 @@ k_team(TeamArgs a) {
     b.fy[gu] = l.fy[tid];
     b.tau[gu] = l.tq[tid];
   }
-  if (me == 0 && tid == 0) a.scal[pk] = s_S[kHeun ? 0 : steps & 1];
+  if (me == 0 && tid == 0) {
+    if (!kHeun) {
+      const MinState& m = s_m[steps & 1];
+      s_S.step = m.step;
+      s_S.fire_dt = m.dt;
+      s_S.fire_alpha = m.alpha;
+      s_S.fire_npos = m.npos;
+      s_S.prec = m.prec;
+      if (s_end) {
+        s_S.converged = s_end;
+        s_S.iters = m.step;
+        s_S.frms = s_frms;
+      }
+    }
+    a.scal[pk] = s_S;
+  }
 }
 
 #define SC_TEAM_INST(M, H)                                      \
