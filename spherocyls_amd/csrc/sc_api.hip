@@ -493,7 +493,7 @@ void bin_all_sized(sc_system* s, int buf, int wrap_angles) {
 void resort(sc_system* s) {
   KernelTimer t(s, SC_KERNEL_SORT);
   int buf = s->cur_buf;
-  hipLaunchKernelGGL(k_scan_cells, dim3(s->npack), dim3(256), 0, s->stream, s->d_packs,
+  hipLaunchKernelGGL(k_scan_cells, dim3(s->npack), dim3(1024), 0, s->stream, s->d_packs,
                      s->d_cnt[buf], s->d_cstart);
   hipLaunchKernelGGL(k_sort_cells, dim3(grid_for(s->ncells, 256)), dim3(256), 0, s->stream,
                      s->d_cstart, s->d_cnt[buf], s->d_slot[buf], s->B().id, s->d_perm, s->ncells,

@@ -761,33 +761,44 @@ __global__ void k_affine(Bank b, const int* pack_of, const double* scale, int nt
 
 // ---- counting sort by cell ------------------------------------------------
 
-// Exclusive scan of bucket counts over the cells of each packing (one
-// workgroup per packing, chunks of blockDim cells).
-__global__ void k_scan_cells(const PackInfo* packs, const int* cnt, int* cstart) {
-  __shared__ int s_w[16];
-  __shared__ int s_carry;
+// Exclusive scan of bucket counts over the cells of each packing: one workgroup
+// per packing, 8192 cells at a time, eight to a thread.  A chunk costs its
+// barriers and one trip to memory whatever its size: 256 cells at a time took 16
+// us for 16k particles and 363 us for 262k, now 6.6 and 104.
+constexpr int kScanThreads = 1024, kScanEach = 8;
+__global__ void __launch_bounds__(kScanThreads) k_scan_cells(const PackInfo* packs, const int* cnt,
+                                                             int* cstart) {
+  __shared__ int s_w[kScanThreads / 64];
   const PackInfo P = packs[blockIdx.x];
   const int ncell = P.rows * P.cols;
-  const int tid = threadIdx.x, nthr = blockDim.x;
-  if (tid == 0) s_carry = P.poff;
-  __syncthreads();
-  for (int base = 0; base < ncell; base += nthr) {
-    int c = base + tid;
-    int v = c < ncell ? min(cnt[P.coff + c], P.cap) : 0;
-    int incl = v;
+  const int tid = threadIdx.x;
+  int carry = P.poff;
+  for (int base = 0; base < ncell; base += kScanThreads * kScanEach) {
+    const int c0 = base + tid * kScanEach;
+    int v[kScanEach], sum = 0;
+#pragma unroll
+    for (int k = 0; k < kScanEach; ++k) {
+      v[k] = c0 + k < ncell ? min(cnt[P.coff + c0 + k], P.cap) : 0;
+      sum += v[k];
+    }
+    int incl = sum;
     for (int off = 1; off < 64; off <<= 1) {
       int t = __shfl_up(incl, off);
       if ((tid & 63) >= off) incl += t;
     }
     if ((tid & 63) == 63) s_w[tid >> 6] = incl;
     __syncthreads();
-    int wpre = 0;
-    for (int w = 0; w < (tid >> 6); ++w) wpre += s_w[w];
-    int carry = s_carry;
-    if (c < ncell) cstart[P.coff + c] = carry + wpre + incl - v;
-    __syncthreads();
-    if (tid == nthr - 1) s_carry = carry + wpre + incl;
-    __syncthreads();
+    int at = carry + incl - sum;
+    for (int w = 0; w < kScanThreads / 64; ++w) {
+      if (w < (tid >> 6)) at += s_w[w];
+      carry += s_w[w];
+    }
+#pragma unroll
+    for (int k = 0; k < kScanEach; ++k) {
+      if (c0 + k < ncell) cstart[P.coff + c0 + k] = at;
+      at += v[k];
+    }
+    __syncthreads();  // s_w read by all
   }
 }
 
