@@ -982,7 +982,7 @@ int run_team(sc_system* s, int mode, const TeamPlan& plan, const FireParams* fp,
       hipLaunchKernelGGL(fn, dim3(nseats), dim3(kTeamThreads), plan.lds, s->stream, a);
     }
     if (nrec > 0)
-      hipLaunchKernelGGL(k_team_records, dim3(nrec), dim3(64), 0, s->stream, a, nseats,
+      hipLaunchKernelGGL(k_team_records, dim3(nrec), dim3(256), 0, s->stream, a, nseats,
                          s->d_se_ring + ((size_t)(step0 + se_every - 1) / se_every -
                                          (step0 > 0 ? 1 : 0)) * kNSe);
     HIPCK(hipMemcpyAsync(words.data(), s->d_team_status, sizeof(int) * nseats,
