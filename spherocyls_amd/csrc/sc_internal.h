@@ -145,7 +145,7 @@ struct TileArgs {
 
 // Neighbour-list force path.  Each particle keeps a list of candidate partners
 // chosen with a skin; a force kernel rebuilds the lists of a packing (each
-// thread its own row) when the previous kernel raised the packing's flag.
+// particle's lanes its row) when the previous kernel raised the packing's flag.
 constexpr int kNbrCap = 64;
 // Partners a list-kernel thread holds between its prefilter and pair-math
 // phases (a longer run is processed in pieces); the kernel's dynamic LDS is

@@ -12,8 +12,8 @@
 // particle has moved more than skin/2 (per sheared coordinate) from its position
 // at the last build, when a Lees-Edwards remap happened, or when the strain
 // leaves the window the lists were built for.  The next force pass then rebuilds
-// every row of that packing from the exact per-pass cell buckets, each thread its
-// own row, before using it; no host decision and no extra launch are involved.
+// every row of that packing from the exact per-pass cell buckets, a particle's
+// lanes its row, before using it; no host decision and no extra launch are involved.
 //
 // Selection rule (skin s <= cell pad; S = R_p + A_p + R_q + A_q; dx_s, dy minimum
 // images in sheared coordinates; strain window [g_lo, g_hi]; c = max(1.5,
@@ -209,7 +209,7 @@ __device__ int build_row(const ListArgs& a, const PackInfo& P, double Lx, double
 // LANES threads share a particle: lane l takes list entries l, l + LANES, ...
 // in batches of kGather whose loads are all issued before any is used, so a
 // lane has several independent gathers in flight.  The LANES partial sums are
-// combined with xor shuffles (fixed order for a given LANES).
+// combined as a tree (fixed order for a given LANES).
 constexpr int kGather = 4;
 
 // MIXED: the kernel carries the FP32-force pair path besides the FP64 one and
