@@ -131,6 +131,13 @@ int sc_set_graphs(sc_system* s, int enable);
  * on, a minimiser's launch is counted under SC_KERNEL_FIRE_FORCE; sheared steps
  * are then launched one by one. */
 int sc_set_small_fire(sc_system* s, int max_particles, int steps_per_launch);
+/* Team launches of this system so far, and why the last one handed its steps
+ * back to the launches per step (0: it did not).  Either may be NULL. */
+#define SC_TEAM_ABSENT 1   /* a workgroup was not resident in time; nothing was written */
+#define SC_TEAM_STALLED 2  /* a wait ran out later (the call returns SC_ERR_HIP) */
+#define SC_TEAM_NO_ROOM 4  /* a workgroup's neighbourhood or a row did not fit its LDS */
+#define SC_TEAM_OUTRAN 8   /* a sheared particle outran the rows */
+int sc_team_info(const sc_system* s, long long* launches, int* status);
 int sc_get_contact_model(const sc_system* s, int* model);
 /* Force-pass implementation (no reference counterpart; both give the same
  * forces to rounding):

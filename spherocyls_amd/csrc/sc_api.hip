@@ -130,6 +130,8 @@ struct sc_system {
   TeamSeat* d_team_seats = nullptr;
   int* d_team_status = nullptr;
   int team_seat_cap = 0;
+  long long team_launches = 0;  // so far, and the last one's status bits (sc_team_info)
+  int team_status = 0;
   double* d_team_se = nullptr;
   size_t team_se_cap = 0;
   int ncells = 0, ntiles = 0, npblocks = 0;
@@ -854,6 +856,10 @@ TeamFn team_kernel(int mode, bool two_point, bool mixed, int shape) {
   return table[shape][mode][two_point ? 1 : 0][mixed ? 1 : 0];
 }
 
+static_assert(kTeamAbsent == SC_TEAM_ABSENT && kTeamStalled == SC_TEAM_STALLED &&
+                  kTeamOver == SC_TEAM_NO_ROOM && kTeamFast == SC_TEAM_OUTRAN,
+              "status bits of a team launch");
+
 // A device runs one team launch of this process at a time: two launches that
 // each hold part of the CUs would wait for each other.  Held from the launch
 // to its end.
@@ -993,6 +999,8 @@ int run_team(sc_system* s, int mode, const TeamPlan& plan, const FireParams* fp,
   }
   int status = 0;
   for (int w : words) status |= w;
+  s->team_launches++;
+  s->team_status = status;
   force_rebuild(s);
   if (status & kTeamStalled) throw StatusError{SC_ERR_HIP, "a team of workgroups stalled"};
   return status;
@@ -1306,6 +1314,13 @@ int sc_set_small_fire(sc_system* s, int max_particles, int steps_per_launch) {
     return SC_ERR_ARG;
   s->small_max = max_particles;
   s->small_steps = steps_per_launch > 0 ? steps_per_launch : 50000;
+  return SC_OK;
+}
+
+int sc_team_info(const sc_system* s, long long* launches, int* status) {
+  if (!s) return SC_ERR_ARG;
+  if (launches) *launches = s->team_launches;
+  if (status) *status = s->team_status;
   return SC_OK;
 }
 

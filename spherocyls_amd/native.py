@@ -66,6 +66,7 @@ def load():
         "sc_set_contact_model": ([sysp, C.c_int], C.c_int),
         "sc_set_graphs": ([sysp, C.c_int], C.c_int),
         "sc_set_small_fire": ([sysp, C.c_int, C.c_int], C.c_int),
+        "sc_team_info": ([sysp, C.POINTER(C.c_longlong), _ip], C.c_int),
         "sc_get_contact_model": ([sysp, _ip], C.c_int),
         "sc_set_tiling": ([sysp, C.c_int, C.c_int], C.c_int),
         "sc_set_path": ([sysp, C.c_int], C.c_int),
@@ -348,6 +349,12 @@ class System:
         (0); at most steps_per_launch minimiser iterations per launch (0: the
         default, 50000)."""
         self._ck(self.lib.sc_set_small_fire(self.h, int(max_particles), int(steps_per_launch)))
+
+    def team_info(self):
+        """(team launches so far, status bits of the last one: SC_TEAM_*)."""
+        n, st = C.c_longlong(), C.c_int()
+        self._ck(self.lib.sc_team_info(self.h, C.byref(n), C.byref(st)))
+        return n.value, st.value
 
     def contact_model(self):
         m = C.c_int()

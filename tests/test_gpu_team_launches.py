@@ -1,0 +1,145 @@
+"""Which calls run as teams of workgroups, and what a team does where it cannot
+go on: the launch counter and its status say so, and the steps are compared with
+the launches per step (whose results the other files compare with the oracle).
+
+A member of a team holds 64 particles and at most 448 around them.  With a few
+large discs the cells are large, and a member's cells hold more particles than
+that, at once or once its own have drifted over more cells; _halo computes the
+count.  Both sides evaluate the same formulas and differ in the order of sums (a
+few units in the last place per step, as 1e-13 over 150, with a factor of 1e4
+left for contacts that amplify it)."""
+import numpy as np
+import pytest
+
+from spherocyls_amd import configs, native
+
+pytestmark = pytest.mark.gpu
+ROOM = 448
+TOL = 1e-9
+
+
+def _packing(n, seed, discs=0, radius=0.0, phi=0.84):
+    R, A = configs.bidisperse(n, aspect=1.5)
+    R[:discs], A[:discs] = radius, 0.0
+    return configs.make_packing(R, A, phi, seed, f"N={n} with {discs} discs")
+
+
+def _cells(pk, x, y):
+    g = int(pk.L / (2 * (pk.R.max() + pk.A.max()) + 0.1))
+    return g, (y % pk.L * (g / pk.L)).astype(int) % g, (x % pk.L * (g / pk.L)).astype(int) % g
+
+
+def _halo(pk, x, y):
+    """Most particles around a member, of members that hold runs of the
+    packing's storage order (by cell and number at its start)."""
+    g, r0, c0 = _cells(pk, pk.x, pk.y)
+    order = np.lexsort((np.arange(pk.n), r0 * g + c0))
+    _, r, c = _cells(pk, x, y)
+    per = -(-pk.n // -(-pk.n // 64))
+    most = 0
+    for at in range(0, pk.n, per):
+        own, near = order[at:at + per], np.zeros((g, g), bool)
+        for d in (-1, 0, 1):
+            for e in (-1, 0, 1):
+                near[(r[own] + d) % g, (c[own] + e) % g] = True
+        most = max(most, int(near[r, c].sum()) - len(own))
+    return most
+
+
+def _system(pk, small):
+    s = native.System(pk, pads=0.1)
+    s.set_contact_model("two_point")
+    s.set_small_fire(small)
+    return s
+
+
+def _same(a, b, L, tol=TOL):
+    for u, v, side in zip(a[0], b[0], (L, L, 2 * np.pi)):
+        d = u - v
+        assert np.max(np.abs(d - side * np.round(d / side))) < tol
+    for u, v in zip(a[1], b[1]):
+        assert np.max(np.abs(u - v)) < tol * max(1.0, np.max(np.abs(v)))
+
+
+@pytest.mark.parametrize("n", [100, 700, 16384])
+def test_calls_that_run_as_teams(n):
+    pk = _packing(n, 3, phi=0.80)
+    s = _system(pk, 256)
+    try:
+        print("teams", n, flush=True)
+        s.fire(native.fire_params(max_move=0.02, ftol=1e-12, max_iter=200), check=False)
+        assert s.team_info() == (1, 0)
+        s.gd_steps(30)
+        assert s.team_info() == (2, 0)
+        s.set_dynamics(strain_rate=1e-3, step=0.005)
+        s.strain_steps(100)
+        assert s.team_info() == (3, 0)
+        s.strain_steps(100, 20)
+        assert s.team_info() == (4, 0)
+        s.set_small_fire(0)
+        s.strain_steps(100)
+        s.gd_steps(5)
+        assert s.team_info() == (4, 0)
+    finally:
+        s.close()
+
+
+def test_no_room_while_minimising():
+    """FIRE and gradient descent whose members run out of room on the way: the
+    state reached goes on with the launches per step."""
+    pk = _packing(1000, 1, discs=2, radius=3.0)
+    assert _halo(pk, pk.x, pk.y) <= ROOM  # a team starts
+    params = native.fire_params(dt0=0.05, dt_max=0.5, max_move=0.02, ftol=1e-12, max_iter=60)
+    for name, run in (("fire", lambda s: s.fire(params, check=False)[0][0]),
+                      ("descent", lambda s: s.gd_steps(60))):
+        out = []
+        for small in (256, 0):
+            print("no room,", name, small, flush=True)
+            s = _system(pk, small)
+            try:
+                s.set_dynamics(step=0.05)
+                assert run(s) == 60
+                assert s.team_info() == ((1, native.SC_TEAM_NO_ROOM) if small else (0, 0))
+                out.append((s.positions(), s.forces()))
+            finally:
+                s.close()
+        assert _halo(pk, *out[1][0][:2]) > ROOM
+        _same(*out, pk.L)
+
+
+def test_no_room_during_sheared_steps_with_records():
+    pk = _packing(1000, 1, discs=2, radius=3.0)
+    assert _halo(pk, pk.x, pk.y) <= ROOM
+    out = []
+    for small in (256, 0):
+        print("no room, shear", small, flush=True)
+        s = _system(pk, small)
+        try:
+            s.set_dynamics(strain_rate=1e-3, step=0.004)
+            se = s.strain_steps(150, 7)
+            assert s.team_info() == ((1, native.SC_TEAM_NO_ROOM) if small else (0, 0))
+            out.append((s.positions(), s.forces(), se, s.box(0)))
+        finally:
+            s.close()
+    assert _halo(pk, *out[1][0][:2]) > ROOM
+    _same(out[0], out[1], pk.L)
+    assert out[0][2].shape == (21, 1, 9)
+    np.testing.assert_allclose(out[0][2], out[1][2], rtol=0, atol=TOL * np.abs(out[1][2]).max())
+    assert out[0][3]["gamma"] == pytest.approx(out[1][3]["gamma"], abs=1e-14)
+
+
+def test_outrun_rows():
+    """Steps in which particles move more than half the skin."""
+    pk = _packing(700, 5, phi=0.80)
+    out = []
+    for small in (256, 0):
+        print("outrun", small, flush=True)
+        s = _system(pk, small)
+        try:
+            s.set_dynamics(strain_rate=1e-3, step=0.5)
+            s.strain_steps(100)
+            assert s.team_info() == ((1, native.SC_TEAM_OUTRAN) if small else (0, 0))
+            out.append((s.positions(), s.forces()))
+        finally:
+            s.close()
+    _same(*out, pk.L)
