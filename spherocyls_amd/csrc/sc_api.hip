@@ -274,9 +274,11 @@ struct GraphExec {
     }
   }
   void launch() { HIPCK(hipGraphLaunch(exec, s->stream)); }
-  ~GraphExec() {
+  void drop() {  // the stream is idle
     if (exec) (void)hipGraphExecDestroy(exec);
+    exec = nullptr;
   }
+  ~GraphExec() { drop(); }
 };
 
 struct KernelTimer {
@@ -1851,7 +1853,12 @@ int sc_fire_minimize(sc_system* s, const double* params, double switch_frms, int
   TeamPlan plan;
   while (true) {
     const bool team = teams && team_plan(s, kTeamFire, active, plan);
-    if (was_team && !team) leave_team(s);
+    if (was_team && !team) {
+      // a graph captured before the team may read another bucket buffer than
+      // leave_team fills, and slots that it reallocates
+      g.drop();
+      leave_team(s);
+    }
     was_team = team;
     if (team) {
       // CUs left idle by finished packings: back to the host for a new plan
@@ -1890,10 +1897,7 @@ int sc_fire_minimize(sc_system* s, const double* params, double switch_frms, int
       if (!s->scal[k].converged) active.push_back(k);
     if (active.empty()) break;
     if (!team && s->path == SC_PATH_LIST && 2 * (int)active.size() <= last_active) {
-      if (g.exec) {  // the captured launches name the old lists
-        HIPCK(hipGraphExecDestroy(g.exec));
-        g.exec = nullptr;
-      }
+      g.drop();  // the captured launches name the old lists
       // A tail of few particles leaves most of the GPU idle and each pass is
       // as long as one particle's chain of dependent gathers: give every
       // particle more lanes (up to 8) until the launch has about one lane

@@ -143,3 +143,35 @@ def test_outrun_rows():
         finally:
             s.close()
     _same(*out, pk.L)
+
+
+def test_launches_go_on_after_a_team_in_the_middle():
+    """A batch too large for teams, whose loose packings finish at once: the
+    rest go on as teams, which have no room from their first pass on, and then
+    with the launches per step again.  (The sheared step before turns the
+    bucket buffers, so that the launches before and after the team read
+    different ones.)"""
+    tight = _packing(1000, 1, discs=2, radius=4.0)
+    at = np.arange(1000)  # on a lattice, out of reach of each other
+    loose = configs.Packing(80.0, 2.5 * (at % 32) + 1.0, 2.5 * (at // 32) + 1.0, 0.1 * at,
+                            0.5 * np.ones(1000), 0.5 * np.ones(1000), 0.0, "loose")
+    assert _halo(tight, tight.x, tight.y) > ROOM
+    packs = [tight if k % 8 < 3 else loose for k in range(80)]  # 30 tight
+    params = native.fire_params(dt0=0.05, dt_max=0.5, max_move=0.02, ftol=1e-12, max_iter=120)
+    out = []
+    for small in (256, 0):
+        print("team in the middle", small, flush=True)
+        s = _system(packs, small)
+        try:
+            s.set_dynamics(strain_rate=1e-4, step=0.001)
+            s.strain_steps(1)
+            it, fr, _ = s.fire(params, check=False)
+            assert s.team_info() == ((1, native.SC_TEAM_NO_ROOM) if small else (0, 0))
+            out.append((s.positions(), s.forces(), it, fr))
+        finally:
+            s.close()
+    np.testing.assert_array_equal(out[0][2], out[1][2])
+    assert sorted(set(out[0][2].tolist())) == [0, 120]
+    np.testing.assert_allclose(out[0][3], out[1][3], rtol=1e-6)
+    side = np.concatenate([np.full(p.n, p.L) for p in packs])
+    _same(out[0], out[1], side)
