@@ -131,6 +131,13 @@ int sc_set_graphs(sc_system* s, int enable);
  * on, a minimiser's launch is counted under SC_KERNEL_FIRE_FORCE; sheared steps
  * are then launched one by one. */
 int sc_set_small_fire(sc_system* s, int max_particles, int steps_per_launch);
+/* How long (0 to 5 s; default 0.2) the workgroups of a team launch wait for
+ * each other to become resident, as another process on the GPU may keep some
+ * out; with 0 they leave unless all are there at the first look.  A launch that
+ * waited in vain has written nothing: launches per step go on (the results then
+ * differ by rounding from a team's), without another try for 20 s or until this
+ * is called. */
+int sc_set_team_wait(sc_system* s, double seconds);
 /* Team launches of this system so far, and why the last one handed its steps
  * back to the launches per step (0: it did not).  Either may be NULL. */
 #define SC_TEAM_ABSENT 1   /* a workgroup was not resident in time; nothing was written */

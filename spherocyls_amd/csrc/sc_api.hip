@@ -132,6 +132,8 @@ struct sc_system {
   int team_seat_cap = 0;
   long long team_launches = 0;  // so far, and the last one's status bits (sc_team_info)
   int team_status = 0;
+  double team_wait = 0.2;  // seconds of a launch's roll call
+  std::chrono::steady_clock::time_point team_off{};  // no team before this time
   double* d_team_se = nullptr;
   size_t team_se_cap = 0;
   int ncells = 0, ntiles = 0, npblocks = 0;
@@ -868,6 +870,10 @@ static_assert(kTeamAbsent == SC_TEAM_ABSENT && kTeamStalled == SC_TEAM_STALLED &
 constexpr int kMaxDevices = 64;
 std::mutex g_team_mu[kMaxDevices];
 
+// After a roll call that ran out the system's calls launch per step for this
+// long: where another process keeps the CUs, waiting for them costs at most 1%.
+constexpr std::chrono::seconds kTeamOff{20};
+
 struct TeamPlan {
   int shape = 0;
   std::vector<TeamSeat> seats;
@@ -878,7 +884,9 @@ struct TeamPlan {
 // particles, of equal size within a packing, in the smallest shape whose
 // workgroups are all resident at once.  False when they do not fit.
 bool team_plan(sc_system* s, int mode, const std::vector<int>& want, TeamPlan& plan) {
-  if (s->path != SC_PATH_LIST || s->device >= kMaxDevices || want.empty()) return false;
+  if (s->path != SC_PATH_LIST || s->small_max <= 0 || s->device >= kMaxDevices || want.empty() ||
+      std::chrono::steady_clock::now() < s->team_off)
+    return false;
   long particles = 0;
   int cell_words = 0;
   for (int k : want) {
@@ -963,6 +971,7 @@ int run_team(sc_system* s, int mode, const TeamPlan& plan, const FireParams* fp,
   a.err = s->d_err;
   if (fp) a.fire = *fp;
   a.gamma_window = s->gamma_window;
+  a.roll_call = (unsigned long long)(s->team_wait * 1e8);
   a.ntot = s->ntot;
   a.nseats = nseats;
   a.max_steps = max_steps;
@@ -1003,6 +1012,7 @@ int run_team(sc_system* s, int mode, const TeamPlan& plan, const FireParams* fp,
   for (int w : words) status |= w;
   s->team_launches++;
   s->team_status = status;
+  if (status & kTeamAbsent) s->team_off = std::chrono::steady_clock::now() + kTeamOff;
   force_rebuild(s);
   if (status & kTeamStalled) throw StatusError{SC_ERR_HIP, "a team of workgroups stalled"};
   return status;
@@ -1319,6 +1329,13 @@ int sc_set_small_fire(sc_system* s, int max_particles, int steps_per_launch) {
   return SC_OK;
 }
 
+int sc_set_team_wait(sc_system* s, double seconds) {
+  if (!s || !(seconds >= 0.0 && seconds <= 5.0)) return SC_ERR_ARG;
+  s->team_wait = seconds;
+  s->team_off = {};
+  return SC_OK;
+}
+
 int sc_team_info(const sc_system* s, long long* launches, int* status) {
   if (!s) return SC_ERR_ARG;
   if (launches) *launches = s->team_launches;
@@ -1518,7 +1535,7 @@ int sc_strain_steps(sc_system* s, int nsteps, int se_every, double* se_out) {
   const int mode = se ? kTeamHeunSe : kTeamHeun;
   const std::vector<int> only{0};
   TeamPlan plan;
-  if (s->npack == 1 && s->small_max > 0 && !s->timing && nsteps > 1 &&
+  if (s->npack == 1 && !s->timing && nsteps > 1 &&
       !(se && s->prec == SC_PREC_MIXED) && team_plan(s, mode, only, plan)) {
     while (st < nsteps) {
       const int upto = std::min(nsteps, st + 2 * resort_every);
@@ -1703,7 +1720,7 @@ int sc_gd_steps(sc_system* s, int nmax, double emin, int* steps_done) {
   std::vector<int> every;
   for (int k = 0; k < s->npack; ++k) every.push_back(k);
   TeamPlan plan;
-  bool teams = s->small_max > 0 && team_plan(s, kTeamGd, every, plan);
+  bool teams = team_plan(s, kTeamGd, every, plan);
   while (true) {
     if (teams) {
       if (run_team(s, kTeamGd, plan, &fp, s->small_steps)) {
@@ -1849,7 +1866,7 @@ int sc_fire_minimize(sc_system* s, const double* params, double switch_frms, int
   // where they would.
   std::vector<int> active;
   for (int k = 0; k < s->npack; ++k) active.push_back(k);
-  bool teams = s->small_max > 0, was_team = false;
+  bool teams = true, was_team = false;
   TeamPlan plan;
   while (true) {
     const bool team = teams && team_plan(s, kTeamFire, active, plan);

@@ -258,6 +258,7 @@ struct TeamArgs {
   int* err;
   FireParams fire;
   double gamma_window;
+  unsigned long long roll_call;  // ticks of 10 ns that members wait for each other to come up
   int ntot, nseats;
   int max_steps;             // iterations (Heun: steps) of this launch
   // kTeamHeunSe: a record where (step0 + steps) % se_every == 0, before the

@@ -39,10 +39,10 @@
 // everyone who will poll the buffer's next positions reads first.  Sum slots
 // follow the same rule with the sums themselves.
 //
-// Every wait is bounded.  The first pass of a launch doubles as the roll call:
-// a member that never becomes resident (another kernel holds the CUs) makes the
-// others leave without having written anything, and the host goes on with the
-// launches per step.  The host launches at most as many workgroups as are
+// Every wait is bounded.  The first pass's rebuild doubles as the roll call: a
+// member that is not resident within a.roll_call (another process's kernels
+// hold the CUs) makes the others leave without having written anything, and the
+// host goes on with the launches per step, for some time without another try.  The host launches at most as many workgroups as are
 // resident at once.
 //
 // Measured, all-gather of 4 words by G workgroups over all XCDs: 1.05 us (G = 2),
@@ -94,16 +94,17 @@ __device__ __forceinline__ int opaque(int v) {
 }
 
 // A wait that ends: over() is true once `limit` ticks (100 MHz) have passed
-// since its first call, or, after 0.1 ms, when a member of the team has
-// reported that it gave up.  (The clock is not read while words arrive at the
-// first look.)
+// since its first call (at once for a limit of 0), or, after 0.1 ms, when a
+// member of the team has reported that it gave up.  One serves all words of a
+// stage, so a stage ends at its limit however many words are missing.  (The
+// clock is not read while words arrive at the first look.)
 struct Wait {
   u64 t0 = 0;
   __device__ __forceinline__ bool over(u64 limit, const int* status) {
     const u64 t = wall_clock64();
     if (t0 == 0) {
       t0 = t;
-      return false;
+      return limit == 0;
     }
     return t - t0 > limit ||
            (t - t0 > 10000 &&
@@ -274,7 +275,7 @@ k_team(TeamArgs a) {
   const double skin = P.pad, sx = fmax(1.5, 1.0 + 0.5 * Lx / Ly) * P.pad, hs = 0.5 * P.pad;
   double gam = a.scal[pk].gamma, gam_eval = gam, center = gam;
   const double window = kHeun ? a.gamma_window : 0.0;
-  const u64 kRollCall = 20000000ull, kStall = 500000000ull;  // 0.2 s, 5 s
+  const u64 kStall = 500000000ull;  // 5 s
 
   auto record_of = [&](int j, int g) {
     return a.pos + ((size_t)(j & (kBufs - 1)) * a.ntot + g) * 4;
@@ -321,11 +322,11 @@ k_team(TeamArgs a) {
   };
   // halo entries' positions of pass j into LDS
   auto fetch_halo = [&](int j, int H, u64 limit) {
+    Wait wait;
     if (!wide) {
       for (int e = tid; e < H; e += kTeamThreads) {
         const u64* r = record_of(j, l.halo[e]);
         u64 v[4];
-        Wait wait;
         while (true) {
 #pragma unroll
           for (int k = 0; k < 4; ++k) v[k] = word_load(r + k);
@@ -348,7 +349,6 @@ k_team(TeamArgs a) {
 #pragma unroll
       for (int k = 0; k < kAhead; ++k)
         if (i0 + k * kTeamThreads < n4) r[k] = record_of(j, l.halo[(i0 + k * kTeamThreads) >> 2]) + w;
-      Wait wait;
       while (true) {
         bool all = true;
 #pragma unroll
@@ -374,9 +374,9 @@ k_team(TeamArgs a) {
   // every member's flag word numbered seq in slot `slot`, ORed into s_bits
   auto gather_flags = [&](int slot, unsigned seq, u64 limit) {
     const u64* f = flags + (size_t)slot * a.nseats;
+    Wait wait;
     for (int m = tid; m < T; m += kTeamThreads) {
       u64 v;
-      Wait wait;
       while (((v = word_load(f + m)) >> 8) != seq)
         if (wait.over(limit, status)) {
           s_fail = 1;
@@ -412,7 +412,8 @@ k_team(TeamArgs a) {
     tid = opaque(tid0);
     gu = first + (upd ? tid : 0);
     const int p = opaque(p0);
-    const u64 limit = pass == 0 ? kRollCall : kStall;
+    const u64 limit = pass == 0 ? a.roll_call : kStall;
+    const int missed = pass == 0 ? kTeamAbsent : kTeamStalled;  // a wait that ran out
     // ---- positions of this pass
     if (T > 1) {
       if (kHeun && pass > 0) gather_flags((pass - 1) & 3, (unsigned)pass, kStall);
@@ -420,7 +421,7 @@ k_team(TeamArgs a) {
     }
     __syncthreads();
     if (s_fail) {
-      if (tid == 0) give_up(pass == 0 ? kTeamAbsent : kTeamStalled);
+      if (tid == 0) give_up(missed);
       return;
     }
     if (kHeun) {
@@ -498,14 +499,15 @@ k_team(TeamArgs a) {
         // order (s_count: each wavefront's number of them)
         const u64 near_row = s_near[0], near_col = s_near[1];
         int nrun = 0;
+        bool failed = false;
+        Wait come;
         for (int c0 = 0; c0 < T * nuw; c0 += kTeamThreads) {
           const int c = c0 + tid, m = c / nuw, part = c - m * nuw;
           bool look = false;
           if (c < T * nuw && part * 64 < min(seat.most, P.n - m * seat.most)) {
             const u64* w = a.chunks + ((size_t)(seat.base + m) * kTeamUpdWaves + part) * 4;
-            Wait wait;
             while (word_load(w + 2) != rebuilds)
-              if (wait.over(limit, status)) {
+              if (come.over(limit, status)) {
                 s_fail = 1;
                 break;
               }
@@ -514,6 +516,7 @@ k_team(TeamArgs a) {
           const u64 looks = __ballot(look);
           if (lane64 == 0) s_count[wave] = __popcll(looks);
           __syncthreads();
+          failed = failed || s_fail;
           int to = nrun;
           for (int w = 0; w < kWaves; ++w) {
             if (w < wave) to += s_count[w];
@@ -522,6 +525,12 @@ k_team(TeamArgs a) {
           if (look) l.scan.run[to + __popcll(looks & ((1ull << lane64) - 1ull))] = c;
           __syncthreads();
         }
+        // The roll call: nothing has been written, and no flag that the others
+        // would go on from.
+        if (failed) {
+          if (tid == 0) give_up(missed);
+          return;
+        }
         // their particles in marked cells
         constexpr int kAhead = 4;
         auto run_at = [&](int k, int& count) {  // first particle of the packing, and how many
@@ -529,9 +538,9 @@ k_team(TeamArgs a) {
           count = min(64, min(seat.most, P.n - m * seat.most) - part * 64);
           return m * seat.most + part * 64;
         };
+        Wait wait;
         for (int k0 = wave; k0 < nrun; k0 += kWaves * kAhead) {
           u64 wx[kAhead], wy[kAhead];
-          Wait wait;
           while (true) {
             bool all = true;
 #pragma unroll
@@ -584,6 +593,10 @@ k_team(TeamArgs a) {
         }
         __syncthreads();
         H = s_count[0];
+        if (s_fail) {  // (set again only after the next barrier)
+          if (tid == 0) give_up(missed);
+          return;
+        }
         if (own + H <= kCap) {
           for (int k = wave; k < nrun; k += kWaves) {
             const u64 m = l.scan.hit[k];
@@ -607,6 +620,10 @@ k_team(TeamArgs a) {
         }
       }
       __syncthreads();
+      if (s_fail) {
+        if (tid == 0) give_up(missed);
+        return;
+      }
       // rows: the list kernels' selection rule, a ballot placing the hits in
       // increasing local index
       cnt = 0;
@@ -636,11 +653,11 @@ k_team(TeamArgs a) {
       bool over = s_over != 0;
       if (T > 1) {
         if (tid == 0) put_flag(4 + (rebuilds & 1), rebuilds, over ? kFlagOver : 0);
-        gather_flags(4 + (rebuilds & 1), rebuilds, kStall);
+        gather_flags(4 + (rebuilds & 1), rebuilds, limit);
         __syncthreads();
         over = (s_bits & kFlagOver) != 0;
         if (s_fail) {
-          if (tid == 0) give_up(pass == 0 ? kTeamAbsent : kTeamStalled);
+          if (tid == 0) give_up(missed);
           return;
         }
       }
@@ -965,8 +982,8 @@ k_team(TeamArgs a) {
     ++xch;
     __syncthreads();  // new coordinates, s_need, s_next and s_fail visible
     if (!kHeun) {
-      if (s_fail) {
-        if (tid == 0) give_up(pass == 0 ? kTeamAbsent : kTeamStalled);
+      if (s_fail) {  // (in the first pass too: others may have the sums, and finish)
+        if (tid == 0) give_up(kTeamStalled);
         return;
       }
       const int next = s_next;

@@ -66,6 +66,7 @@ def load():
         "sc_set_contact_model": ([sysp, C.c_int], C.c_int),
         "sc_set_graphs": ([sysp, C.c_int], C.c_int),
         "sc_set_small_fire": ([sysp, C.c_int, C.c_int], C.c_int),
+        "sc_set_team_wait": ([sysp, C.c_double], C.c_int),
         "sc_team_info": ([sysp, C.POINTER(C.c_longlong), _ip], C.c_int),
         "sc_get_contact_model": ([sysp, _ip], C.c_int),
         "sc_set_tiling": ([sysp, C.c_int, C.c_int], C.c_int),
@@ -349,6 +350,11 @@ class System:
         (0); at most steps_per_launch minimiser iterations per launch (0: the
         default, 50000)."""
         self._ck(self.lib.sc_set_small_fire(self.h, int(max_particles), int(steps_per_launch)))
+
+    def set_team_wait(self, seconds):
+        """Longest wait of a team launch's workgroups for each other to become
+        resident; also ends the time without teams after a wait in vain."""
+        self._ck(self.lib.sc_set_team_wait(self.h, float(seconds)))
 
     def team_info(self):
         """(team launches so far, status bits of the last one: SC_TEAM_*)."""

@@ -175,3 +175,43 @@ def test_launches_go_on_after_a_team_in_the_middle():
     np.testing.assert_allclose(out[0][3], out[1][3], rtol=1e-6)
     side = np.concatenate([np.full(p.n, p.L) for p in packs])
     _same(out[0], out[1], side)
+
+
+def test_a_roll_call_in_vain():
+    """With no time to wait for each other, 256 workgroups leave at once and
+    unwritten (they do not come up within one look of the first): the calls give
+    what the launches per step give, bit for bit, and the next ones don't try."""
+    pk = _packing(16384, 4, phi=0.80)
+    params = native.fire_params(dt0=0.05, dt_max=0.5, max_move=0.02, ftol=1e-12, max_iter=20)
+    out = []
+    for small in (256, 0):
+        s = _system(pk, small)
+        try:
+            for name, run in (("fire", lambda: s.fire(params, check=False)),
+                              ("descent", lambda: s.gd_steps(20)),
+                              ("shear", lambda: s.strain_steps(40, 10))):
+                print("roll call,", name, small, flush=True)
+                s.set_positions(pk.x, pk.y, pk.phi)
+                s.set_dynamics(strain_rate=1e-3, step=0.005)
+                s.set_team_wait(0.0)
+                n = s.team_info()[0]
+                run()
+                got = [np.concatenate([*s.positions(), *s.forces()])]
+                if small:
+                    assert s.team_info() == (n + 1, native.SC_TEAM_ABSENT)
+                run()
+                got.append(np.concatenate([*s.positions(), *s.forces()]))
+                if small:
+                    assert s.team_info() == (n + 1, native.SC_TEAM_ABSENT)
+                out.append(got)
+            s.set_team_wait(0.2)
+            s.gd_steps(5)
+            assert s.team_info() == ((4, 0) if small else (0, 0))
+            for bad in (-0.1, 5.1, float("nan")):
+                with pytest.raises(native.SpherocylsError):
+                    s.set_team_wait(bad)
+        finally:
+            s.close()
+    for a, b in zip(out[:3], out[3:]):
+        for u, v in zip(a, b):
+            np.testing.assert_array_equal(u, v)
