@@ -207,14 +207,16 @@ k_team(TeamArgs a) {
   // Raised and read in phases separated by barriers, so that all threads leave
   // a loop together: s_need (own particles ask for a rebuild), s_bits (flags
   // gathered from the team), s_fail (a wait ran out), s_over (halo or row
-  // overflow), s_next (what the minimiser does next).
-  __shared__ int s_need, s_bits, s_fail, s_over, s_next;
+  // overflow), s_next (what the minimiser does next).  s_stop, of
+  // a single member: kFlagStop for this (the next) pass; by turns, since one
+  // update wavefront may be at the new positions before the other has looked.
+  __shared__ int s_need, s_bits, s_fail, s_over, s_next, s_stop[2];
   enum : int { kGoOn = 0, kDone = 1, kAgain = 2 };
   // A minimiser's state of iteration k in slot k & 1: thread 0 writes the next
   // iteration's while others still read this one's.
   __shared__ MinState s_m[2];
   __shared__ double s_frms;
-  __shared__ int s_end;
+  __shared__ int s_end;                     // MinStep::end; -1: stopped on such a coordinate
   __shared__ PackScal s_S;                  // thread 0's: Heun strain, and what goes back
   __shared__ u64 s_near[2];                 // rebuild: rows, columns of cells around own particles
   const int tid0 = threadIdx.x, lane64 = tid0 & 63, wave = tid0 >> 6;
@@ -266,7 +268,7 @@ k_team(TeamArgs a) {
     if (kHeun) l.rc[tid] = b.RC[gu];
   }
   if (tid == 0) {
-    s_need = s_bits = s_fail = s_over = s_next = s_end = 0;
+    s_need = s_bits = s_fail = s_over = s_next = s_end = s_stop[0] = s_stop[1] = 0;
     s_S = a.scal[pk];
     s_m[0] = min_state(s_S);
   }
@@ -821,7 +823,7 @@ k_team(TeamArgs a) {
           for (int w = 0; w < kWaves; ++w) s0 += s_part[w];
         }
       }
-      const int need = s_need;
+      const int need = *(T > 1 ? &s_need : &s_stop[pass & 1]);
       bool again = false, stop = (need & kFlagStop) != 0;
       if (nsum > 1) {
         u64* const cur = sums + (size_t)(xch % 3) * a.nseats * 4 * kTeamUpdWaves;
@@ -871,7 +873,10 @@ k_team(TeamArgs a) {
         s0 = kFire ? quad_sum(s0) : wave_sum(s0);
       }
       if (stop || again) {
-        if (tid == 0) s_next = stop ? kDone : kAgain;
+        if (tid == 0) {
+          s_next = stop ? kDone : kAgain;
+          if (stop) s_end = -1;
+        }
       } else {
         mark_empty(pass);  // all have read this pass's positions
         const MinState S0 = s_m[steps & 1];
@@ -947,6 +952,7 @@ k_team(TeamArgs a) {
       if (!okx || !oky || !isfinite(phi)) {
         atomicOr(a.err, kErrNonFinite);
         need = kFlagStop;
+        s_stop[(pass + 1) & 1] = kFlagStop;
       }
       if (!(kHeun && predicted)) {  // a predicted state stays unwrapped
         x = wx;
@@ -1031,13 +1037,14 @@ k_team(TeamArgs a) {
   }
   if (me == 0 && tid == 0) {
     if (!kHeun) {
-      const MinState& m = s_m[steps & 1];
+      // (a stop counted the iteration that it did not take)
+      const MinState& m = s_m[(steps - (s_end < 0 ? 1 : 0)) & 1];
       s_S.step = m.step;
       s_S.fire_dt = m.dt;
       s_S.fire_alpha = m.alpha;
       s_S.fire_npos = m.npos;
       s_S.prec = m.prec;
-      if (s_end) {
+      if (s_end > 0) {
         s_S.converged = s_end;
         s_S.iters = m.step;
         s_S.frms = s_frms;

@@ -215,3 +215,21 @@ def test_a_roll_call_in_vain():
     for a, b in zip(out[:3], out[3:]):
         for u, v in zip(a, b):
             np.testing.assert_array_equal(u, v)
+
+
+@pytest.mark.parametrize("n", [60, 128, 200, 700])
+def test_scalars_of_a_run_that_ends_non_finite(n):
+    """The first iteration raises the time step without bound and moves
+    particles out of the numbers; the run ends there, and the scalars are those
+    after that iteration, as the positions are."""
+    s = _system(_packing(n, 6), 256)
+    try:
+        print("non-finite", n, flush=True)
+        p = native.fire_params(dt0=0.01, dt_max=1e300, n_min=0, f_inc=1e200, max_move=0.02)
+        with pytest.raises(native.SpherocylsError, match="non-finite"):
+            s.fire(p)
+        assert s.team_info() == (1, 0)
+        b = s.box(0)
+        assert b["fire_dt"] == pytest.approx(1e198) and b["fire_alpha"] == pytest.approx(0.099)
+    finally:
+        s.close()
