@@ -138,13 +138,14 @@ int sc_set_small_fire(sc_system* s, int max_particles, int steps_per_launch);
  * differ by rounding from a team's), without another try for 20 s or until this
  * is called. */
 int sc_set_team_wait(sc_system* s, double seconds);
-/* Team launches of this system so far, and why the last one handed its steps
- * back to the launches per step (0: it did not).  Either may be NULL. */
+/* Team launches of this system so far, sheared steps that teams have taken, and
+ * why the last launch handed on to the launches per step (0: it did not).  Each
+ * may be NULL. */
 #define SC_TEAM_ABSENT 1   /* a workgroup was not resident in time; nothing was written */
 #define SC_TEAM_STALLED 2  /* a wait ran out later (the call returns SC_ERR_HIP) */
 #define SC_TEAM_NO_ROOM 4  /* a workgroup's neighbourhood or a row did not fit its LDS */
-#define SC_TEAM_OUTRAN 8   /* a sheared particle outran the rows */
-int sc_team_info(const sc_system* s, long long* launches, int* status);
+#define SC_TEAM_OUTRAN 8   /* a sheared particle outran the rows; its step is taken again */
+int sc_team_info(const sc_system* s, long long* launches, long long* sheared, int* status);
 int sc_get_contact_model(const sc_system* s, int* model);
 /* Force-pass implementation (no reference counterpart; both give the same
  * forces to rounding):

@@ -130,7 +130,9 @@ struct sc_system {
   TeamSeat* d_team_seats = nullptr;
   int* d_team_status = nullptr;
   int team_seat_cap = 0;
-  long long team_launches = 0;  // so far, and the last one's status bits (sc_team_info)
+  // team launches and sheared steps taken by them so far, the last launch's status
+  // bits (sc_team_info)
+  long long team_launches = 0, team_steps = 0;
   int team_status = 0;
   double team_wait = 0.2;  // seconds of a launch's roll call
   std::chrono::steady_clock::time_point team_off{};  // no team before this time
@@ -1336,9 +1338,10 @@ int sc_set_team_wait(sc_system* s, double seconds) {
   return SC_OK;
 }
 
-int sc_team_info(const sc_system* s, long long* launches, int* status) {
+int sc_team_info(const sc_system* s, long long* launches, long long* sheared, int* status) {
   if (!s) return SC_ERR_ARG;
   if (launches) *launches = s->team_launches;
+  if (sheared) *sheared = s->team_steps;
   if (status) *status = s->team_status;
   return SC_OK;
 }
@@ -1542,6 +1545,7 @@ int sc_strain_steps(sc_system* s, int nsteps, int se_every, double* se_out) {
       // states st .. upto - 1 that are recorded (never state 0)
       const int recs = se ? (upto - 1) / se_every - (st > 0 ? (st - 1) / se_every : 0) : 0;
       const int status = run_team(s, mode, plan, nullptr, upto - st, se_every, st, recs);
+      s->team_steps += s->scal[0].step - st;
       st = s->scal[0].step;
       if (status) break;
       if (st < nsteps) {

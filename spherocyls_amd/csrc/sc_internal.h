@@ -235,8 +235,8 @@ enum TeamMode : int { kTeamFire = 0, kTeamGd = 1, kTeamHeun = 2, kTeamHeunSe = 3
 enum TeamFlag : int { kFlagRebuild = 1, kFlagStop = 2, kFlagOver = 4, kFlagFast = 8 };
 constexpr int kTeamFlagSlots = 6;  // four of pass flags, two of rebuild flags
 // launch status: a member never came up (nothing was written); a wait ran out
-// later; a member's halo or a row did not fit (the state reached is written
-// back); a particle outran the rebuild of a Heun launch (nothing was written)
+// later; a member's halo or a row did not fit; a particle outran the rebuild of a
+// Heun launch (either way the state of the last whole step is written back)
 enum TeamStatus : int { kTeamAbsent = 1, kTeamStalled = 2, kTeamOver = 4, kTeamFast = 8 };
 // One workgroup: particles first .. first + count - 1 of the packing; member
 // `member` of its team of `team`, whose members are seats base .. base + team - 1.

@@ -30,8 +30,9 @@
 // pass has no exchange for it.  Heun steps have no team-wide exchange to
 // carry that: a member asks at 0.6 of the limit, all read the flags one pass
 // late, when they have long arrived, and a particle that reached the limit
-// before the rebuild makes the launch give up with nothing written (the host
-// then takes these steps with the launches per step).
+// before the rebuild makes the launch end at the start of the step whose forces
+// it missed, which every member still holds (the host goes on from there with
+// the launches per step).
 // Buffer reuse.  Positions of a pass are marked empty once every member is
 // known to have read them: in a minimiser when all sums of the pass are in, in
 // Heun two passes later, when all flags of the pass in between are in.  The
@@ -218,6 +219,7 @@ k_team(TeamArgs a) {
   __shared__ double s_frms;
   __shared__ int s_end;                     // MinStep::end; -1: stopped on such a coordinate
   __shared__ PackScal s_S;                  // thread 0's: Heun strain, and what goes back
+  __shared__ double s_gamma0, s_total0;     // thread 0's: Heun strain at the start of the step
   __shared__ u64 s_near[2];                 // rebuild: rows, columns of cells around own particles
   const int tid0 = threadIdx.x, lane64 = tid0 & 63, wave = tid0 >> 6;
   int tid = tid0;
@@ -406,6 +408,7 @@ k_team(TeamArgs a) {
   bool build = true;       // this pass starts with new rows (uniform over the team)
   bool was_built = false;  // Heun: the previous pass did
   bool predicted = false;  // Heun: the positions are a step's predicted ones
+  bool outran = false;     // Heun: the last pass's positions had outrun the rows
   if (wave < nuw) publish(0);
   if (kHeun && T > 1 && tid == 0) put_flag(0, 1, 0);
   __syncthreads();
@@ -430,10 +433,8 @@ k_team(TeamArgs a) {
       const int bits = T > 1 ? s_bits : s_need;
       if (bits & kFlagStop) break;  // a non-finite coordinate: the error word says so
       if (T > 1) {
-        if ((bits & kFlagFast) && !was_built) {
-          if (tid == 0) give_up(kTeamFast);
-          return;
-        }
+        outran = (bits & kFlagFast) && !was_built;
+        if (outran) break;
         build = build || ((bits & kFlagRebuild) && !was_built);
         if (pass >= 2 && wave < nuw) mark_empty(pass - 2);
       } else {
@@ -783,6 +784,8 @@ k_team(TeamArgs a) {
         if (tid == 0) {
           double gt = s_S.gamma_total + gd * dt;
           if (build && le_ratio == 1.0) gt = (double)(int)(gt + 1) + g2;
+          s_gamma0 = s_S.gamma;
+          s_total0 = s_S.gamma_total;
           s_S.gamma = g2;
           s_S.gamma_total = gt;
           s_S.step = s_S.step + 1;
@@ -1005,18 +1008,27 @@ k_team(TeamArgs a) {
     if (steps == a.max_steps && !predicted) break;
     if (kHeun && T > 1 && tid == 0) put_flag(pass & 3, (unsigned)pass + 1, s_need);
   }
-  if (kHeun && T > 1 && pass > 0 && !s_over && steps == a.max_steps) {
-    // the last evaluated pass had valid rows on every member
+  if (kHeun && T > 1 && !outran && steps == a.max_steps) {
+    // did the last evaluated pass have valid rows on every member?
     gather_flags((pass - 1) & 3, (unsigned)pass, kStall);
     __syncthreads();
-    if (s_fail || ((s_bits & kFlagFast) && !was_built)) {
-      if (tid == 0) give_up(s_fail ? kTeamStalled : kTeamFast);
+    if (s_fail) {
+      if (tid == 0) give_up(kTeamStalled);
       return;
     }
+    outran = (s_bits & kFlagFast) && !was_built;
   }
   __syncthreads();
+  if (kHeun && outran && tid == 0) {
+    give_up(kTeamFast);
+    if (!predicted) {  // the step was counted
+      s_S.gamma = s_gamma0;
+      s_S.gamma_total = s_total0;
+      s_S.step = s_S.step - 1;
+    }
+  }
   if (upd) {
-    const bool back = kHeun && predicted;  // left inside a step: to its start
+    const bool back = kHeun && (predicted || outran);  // to the start of the step
     const double x = back ? l.ox[tid] : l.x[tid], y = back ? l.oy[tid] : l.y[tid];
     const double phi = back ? l.op[tid] : l.phi[tid];
     double sn, cs;

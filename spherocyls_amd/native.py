@@ -67,7 +67,8 @@ def load():
         "sc_set_graphs": ([sysp, C.c_int], C.c_int),
         "sc_set_small_fire": ([sysp, C.c_int, C.c_int], C.c_int),
         "sc_set_team_wait": ([sysp, C.c_double], C.c_int),
-        "sc_team_info": ([sysp, C.POINTER(C.c_longlong), _ip], C.c_int),
+        "sc_team_info": ([sysp, C.POINTER(C.c_longlong), C.POINTER(C.c_longlong), _ip],
+                         C.c_int),
         "sc_get_contact_model": ([sysp, _ip], C.c_int),
         "sc_set_tiling": ([sysp, C.c_int, C.c_int], C.c_int),
         "sc_set_path": ([sysp, C.c_int], C.c_int),
@@ -359,8 +360,14 @@ class System:
     def team_info(self):
         """(team launches so far, status bits of the last one: SC_TEAM_*)."""
         n, st = C.c_longlong(), C.c_int()
-        self._ck(self.lib.sc_team_info(self.h, C.byref(n), C.byref(st)))
+        self._ck(self.lib.sc_team_info(self.h, C.byref(n), None, C.byref(st)))
         return n.value, st.value
+
+    def team_steps(self):
+        """Sheared steps taken by teams so far."""
+        n = C.c_longlong()
+        self._ck(self.lib.sc_team_info(self.h, None, C.byref(n), None))
+        return n.value
 
     def contact_model(self):
         m = C.c_int()

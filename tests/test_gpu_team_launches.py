@@ -233,3 +233,37 @@ def test_scalars_of_a_run_that_ends_non_finite(n):
         assert b["fire_dt"] == pytest.approx(1e198) and b["fire_alpha"] == pytest.approx(0.099)
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("n,rate,gamma,every", [
+    (512, 0.04, 0.0, 3), (512, 0.04, 0.3, 4), (4096, 0.03, 0.2, 1), (4096, 0.04, 0.24, 2),
+    (16384, 0.04, 0.0, 5), (16384, 0.03, 0.3, 0)])
+def test_steps_before_one_that_outran_the_rows_stay(n, rate, gamma, every):
+    """A relaxed packing sheared so fast that overlaps and speeds grow: the
+    launches per step go on from the last step whose rows held, with its strain
+    (before or across the remap at 0.5) and records."""
+    pk = _packing(n, 8, phi=0.84)
+    params = native.fire_params(dt0=0.05, dt_max=0.5, max_move=0.02, ftol=1e-9, max_iter=400)
+    steps, out = 24, []
+    for small in (256, 0):
+        print("outrun on the way", n, rate, gamma, small, flush=True)
+        s = _system(pk, 0)
+        try:
+            s.set_gamma(gamma, gamma)
+            s.fire(params, check=False)
+            s.set_small_fire(small)
+            s.set_dynamics(strain_rate=rate / 0.4, step=0.4)
+            se = s.strain_steps(steps, every)
+            if small:
+                print("steps of the team", s.team_steps(), flush=True)
+                assert s.team_info() == (1, native.SC_TEAM_OUTRAN)
+                assert 0 < s.team_steps() < steps
+            out.append((s.positions(), s.forces(), se, s.box(0)))
+        finally:
+            s.close()
+    _same(out[0], out[1], pk.L)
+    if every:
+        scale = np.abs(out[1][2]).max()
+        np.testing.assert_allclose(out[0][2], out[1][2], rtol=0, atol=TOL * scale)
+    for key in ("gamma", "gamma_total"):
+        assert out[0][3][key] == pytest.approx(out[1][3][key], abs=1e-13)
