@@ -280,19 +280,25 @@ k_team(TeamArgs a) {
   double gam = a.scal[pk].gamma, gam_eval = gam, center = gam;
   const double window = kHeun ? a.gamma_window : 0.0;
   const u64 kStall = 500000000ull;  // 5 s
+  u64 limit = a.roll_call;          // of a rebuild's waits
+  int missed = kTeamAbsent;         // what one that runs out means
 
   auto record_of = [&](int j, int g) {
     return a.pos + ((size_t)(j & (kBufs - 1)) * a.ntot + g) * 4;
   };
   // Large teams move records word by word with four lanes to a record, so that
   // an instruction touches 16 whole records (512 bytes in a row) and not one
-  // word of 64: all members' words are under way at once (469 members' shear of
-  // 60k particles, 100 passes: 1.81 ms the other way, 1.70 this way; 256
-  // members' FIRE 4.21 and 4.13).  Small teams wait for one trip, which the way
-  // through LDS and the further rounds lengthen (16 members' descent 1.34 and
-  // 1.47 ms), and so do 256 members' sheared steps, whose passes wait for
-  // nothing else (1.47 and 1.58 ms).
-  const bool wide = T >= (kHeun ? 384 : 128);
+  // word of 64: all members' words are under way at once.  Small teams wait for
+  // one trip, which the way through LDS and the further rounds lengthen.  Record
+  // by record and word by word, ms: 200 sheared steps of 8192 particles (128
+  // members) 2.28 and 2.41, of 20000 (313) 3.33 and 3.33, of 24000 (375) 3.74
+  // and 3.46, of 32700 (511) 4.09 and 3.62; with 128 particles a member of 33000
+  // (258 members) 3.85 and 4.23, of 40000 (313) 4.44 and 4.39, of 60001 (469)
+  // 5.11 and 4.71.  150 steps of descent of 16384 (256) 1.51 and 1.54, of 24000
+  // 2.06 and 1.96.  FIRE, whose members all wait for all sums, gains earlier: 400
+  // iterations of 1000 (16) 4.51 and 4.54, of 8192 (128) 5.81 and 5.72, of 32700
+  // 9.25 and 8.58.
+  const bool wide = T >= (kFire ? 128 : 320);
   // publish this wavefront's own positions, which it has written to LDS, as
   // pass j's
   auto publish = [&](int j) {
@@ -417,16 +423,14 @@ k_team(TeamArgs a) {
     tid = opaque(tid0);
     gu = first + (upd ? tid : 0);
     const int p = opaque(p0);
-    const u64 limit = pass == 0 ? a.roll_call : kStall;
-    const int missed = pass == 0 ? kTeamAbsent : kTeamStalled;  // a wait that ran out
     // ---- positions of this pass
     if (T > 1) {
       if (kHeun && pass > 0) gather_flags((pass - 1) & 3, (unsigned)pass, kStall);
-      if (!build) fetch_halo(pass, H, limit);
+      if (!build) fetch_halo(pass, H, kStall);  // (the first pass builds)
     }
     __syncthreads();
     if (s_fail) {
-      if (tid == 0) give_up(missed);
+      if (tid == 0) give_up(kTeamStalled);
       return;
     }
     if (kHeun) {
@@ -1005,6 +1009,8 @@ k_team(TeamArgs a) {
     }
     was_built = built;
     ++pass;
+    limit = kStall;  // (everyone has come up)
+    missed = kTeamStalled;
     if (steps == a.max_steps && !predicted) break;
     if (kHeun && T > 1 && tid == 0) put_flag(pass & 3, (unsigned)pass + 1, s_need);
   }
