@@ -856,7 +856,8 @@ TeamFn team_kernel(int mode, bool two_point, bool mixed, int shape) {
    {{&k_team<kTeamHeunSe, false, false, H>, nullptr},                             \
     {&k_team<kTeamHeunSe, true, false, H>, nullptr}}}
   // [shape][mode][contact model][pair precision]
-  static const TeamFn table[kTeamShapes][4][2][2] = {SC_TEAM_SHAPE(0), SC_TEAM_SHAPE(1)};
+  static const TeamFn table[kTeamShapes][4][2][2] = {
+      SC_TEAM_SHAPE(0), SC_TEAM_SHAPE(1), {SC_TEAM_ROW(kTeamFire, 2)}};
 #undef SC_TEAM_SHAPE
 #undef SC_TEAM_ROW
   return table[shape][mode][two_point ? 1 : 0][mixed ? 1 : 0];
@@ -866,9 +867,9 @@ static_assert(kTeamAbsent == SC_TEAM_ABSENT && kTeamStalled == SC_TEAM_STALLED &
                   kTeamOver == SC_TEAM_NO_ROOM && kTeamFast == SC_TEAM_OUTRAN,
               "status bits of a team launch");
 
-// A device runs one team launch of this process at a time: two launches that
-// each hold part of the CUs would wait for each other.  Held from the launch
-// to its end.
+// A device runs one launch of this process with teams of several members at a
+// time: two launches that each hold part of the CUs would wait for each other.
+// Held from the launch to its end.
 constexpr int kMaxDevices = 64;
 std::mutex g_team_mu[kMaxDevices];
 
@@ -878,60 +879,73 @@ constexpr std::chrono::seconds kTeamOff{20};
 
 struct TeamPlan {
   int shape = 0;
+  bool exchange = false;  // some team has several members
   std::vector<TeamSeat> seats;
   size_t lds = 0;
 };
 
 // Seats for the packings in `want`: members of at most kTeamOwn[shape]
-// particles, of equal size within a packing, in the smallest shape whose
-// workgroups are all resident at once.  False when they do not fit.
+// particles, of equal size within a packing.  Teams of several members come
+// first and must all be resident at once; packings that are a single member wait
+// for nobody and may queue behind them, as many as there are.  False where the
+// launches per step go on.
+//   Up to 128 particles one member of shape 1 is as fast as two of 64 (two-point
+// FIRE of 128: 7.86 us an iteration either way) and waits for nobody; above,
+// smaller members have fewer pairs each (N = 700: 64 a member 8.7 us), so the
+// smallest shape whose members are resident is taken.  FIRE of packings of up to
+// 256 that fit neither way runs them as single members of shape 2.  300 mixed
+// iterations against the launches per step: 1000 packings of 100 7.3 and 12.2 ms,
+// 2000 of 64 9.4 and 20.8; in shape 2, 300 of 200 7.5 and 11.6, 1000 of 256 15.3
+// and 20.2; but 64 of 200, whose 256 members fit, 3.6 in shape 0 and, one
+// workgroup to a packing, 5.1.
 bool team_plan(sc_system* s, int mode, const std::vector<int>& want, TeamPlan& plan) {
-  if (s->path != SC_PATH_LIST || s->small_max <= 0 || s->device >= kMaxDevices || want.empty() ||
-      std::chrono::steady_clock::now() < s->team_off)
+  if (s->path != SC_PATH_LIST || s->small_max <= 0 || s->device >= kMaxDevices || want.empty())
     return false;
-  long particles = 0;
-  int cell_words = 0;
+  const bool waited = std::chrono::steady_clock::now() < s->team_off;
+  int cell_words = 0, most = 0, cu = 0;
   for (int k : want) {
-    particles += s->packs[k].n;
     cell_words = std::max(cell_words, (s->packs[k].rows * s->packs[k].cols + 31) / 32);
+    most = std::max(most, s->packs[k].n);
   }
-  int cu = 0;
   HIPCK(hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, s->device));
-  // Up to 128 particles one member of shape 1 is as fast as two of 64 (two-point
-  // FIRE of 128: 7.86 us an iteration either way) and waits for nobody; above,
-  // smaller members have fewer pairs each (N = 700: 64 a member 8.7 us).
-  int most = 0;
-  for (int k : want) most = std::max(most, s->packs[k].n);
+  auto seat = [&](int k, int own) {
+    const PackInfo& P = s->packs[k];
+    const int team = (P.n + own - 1) / own, per = (P.n + team - 1) / team;
+    const int base = (int)plan.seats.size();
+    for (int m = 0, at = 0; m < team; ++m, at += per)
+      plan.seats.push_back(
+          TeamSeat{k, P.poff + at, std::min(per, P.n - at), m, team, base, per, 0});
+  };
   for (int shape = most <= kTeamOwn[1] ? 1 : 0; shape < kTeamShapes; ++shape) {
     const int own = kTeamOwn[shape];
+    if (shape == 2 && (mode != kTeamFire || most > own)) continue;
+    // members of teams of several, and whether a rebuild's words (one for every
+    // run of 64 particles) fit
+    long members = 0;
+    bool fits = true;
+    for (int k : want) {
+      const int n = s->packs[k].n, team = (n + own - 1) / own, per = (n + team - 1) / team;
+      if (team > 1) members += team;
+      fits = fits && team * ((per + 63) / 64) <= 8 * own;
+    }
     const size_t lds = team_lds_bytes(shape, cell_words);
-    if (particles > (long)own * 4 * cu || lds + 1024 > (size_t)s->lds_max) continue;
+    if (!fits || (members > 0 && waited) || members > 4l * cu || lds + 1024 > (size_t)s->lds_max)
+      continue;
     TeamFn fn = team_kernel(mode, s->contact_model == SC_CONTACT_TWO_POINT,
                             s->prec == SC_PREC_MIXED, shape);
     HIPCK(hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     int per_cu = 0;
     HIPCK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kTeamThreads, lds));
-    const long room = (long)per_cu * cu;
+    if (per_cu < 1 || members > (long)per_cu * cu) continue;
     plan = TeamPlan{};
     plan.shape = shape;
     plan.lds = lds;
-    bool fits = true;
-    for (int k : want) {
-      const PackInfo& P = s->packs[k];
-      const int team = (P.n + own - 1) / own, per = (P.n + team - 1) / team;
-      // (a rebuild keeps a word for every run of 64 particles)
-      fits = (long)plan.seats.size() + team <= room && team * ((per + 63) / 64) <= 8 * own;
-      if (!fits) break;
-      const int base = (int)plan.seats.size();
-      int at = 0;
-      for (int m = 0; m < team; ++m) {
-        const int c = std::min(per, P.n - at);
-        plan.seats.push_back(TeamSeat{k, P.poff + at, c, m, team, base, per, 0});
-        at += c;
-      }
-    }
-    if (fits) return true;
+    plan.exchange = members > 0;
+    for (int several = 1; several >= 0; --several)
+      for (int k : want)
+        if ((s->packs[k].n > own) == (several == 1)) seat(k, own);
+    return true;
   }
   return false;
 }
@@ -942,9 +956,8 @@ bool team_plan(sc_system* s, int mode, const std::vector<int>& want, TeamPlan& p
 int run_team(sc_system* s, int mode, const TeamPlan& plan, const FireParams* fp, int max_steps,
              int se_every = 0, int step0 = 0, int nrec = 0) {
   const int nseats = (int)plan.seats.size();
-  if (!s->d_team_pos) {
+  if (plan.exchange && !s->d_team_pos)
     s->d_team_pos = s->dalloc<unsigned long long>((size_t)16 * s->ntot);
-  }
   if (nseats > s->team_seat_cap) {
     s->dfree(s->d_team_sums);
     s->dfree(s->d_team_flags);
@@ -993,9 +1006,12 @@ int run_team(sc_system* s, int mode, const TeamPlan& plan, const FireParams* fp,
                           s->prec == SC_PREC_MIXED, plan.shape);
   std::vector<int> words(nseats);
   {
-    std::lock_guard<std::mutex> lk(g_team_mu[s->device]);
-    hipLaunchKernelGGL(k_team_clear, dim3(std::min(1024, grid_for(16 * s->ntot, 256))), dim3(256),
-                       0, s->stream, a);
+    std::unique_lock<std::mutex> lk(g_team_mu[s->device], std::defer_lock);
+    if (plan.exchange) {
+      lk.lock();
+      hipLaunchKernelGGL(k_team_clear, dim3(std::min(1024, grid_for(16 * s->ntot, 256))),
+                         dim3(256), 0, s->stream, a);
+    }
     {
       KernelTimer t(s, mode >= kTeamHeun ? SC_KERNEL_PREDICT : SC_KERNEL_FIRE_FORCE);
       hipLaunchKernelGGL(fn, dim3(nseats), dim3(kTeamThreads), plan.lds, s->stream, a);
@@ -1863,8 +1879,8 @@ int sc_fire_minimize(sc_system* s, const double* params, double switch_frms, int
       alloc_pblocks(s);
     }
   };
-  // Once the workgroups of all packings still running fit the GPU together,
-  // they run as teams, many iterations in one launch.  List path only: a
+  // Once all packings still running can be seated (team_plan), they run as
+  // teams, many iterations in one launch.  List path only: a
   // team's rows hold as many partners as the list kernels' (64) and are chosen
   // by a rule no wider than theirs, so it stops with SC_ERR_LIST_OVERFLOW only
   // where they would.
@@ -1883,9 +1899,10 @@ int sc_fire_minimize(sc_system* s, const double* params, double switch_frms, int
     was_team = team;
     if (team) {
       // CUs left idle by finished packings: back to the host for a new plan
-      // before long
+      // before long, unless the plan would be the same
       int steps = s->small_steps;
-      if (active.size() > 1) steps = std::min(steps, 128);
+      if (active.size() > 1 && plan.exchange) steps = std::min(steps, 128);
+      else if (active.size() > 1 && plan.shape == 2) steps = std::min(steps, 1024);
       const int st = run_team(s, kTeamFire, plan, &fp, steps);
       if (st & (kTeamAbsent | kTeamOver)) teams = false;
     } else if (graph) {
@@ -1903,9 +1920,10 @@ int sc_fire_minimize(sc_system* s, const double* params, double switch_frms, int
         }
       }
     }
-    // the scalars come back with the error word: one synchronisation per chunk
-    HIPCK(hipMemcpyAsync(s->scal.data(), s->d_scal[s->cur_scal], sizeof(PackScal) * s->npack,
-                         hipMemcpyDeviceToHost, s->stream));
+    // the scalars come back with the error word (a team has brought them)
+    if (!team)
+      HIPCK(hipMemcpyAsync(s->scal.data(), s->d_scal[s->cur_scal], sizeof(PackScal) * s->npack,
+                           hipMemcpyDeviceToHost, s->stream));
     int e = check_errors(s);
     if (e != SC_OK) {
       s->velocity_live = false;

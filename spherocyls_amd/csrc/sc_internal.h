@@ -227,9 +227,10 @@ constexpr int kSmallMax = 256;
 constexpr int kTeamThreads = 512;
 constexpr int kTeamRow = kNbrCap;   // partners a particle's LDS row holds
 // Launch shapes: own particles of a member, and own + halo particles its LDS holds.
-constexpr int kTeamShapes = 2;
-constexpr int kTeamUpdWaves = 2;  // wavefronts that hold own particles, at most
-constexpr int kTeamOwn[kTeamShapes] = {64, 128}, kTeamCap[kTeamShapes] = {512, 768};
+// The last is FIRE's for packings that are a single member.
+constexpr int kTeamShapes = 3;
+constexpr int kTeamOwn[kTeamShapes] = {64, 128, 256}, kTeamCap[kTeamShapes] = {512, 768, 256};
+constexpr int kTeamUpdWaves = 2;  // wavefronts that hold own particles of a team of several
 enum TeamMode : int { kTeamFire = 0, kTeamGd = 1, kTeamHeun = 2, kTeamHeunSe = 3 };
 // bits of a member's flag word
 enum TeamFlag : int { kFlagRebuild = 1, kFlagStop = 2, kFlagOver = 4, kFlagFast = 8 };

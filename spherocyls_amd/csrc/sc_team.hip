@@ -43,8 +43,10 @@
 // Every wait is bounded.  The first pass's rebuild doubles as the roll call: a
 // member that is not resident within a.roll_call (another process's kernels
 // hold the CUs) makes the others leave without having written anything, and the
-// host goes on with the launches per step, for some time without another try.  The host launches at most as many workgroups as are
-// resident at once.
+// host goes on with the launches per step, for some time without another try.
+// The host launches at most as many members of teams of several as are resident
+// at once.  A packing that is a single member waits for nobody: any number of
+// them go in one launch, behind the others.
 //
 // Measured, all-gather of 4 words by G workgroups over all XCDs: 1.05 us (G = 2),
 // 1.5 (16), 1.8 (64), 2.0 (128), 2.8 (256); an empty kernel in a captured graph
@@ -143,12 +145,14 @@ struct TeamLds {
 // Bytes of dynamic LDS of a launch of shape `shape` over grids of up to
 // cell_words * 32 cells.
 size_t team_lds_bytes(int shape, int cell_words) {
-  const size_t fixed = shape == 0 ? sizeof(TeamLds<kTeamOwn[0], kTeamCap[0]>)
-                                  : sizeof(TeamLds<kTeamOwn[1], kTeamCap[1]>);
+  const size_t fixed = shape == 0   ? sizeof(TeamLds<kTeamOwn[0], kTeamCap[0]>)
+                       : shape == 1 ? sizeof(TeamLds<kTeamOwn[1], kTeamCap[1]>)
+                                    : sizeof(TeamLds<kTeamOwn[2], kTeamCap[2]>);
   return fixed + (size_t)cell_words * sizeof(unsigned);
 }
 
-// Empty marks for every word a launch polls, zero flags.
+// Empty marks for every word a launch polls, zero flags.  (A launch of single
+// members polls none, and needs none of it.)
 __global__ void k_team_clear(TeamArgs a) {
   const size_t np = (size_t)kBufs * a.ntot * 4, ns = (size_t)3 * a.nseats * 4 * kTeamUpdWaves,
                nf = (size_t)kTeamFlagSlots * a.nseats, nc = (size_t)a.nseats * 4 * kTeamUpdWaves;
@@ -226,6 +230,7 @@ k_team(TeamArgs a) {
   const TeamSeat seat = a.seats[blockIdx.x];
   const int pk = seat.pack, T = seat.team, me = seat.member;
   const PackInfo P = a.packs[pk];
+  if (T == 1 && tid0 == 0) a.status[seat.base] = 0;
   if (!kHeun && a.scal[pk].converged) return;  // the whole team
   const Bank& b = a.b;
   const int own = seat.count, first = seat.first;
@@ -811,9 +816,10 @@ k_team(TeamArgs a) {
     }
     if (T == 1 && kFire && nuw > 1) __syncthreads();
     if (!kHeun && wave < nuw) {
-      if (T == 1 && nuw > 1) {  // two update wavefronts of one member: through LDS
+      if (T == 1 && nuw > 1) {  // several update wavefronts of one member: through LDS
         if (kFire) {
-          s0 = s_part[lane64 & 3] + s_part[4 + (lane64 & 3)];
+          s0 = s_part[lane64 & 3];
+          for (int w = 1; w < nuw; ++w) s0 += s_part[4 * w + (lane64 & 3)];
         } else {
           s0 = 0.0;
           for (int w = 0; w < kWaves; ++w) s0 += s_part[w];
@@ -1074,6 +1080,7 @@ k_team(TeamArgs a) {
   template __global__ void k_team<kTeamHeunSe, true, false, H>(TeamArgs);
 SC_TEAM_INST_SHAPE(0)
 SC_TEAM_INST_SHAPE(1)
+SC_TEAM_INST(kTeamFire, 2)
 #undef SC_TEAM_INST_SHAPE
 #undef SC_TEAM_INST
 
