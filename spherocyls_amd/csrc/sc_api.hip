@@ -133,7 +133,7 @@ struct sc_system {
   // team launches and sheared steps taken by them so far, the last launch's status
   // bits (sc_team_info)
   long long team_launches = 0, team_steps = 0;
-  int team_status = 0;
+  int team_status = 0, team_err = 0;  // (and the error bits after it)
   double team_wait = 0.2;  // seconds of a launch's roll call
   std::chrono::steady_clock::time_point team_off{};  // no team before this time
   double* d_team_se = nullptr;
@@ -176,7 +176,7 @@ struct sc_system {
   double* d_pack_sum = nullptr;
   double* d_se_ring = nullptr;
   size_t se_ring_cap = 0;
-  int* d_err = nullptr;
+  int* d_err = nullptr;  // [2] error bits; status bits of a team launch
   double* d_io = nullptr;  // 3 * ntot staging for caller-order transfers
   int* d_export_q = nullptr;
   int* d_export_n = nullptr;
@@ -1004,7 +1004,7 @@ int run_team(sc_system* s, int mode, const TeamPlan& plan, const FireParams* fp,
   a.step0 = step0;
   TeamFn fn = team_kernel(mode, s->contact_model == SC_CONTACT_TWO_POINT,
                           s->prec == SC_PREC_MIXED, plan.shape);
-  std::vector<int> words(nseats);
+  int words[2] = {0, 0};
   {
     std::unique_lock<std::mutex> lk(g_team_mu[s->device], std::defer_lock);
     if (plan.exchange) {
@@ -1020,14 +1020,14 @@ int run_team(sc_system* s, int mode, const TeamPlan& plan, const FireParams* fp,
       hipLaunchKernelGGL(k_team_records, dim3(nrec), dim3(256), 0, s->stream, a, nseats,
                          s->d_se_ring + ((size_t)(step0 + se_every - 1) / se_every -
                                          (step0 > 0 ? 1 : 0)) * kNSe);
-    HIPCK(hipMemcpyAsync(words.data(), s->d_team_status, sizeof(int) * nseats,
-                         hipMemcpyDeviceToHost, s->stream));
+    HIPCK(hipMemcpyAsync(words, s->d_err, sizeof(words), hipMemcpyDeviceToHost, s->stream));
     HIPCK(hipMemcpyAsync(s->scal.data(), s->d_scal[s->cur_scal], sizeof(PackScal) * s->npack,
                          hipMemcpyDeviceToHost, s->stream));
     HIPCK(hipStreamSynchronize(s->stream));
   }
-  int status = 0;
-  for (int w : words) status |= w;
+  const int status = words[1];
+  s->team_err = words[0];
+  if (status) HIPCK(hipMemsetAsync(s->d_err + 1, 0, sizeof(int), s->stream));
   s->team_launches++;
   s->team_status = status;
   if (status & kTeamAbsent) s->team_off = std::chrono::steady_clock::now() + kTeamOff;
@@ -1035,6 +1035,9 @@ int run_team(sc_system* s, int mode, const TeamPlan& plan, const FireParams* fp,
   if (status & kTeamStalled) throw StatusError{SC_ERR_HIP, "a team of workgroups stalled"};
   return status;
 }
+
+// check_errors, after a team launch that brought the error bits along.
+int team_errors(sc_system* s) { return s->team_err || s->timing ? check_errors(s) : SC_OK; }
 
 // Cells and rows for the launches per step after a team launch.
 void leave_team(sc_system* s) {
@@ -1169,8 +1172,8 @@ int sc_system_create(sc_system** out, int device, int npack, const int* offsets,
     s->d_scal[1] = s->dalloc<PackScal>(npack);
     s->d_pack_sum = s->dalloc<double>((size_t)npack * kNSum);
     HIPCK(hipMemsetAsync(s->d_pack_sum, 0, sizeof(double) * npack * kNSum, s->stream));
-    s->d_err = s->dalloc<int>(1);
-    HIPCK(hipMemsetAsync(s->d_err, 0, sizeof(int), s->stream));
+    s->d_err = s->dalloc<int>(2);
+    HIPCK(hipMemsetAsync(s->d_err, 0, 2 * sizeof(int), s->stream));
     s->bank[0] = alloc_bank(s);
     s->bank[1] = alloc_bank(s);
     alloc_positions(s, s->d_px, s->d_py, s->d_pnx, s->d_pny);
@@ -1742,7 +1745,8 @@ int sc_gd_steps(sc_system* s, int nmax, double emin, int* steps_done) {
   TeamPlan plan;
   bool teams = team_plan(s, kTeamGd, every, plan);
   while (true) {
-    if (teams) {
+    const bool team = teams;
+    if (team) {
       if (run_team(s, kTeamGd, plan, &fp, s->small_steps)) {
         teams = false;
         leave_team(s);
@@ -1757,9 +1761,9 @@ int sc_gd_steps(sc_system* s, int nmax, double emin, int* steps_done) {
       launch_force(s, ps);
       launch_update(s, ps, fp, 0);
     }
-    int e = check_errors(s);
+    int e = team ? team_errors(s) : check_errors(s);
     if (e != SC_OK) return e;
-    download_scal(s);
+    if (!team) download_scal(s);
     bool all = true;
     for (auto& S : s->scal) all &= S.converged != 0;
     if (all) break;
@@ -1920,11 +1924,11 @@ int sc_fire_minimize(sc_system* s, const double* params, double switch_frms, int
         }
       }
     }
-    // the scalars come back with the error word (a team has brought them)
+    // the scalars come back with the error word (a team has brought both)
     if (!team)
       HIPCK(hipMemcpyAsync(s->scal.data(), s->d_scal[s->cur_scal], sizeof(PackScal) * s->npack,
                            hipMemcpyDeviceToHost, s->stream));
-    int e = check_errors(s);
+    int e = team ? team_errors(s) : check_errors(s);
     if (e != SC_OK) {
       s->velocity_live = false;
       s->compact = false;

@@ -255,8 +255,8 @@ struct TeamArgs {
   unsigned long long* sums;  // [3][nseats][kTeamUpdWaves][4]
   unsigned long long* flags; // [kTeamFlagSlots][nseats]
   unsigned long long* chunks;  // [nseats][kTeamUpdWaves][4] where 64 own particles are (rebuilds)
-  int* status;               // [nseats]: TeamStatus bits at a team's first seat
-  int* err;
+  int* status;               // [nseats]: kTeamAbsent, kTeamStalled at a team's first seat
+  int* err;                  // [2]: error bits; TeamStatus bits of the launch
   FireParams fire;
   double gamma_window;
   unsigned long long roll_call;  // ticks of 10 ns that members wait for each other to come up

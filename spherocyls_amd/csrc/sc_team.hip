@@ -409,7 +409,8 @@ k_team(TeamArgs a) {
     if (why == kTeamStalled &&
         (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kTeamAbsent))
       return;
-    atomicOr(status, why);
+    atomicOr(status, why);   // (for the team)
+    atomicOr(a.err + 1, why);  // (for the host)
   };
 
   int H = 0;    // halo entries
@@ -663,7 +664,7 @@ k_team(TeamArgs a) {
         }
       }
       if (over) {
-        if (tid == 0) atomicOr(status, kTeamOver);
+        if (tid == 0) atomicOr(a.err + 1, kTeamOver);
         break;  // the state of this pass is written back
       }
       build = false;
@@ -1021,7 +1022,7 @@ k_team(TeamArgs a) {
   }
   __syncthreads();
   if (kHeun && outran && tid == 0) {
-    give_up(kTeamFast);
+    atomicOr(a.err + 1, kTeamFast);
     if (!predicted) {  // the step was counted
       s_S.gamma = s_gamma0;
       s_S.gamma_total = s_total0;
