@@ -1557,7 +1557,13 @@ int sc_strain_steps(sc_system* s, int nsteps, int se_every, double* se_out) {
   const int mode = se ? kTeamHeunSe : kTeamHeun;
   const std::vector<int> only{0};
   TeamPlan plan;
-  if (s->npack == 1 && !s->timing && nsteps > 1 &&
+  // Short calls stay with the launches: a team builds rows when it comes and
+  // leaves cells and rows to be built when it goes, 60 us at 512 particles and
+  // 200 at 60 thousand.  Launches and team, us: 5 steps of 512 282 and 288, of
+  // 16384 298 and 317; 7 steps 345 and 308, 363 and 334; 10 steps of 32700 446 and
+  // 454, 15 598 and 534; 15 steps of 60001 617 and 679, 20 779 and 784, 30 1101
+  // and 1002.
+  if (s->npack == 1 && !s->timing && nsteps >= 6 + s->ntot / 4000 &&
       !(se && s->prec == SC_PREC_MIXED) && team_plan(s, mode, only, plan)) {
     while (st < nsteps) {
       const int upto = std::min(nsteps, st + 2 * resort_every);

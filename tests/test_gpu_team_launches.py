@@ -267,3 +267,27 @@ def test_steps_before_one_that_outran_the_rows_stay(n, rate, gamma, every):
         np.testing.assert_allclose(out[0][2], out[1][2], rtol=0, atol=TOL * scale)
     for key in ("gamma", "gamma_total"):
         assert out[0][3][key] == pytest.approx(out[1][3][key], abs=1e-13)
+
+
+@pytest.mark.parametrize("n,least", [(100, 6), (700, 6), (16384, 10), (60001, 21)])
+def test_short_sheared_calls_are_launched_step_by_step(n, least):
+    """A team's coming and going costs more than the first few steps save; calls
+    below the line are the launches per step, bit for bit."""
+    pk = _packing(n, 9, phi=0.7)
+    out = []
+    for small in (256, 0):
+        s = _system(pk, small)
+        try:
+            print("short", n, small, flush=True)
+            s.set_dynamics(strain_rate=1e-3, step=0.002)
+            for k in (1, 2, least - 1):
+                s.strain_steps(k, 2)
+            assert s.team_info() == (0, 0)
+            out.append((s.positions(), s.forces()))
+            s.strain_steps(least)
+            assert s.team_info()[0] == (1 if small else 0)
+        finally:
+            s.close()
+    for a, b in zip(*out):
+        for u, v in zip(a, b):
+            np.testing.assert_array_equal(u, v)
