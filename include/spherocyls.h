@@ -119,14 +119,17 @@ int sc_set_contact_model(sc_system* s, int model);
  * (sc_timing_enable) always launches eagerly. */
 int sc_set_graphs(sc_system* s, int enable);
 /* Many steps in one launch (no reference counterpart; a launch choice like
- * sc_set_graphs).  max_particles > 0 (at most 256; the default) lets teams of
- * workgroups that stay resident run FIRE iterations, gradient-descent steps and
- * the sheared steps of a single packing on the list path, wherever the
- * workgroups of all packings still running fit the GPU together (a single
- * packing of about 60 thousand particles does); 0 launches kernels for every
- * step.  Same steps, decisions and stop rules, sums in another order: results
- * agree to rounding, not bit for bit.  A launch of a minimiser runs at most
- * steps_per_launch iterations (0: the default, 50000) and the packings still
+ * sc_set_graphs).  Teams of workgroups that stay resident run FIRE iterations,
+ * gradient-descent steps and the sheared steps of a single packing (but for
+ * calls of a few steps) on the list path, wherever the workgroups of all packings
+ * still running fit the GPU together (a single packing of about 60 thousand
+ * particles does); packings of up to 128 particles, 256 in FIRE, need one
+ * workgroup each, and any number of those fits.  max_particles from 1 to 255
+ * allows this only while every packing that the call still advances holds at most
+ * that many particles; 256, the default, whatever they hold; 0 launches kernels
+ * for every step.  Same steps, decisions and stop rules, sums in another order:
+ * results agree to rounding, not bit for bit.  A launch of a minimiser runs at
+ * most steps_per_launch iterations (0: the default, 50000) and the packings still
  * running are launched again, so no single kernel runs long.  With event timing
  * on, a minimiser's launch is counted under SC_KERNEL_FIRE_FORCE; sheared steps
  * are then launched one by one. */

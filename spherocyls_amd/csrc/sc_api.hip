@@ -122,7 +122,7 @@ struct sc_system {
   int prec = SC_PREC_FP64;
   int contact_model = SC_CONTACT_CLOSEST;
   bool use_graphs = true;
-  int small_max = kSmallMax;  // 0: no teams, launches for every step
+  int small_max = kSmallMax;  // particles of a packing in a team (kSmallMax: no limit, 0: none)
   int small_steps = 50000;    // minimiser iterations of a team launch, at most
   // teams (sc_team.hip): exchange words and the launch's seats
   unsigned long long *d_team_pos = nullptr, *d_team_sums = nullptr, *d_team_flags = nullptr,
@@ -907,6 +907,7 @@ bool team_plan(sc_system* s, int mode, const std::vector<int>& want, TeamPlan& p
     cell_words = std::max(cell_words, (s->packs[k].rows * s->packs[k].cols + 31) / 32);
     most = std::max(most, s->packs[k].n);
   }
+  if (s->small_max < kSmallMax && most > s->small_max) return false;
   HIPCK(hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, s->device));
   auto seat = [&](int k, int own) {
     const PackInfo& P = s->packs[k];

@@ -220,7 +220,7 @@ struct UpdateArgs {
   int fused;               // 1: reduce and decide here; 0: k_reduce already wrote red.scal_next
 };
 
-// Largest argument of sc_set_small_fire.
+// Largest argument of sc_set_small_fire, which sets no limit.
 constexpr int kSmallMax = 256;
 
 // Teams of workgroups that run many steps in one launch (sc_team.hip).

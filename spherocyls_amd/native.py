@@ -347,9 +347,10 @@ class System:
 
     def set_small_fire(self, max_particles, steps_per_launch=0):
         """Teams of workgroups that run many steps in one launch, where they fit
-        the GPU (max_particles > 0, at most 256), or launches for every step
-        (0); at most steps_per_launch minimiser iterations per launch (0: the
-        default, 50000)."""
+        the GPU: for packings of any size (256, the default), only while every
+        packing still advanced holds at most max_particles (1 to 255), or never,
+        with launches for every step (0); at most steps_per_launch minimiser
+        iterations per launch (0: the default, 50000)."""
         self._ck(self.lib.sc_set_small_fire(self.h, int(max_particles), int(steps_per_launch)))
 
     def set_team_wait(self, seconds):

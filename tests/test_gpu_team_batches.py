@@ -92,3 +92,23 @@ def test_threads_beside_each_other():
         for (pa, fa), (pb, fb) in zip(a[0], b[0]):
             for u, v in zip((*pa, *fa), (*pb, *fb)):
                 np.testing.assert_array_equal(u, v)
+
+
+def test_limit_on_the_size():
+    """Below 256 the limit is a number of particles of every packing still
+    advanced; at 256 there is none."""
+    for sizes, limit, launches in (((100,), 99, 0), ((100,), 100, 1), ((60, 100), 64, 0),
+                                   ((60, 64), 64, 1), ((700,), 255, 0), ((700,), 256, 1)):
+        for call in ("fire", "descent"):
+            print("limit", sizes, limit, call, flush=True)
+            _, info = _run(_packs(sizes), limit, (call,))
+            assert info == (launches, 0)
+    s = native.System(_packs((300,)), pads=0.1)
+    try:
+        s.set_dynamics(strain_rate=1e-3, step=0.005)
+        for limit, launches in ((200, 0), (255, 0), (256, 1)):
+            s.set_small_fire(limit)
+            s.strain_steps(50)
+            assert s.team_info()[0] == launches
+    finally:
+        s.close()
