@@ -2216,9 +2216,16 @@ int sc_autotune(sc_system* s, int reps, int* path_out, int* tile_cols_out, int* 
       score[ci] = std::min(score[ci], 1e3 * ms / reps);
     }
   }
+  // Sheared steps of a packing that runs as a team are none of these passes, but
+  // take the list path (a step of 128 or 4096 particles 9.4 us; two passes of the
+  // tile path, the fastest there, 27 and 34): it stays, with the shape of its
+  // fastest pass.
+  sc_set_path(s, SC_PATH_LIST);
+  TeamPlan plan;
+  const bool list_only = s->npack == 1 && team_plan(s, kTeamHeun, {0}, plan);
   size_t bi = 0;
   for (size_t ci = 1; ci < cands.size(); ++ci)
-    if (score[ci] < score[bi]) bi = ci;
+    if (score[ci] < score[bi] && !(list_only && cands[ci].path != SC_PATH_LIST)) bi = ci;
   const double best = score[bi];
   const Cand pick = cands[bi];
   (void)hipEventDestroy(e0);
@@ -2247,6 +2254,16 @@ int sc_autotune_fire(sc_system* s, const double* params, double switch_frms, int
   std::vector<Cand> cands;
   for (int lanes : {1, 2, 4, 8})
     for (int blk : {64, 128, 256}) cands.push_back({SC_PATH_LIST, 0, blk, lanes});
+  // A team takes no notice of these shapes: they are tried by launches per step,
+  // and the system's own teams once a round, as the candidate after them (with
+  // the best shape so far for what a team leaves to the launches).
+  struct Teams {
+    sc_system* s;
+    int small_max;
+    ~Teams() { s->small_max = small_max; }
+  } teams{s, s->small_max};
+  const size_t nlist = cands.size();
+  if (teams.small_max > 0) cands.push_back({SC_PATH_LIST, 0, 0, 0});
   for (Cand c : {Cand{SC_PATH_TILE, 8, 128, 0}, Cand{SC_PATH_TILE, 12, 128, 0},
                  Cand{SC_PATH_TILE, 16, 256, 0}})
     cands.push_back(c);
@@ -2261,7 +2278,15 @@ int sc_autotune_fire(sc_system* s, const double* params, double switch_frms, int
   std::vector<double> score(cands.size(), 1e300);
   for (int round = 0; round < 2; ++round) {
     for (size_t ci = 0; ci < cands.size(); ++ci) {
-      const Cand& c = cands[ci];
+      Cand& c = cands[ci];
+      const bool team = ci == nlist && teams.small_max > 0;
+      s->small_max = team ? teams.small_max : 0;
+      if (team) {
+        const Cand& shape = cands[std::min_element(score.begin(), score.begin() + nlist) -
+                                  score.begin()];
+        c.block = shape.block;
+        c.lanes = shape.lanes;
+      }
       if (c.path == SC_PATH_TILE) {
         if (tile_lds_bytes(3 * (c.tile + 2) * s->cap, c.block / kLanes, c.block) > (size_t)s->lds_max)
           continue;

@@ -291,3 +291,41 @@ def test_short_sheared_calls_are_launched_step_by_step(n, least):
     for a, b in zip(*out):
         for u, v in zip(a, b):
             np.testing.assert_array_equal(u, v)
+
+
+@pytest.mark.parametrize("n", [128, 4096])
+def test_autotuner_keeps_the_path_of_teams(n):
+    """At these sizes a pass of the tile path is the fastest, but a team's
+    sheared step takes less than either path's two passes."""
+    s = _system(_packing(n, 5, phi=0.80), 256)
+    try:
+        print("autotune", n, flush=True)
+        assert s.autotune(reps=3)["path"] == "list"
+        s.set_dynamics(strain_rate=1e-3, step=0.005)
+        s.strain_steps(50)
+        assert s.team_info()[0] == 1
+    finally:
+        s.close()
+
+
+def test_fire_autotuner_tries_shapes_by_launches():
+    """Of the trials (two rounds) only the team's own are team launches; the
+    setting outlives them, also where a trial fails."""
+    pk = _packing(1000, 5)
+    s = _system(pk, 256)
+    try:
+        print("autotune_fire", flush=True)
+        got = s.autotune_fire(native.fire_params(ftol=1e-12), iterations=30)
+        assert s.team_info() == (2, 0) and got["path"] == "list" and got["shape"] in (1, 2, 4, 8)
+        s.gd_steps(5)
+        assert s.team_info() == (3, 0)
+        with pytest.raises(native.SpherocylsError):
+            s.autotune_fire(native.fire_params(max_move=0.06), iterations=10)
+        s.gd_steps(5)
+        assert s.team_info() == (4, 0)
+        s.set_small_fire(0)
+        s.autotune_fire(native.fire_params(ftol=1e-12), iterations=30)
+        s.gd_steps(5)
+        assert s.team_info() == (4, 0)
+    finally:
+        s.close()
