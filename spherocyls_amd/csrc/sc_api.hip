@@ -951,27 +951,49 @@ bool team_plan(sc_system* s, int mode, const std::vector<int>& want, TeamPlan& p
   return false;
 }
 
+// The device buffers of a launch; false when the GPU has no memory for them
+// (the launches per step need none of it).  A buffer that could not be renewed
+// is gone, and its capacity with it.
+bool team_buffers(sc_system* s, const TeamPlan& plan, int nrec) {
+  auto renew = [&](auto*& p, size_t count) {
+    s->dfree(p);
+    p = nullptr;
+    p = s->dalloc<std::remove_reference_t<decltype(*p)>>(count);
+  };
+  const int nseats = (int)plan.seats.size();
+  const size_t nse = (size_t)nrec * nseats * kNSe;
+  try {
+    if (plan.exchange && !s->d_team_pos) renew(s->d_team_pos, (size_t)16 * s->ntot);
+    if (nseats > s->team_seat_cap) {
+      s->team_seat_cap = 0;
+      renew(s->d_team_status, nseats);
+      renew(s->d_team_sums, (size_t)12 * kTeamUpdWaves * nseats);
+      renew(s->d_team_flags, (size_t)kTeamFlagSlots * nseats);
+      renew(s->d_team_chunks, (size_t)4 * kTeamUpdWaves * nseats);
+      renew(s->d_team_seats, nseats);
+      s->team_seat_cap = nseats;
+    }
+    if (nse > s->team_se_cap) {
+      s->team_se_cap = 0;
+      renew(s->d_team_se, nse);
+      s->team_se_cap = nse;
+    }
+  } catch (const HipError& e) {
+    if (e.e != hipErrorOutOfMemory) throw;
+    (void)hipGetLastError();
+    return false;
+  }
+  return true;
+}
+
 // One team launch of at most max_steps iterations or steps, waited for.
 // Returns the launch's status bits (TeamStatus); the scalars are advanced in
 // place, and rows and cells no longer match the moved particles.
 int run_team(sc_system* s, int mode, const TeamPlan& plan, const FireParams* fp, int max_steps,
              int se_every = 0, int step0 = 0, int nrec = 0) {
   const int nseats = (int)plan.seats.size();
-  if (plan.exchange && !s->d_team_pos)
-    s->d_team_pos = s->dalloc<unsigned long long>((size_t)16 * s->ntot);
-  if (nseats > s->team_seat_cap) {
-    s->dfree(s->d_team_sums);
-    s->dfree(s->d_team_flags);
-    s->dfree(s->d_team_chunks);
-    s->dfree(s->d_team_seats);
-    s->dfree(s->d_team_status);
-    s->d_team_status = s->dalloc<int>(nseats);
-    s->d_team_sums = s->dalloc<unsigned long long>((size_t)12 * kTeamUpdWaves * nseats);
-    s->d_team_flags = s->dalloc<unsigned long long>((size_t)kTeamFlagSlots * nseats);
-    s->d_team_chunks = s->dalloc<unsigned long long>((size_t)4 * kTeamUpdWaves * nseats);
-    s->d_team_seats = s->dalloc<TeamSeat>(nseats);
-    s->team_seat_cap = nseats;
-  }
+  s->team_err = 0;
+  if (!team_buffers(s, plan, nrec)) return kTeamAbsent;
   HIPCK(hipMemcpyAsync(s->d_team_seats, plan.seats.data(), sizeof(TeamSeat) * nseats,
                        hipMemcpyHostToDevice, s->stream));
   TeamArgs a{};
@@ -991,15 +1013,7 @@ int run_team(sc_system* s, int mode, const TeamPlan& plan, const FireParams* fp,
   a.ntot = s->ntot;
   a.nseats = nseats;
   a.max_steps = max_steps;
-  if (nrec > 0) {  // records of the states before the launch's steps, step 0 excepted
-    const size_t need = (size_t)nrec * nseats * kNSe;
-    if (need > s->team_se_cap) {
-      s->dfree(s->d_team_se);
-      s->d_team_se = s->dalloc<double>(need);
-      s->team_se_cap = need;
-    }
-    a.se_part = s->d_team_se;
-  }
+  a.se_part = s->d_team_se;  // records of the states before the launch's steps but the call's first
   a.se_every = std::max(se_every, 1);
   a.se_first = step0 > 0 ? 1 : 0;
   a.step0 = step0;

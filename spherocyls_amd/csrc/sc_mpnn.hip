@@ -920,6 +920,7 @@ inline int blocks(size_t n, int b = 256) { return (int)((n + b - 1) / b); }
 template <class T>
 void realloc_dev(sc_mpnn* m, T*& p, size_t count) {
   void* q = p;
+  p = nullptr;
   m->dfree(q);
   p = m->template dalloc<T>(count);
 }
@@ -927,6 +928,7 @@ void realloc_dev(sc_mpnn* m, T*& p, size_t count) {
 void ensure_capacity(sc_mpnn* m, int n, int e) {
   if (n <= m->ncap && e <= m->ecap) return;
   const int nc = std::max(n, m->ncap), ec = std::max(e, m->ecap);
+  m->ncap = m->ecap = m->n = m->e = 0;  // until all of them are there
   realloc_dev(m, m->off, nc + 1);
   realloc_dev(m, m->src, ec);
   realloc_dev(m, m->dst, ec);
@@ -966,11 +968,13 @@ void ensure_incoming(sc_mpnn* m, int n, int e) {
   sc_mpnn::Incoming& in = m->in;
   if (!in.bad) in.bad = m->dalloc<int>(1);
   if (n > in.ncap) {
+    in.ncap = 0;
     realloc_dev(m, in.off, (size_t)n + 1);
     realloc_dev(m, in.nf, (size_t)n * kNodeFeat);
     in.ncap = n;
   }
   if (e > in.ecap) {
+    in.ecap = 0;
     realloc_dev(m, in.src, e);
     realloc_dev(m, in.dst, e);
     realloc_dev(m, in.rev, e);
