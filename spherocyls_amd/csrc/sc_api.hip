@@ -885,9 +885,9 @@ struct TeamPlan {
 };
 
 // Seats for the packings in `want`: members of at most kTeamOwn[shape]
-// particles, of equal size within a packing.  Teams of several members come
-// first and must all be resident at once; packings that are a single member wait
-// for nobody and may queue behind them, as many as there are.  False where the
+// particles, of equal size within a packing.  Teams of several members must all
+// be resident at once; packings that are a single member wait for nobody and may
+// queue behind them, as many as there are (then the teams come first).  False where the
 // launches per step go on.
 //   Up to 128 particles one member of shape 1 is as fast as two of 64 (two-point
 // FIRE of 128: 7.86 us an iteration either way) and waits for nobody; above,
@@ -920,13 +920,14 @@ bool team_plan(sc_system* s, int mode, const std::vector<int>& want, TeamPlan& p
   for (int shape = most <= kTeamOwn[1] ? 1 : 0; shape < kTeamShapes; ++shape) {
     const int own = kTeamOwn[shape];
     if (shape == 2 && (mode != kTeamFire || most > own)) continue;
-    // members of teams of several, and whether a rebuild's words (one for every
-    // run of 64 particles) fit
-    long members = 0;
+    // members of teams of several and of all, and whether a rebuild's words (one
+    // for every run of 64 particles) fit
+    long members = 0, all = 0;
     bool fits = true;
     for (int k : want) {
       const int n = s->packs[k].n, team = (n + own - 1) / own, per = (n + team - 1) / team;
       if (team > 1) members += team;
+      all += team;
       fits = fits && team * ((per + 63) / 64) <= 8 * own;
     }
     const size_t lds = team_lds_bytes(shape, cell_words);
@@ -943,9 +944,13 @@ bool team_plan(sc_system* s, int mode, const std::vector<int>& want, TeamPlan& p
     plan.shape = shape;
     plan.lds = lds;
     plan.exchange = members > 0;
-    for (int several = 1; several >= 0; --several)
-      for (int k : want)
-        if ((s->packs[k].n > own) == (several == 1)) seat(k, own);
+    if (members == 0 || all <= (long)per_cu * cu) {
+      for (int k : want) seat(k, own);
+    } else {
+      for (int several = 1; several >= 0; --several)
+        for (int k : want)
+          if ((s->packs[k].n > own) == (several == 1)) seat(k, own);
+    }
     return true;
   }
   return false;
