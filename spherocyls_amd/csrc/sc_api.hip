@@ -892,12 +892,12 @@ struct TeamPlan {
 //   Up to 128 particles one member of shape 1 is as fast as two of 64 (two-point
 // FIRE of 128: 7.86 us an iteration either way) and waits for nobody; above,
 // smaller members have fewer pairs each (N = 700: 64 a member 8.7 us), so the
-// smallest shape whose members are resident is taken.  FIRE of packings of up to
-// 256 that fit neither way runs them as single members of shape 2.  300 mixed
-// iterations against the launches per step: 1000 packings of 100 7.3 and 12.2 ms,
-// 2000 of 64 9.4 and 20.8; in shape 2, 300 of 200 7.5 and 11.6, 1000 of 256 15.3
-// and 20.2; but 64 of 200, whose 256 members fit, 3.6 in shape 0 and, one
-// workgroup to a packing, 5.1.
+// smallest shape whose members are resident is taken, but for FIRE of packings of
+// up to 256 that do not fit in shape 0: they run as single members of shape 2.
+// 300 mixed iterations, ms: 1000 packings of 100 by launches per step 12.2 and as
+// single members 7.1, 2000 of 64 20.8 and 9.2; 64 of 200 in shape 0 3.6, 200 of
+// 200 in shape 1 6.0 and in shape 2 4.8, 300 of 200 by launches 11.5 and in shape
+// 2 7.1, 1000 of 256 20.1 and 14.4.
 bool team_plan(sc_system* s, int mode, const std::vector<int>& want, TeamPlan& plan) {
   if (s->path != SC_PATH_LIST || s->small_max <= 0 || s->device >= kMaxDevices || want.empty())
     return false;
@@ -919,7 +919,8 @@ bool team_plan(sc_system* s, int mode, const std::vector<int>& want, TeamPlan& p
   };
   for (int shape = most <= kTeamOwn[1] ? 1 : 0; shape < kTeamShapes; ++shape) {
     const int own = kTeamOwn[shape];
-    if (shape == 2 && (mode != kTeamFire || most > own)) continue;
+    const bool whole = mode == kTeamFire && most <= kTeamOwn[2];  // shape 2 would do
+    if (shape == 2 ? !whole : shape == 1 && whole && most > own) continue;
     // members of teams of several and of all, and whether a rebuild's words (one
     // for every run of 64 particles) fit
     long members = 0, all = 0;
