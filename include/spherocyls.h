@@ -17,7 +17,8 @@
  *     the particles offsets[k] .. offsets[k+1]-1 of the concatenated arrays.  The
  *     reference's single box is a system with one packing.
  *   - One system per host thread; calls on one system are serialised on its own
- *     HIP stream.  No global mutable state is shared between systems.
+ *     HIP stream.  No global mutable state is shared between systems, but for a
+ *     lock per GPU: launches whose workgroups wait for each other take turns.
  */
 #ifndef SPHEROCYLS_H
 #define SPHEROCYLS_H

@@ -1913,8 +1913,9 @@ int sc_fire_minimize(sc_system* s, const double* params, double switch_frms, int
   // Once all packings still running can be seated (team_plan), they run as
   // teams, many iterations in one launch.  List path only: a
   // team's rows hold as many partners as the list kernels' (64) and are chosen
-  // by a rule no wider than theirs, so it stops with SC_ERR_LIST_OVERFLOW only
-  // where they would.
+  // by a rule no wider than theirs.  A team in which a row or a member's
+  // neighbourhood does not fit hands its state on to the launches, which alone
+  // report SC_ERR_LIST_OVERFLOW.
   std::vector<int> active;
   for (int k = 0; k < s->npack; ++k) active.push_back(k);
   bool teams = true, was_team = false;

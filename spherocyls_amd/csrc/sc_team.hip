@@ -50,13 +50,16 @@
 //
 // Measured, all-gather of 4 words by G workgroups over all XCDs: 1.05 us (G = 2),
 // 1.5 (16), 1.8 (64), 2.0 (128), 2.8 (256); an empty kernel in a captured graph
-// takes 1.65 us.  Against the launches per step, two-point FIRE iterations of
-// 16384 particles 19.1 -> 12.1 us, of 700 15.4 -> 9.8; sheared steps of 16384
-// 20.8 -> 14.6 us, of 512 14.3 -> 11.9; descent of 1000 16.4 -> 9.0.
-// Where a FIRE pass of 16384 (11 us, 26k cycles) goes: gathering the sums 7.6k,
-// pair math 3.0k, rebuilds 3.2k (22 in 381 passes; 4.4k when every member looked
-// at every particle), new positions 1.9k, halo 1.7k, row tests 1.3k, sums 0.9k,
-// decision 0.7k (1.8k by one thread on the whole record of scalars).
+// takes 1.65 us.  Against the launches per step, wall time of a long
+// call over its steps: two-point FIRE from a random start to convergence, 16384
+// particles 24.1 -> 12.4 us an iteration, 700 22.9 -> 9.7, 128 20.9 -> 8.2; sheared
+// steps of a relaxed packing of 16384 23.5 -> 10.6 us, of 512 and 700 21.3 -> 10.1;
+// descent of 1000 20.9 -> 8.0.
+// Where a FIRE iteration of 16384 goes in a compression step, which rebuilds less
+// often (10.9 us, 26k cycles): gathering the sums 7.6k, pair math 3.0k, rebuilds
+// 3.2k (22 in 381 passes; 4.4k when every member looked at every particle), new
+// positions 1.9k, halo 1.7k, row tests 1.3k, sums 0.9k, decision 0.7k (1.8k by one
+// thread on the whole record of scalars).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
