@@ -1770,11 +1770,13 @@ int sc_gd_steps(sc_system* s, int nmax, double emin, int* steps_done) {
   std::vector<int> every;
   for (int k = 0; k < s->npack; ++k) every.push_back(k);
   TeamPlan plan;
-  bool teams = team_plan(s, kTeamGd, every, plan);
+  bool teams = team_plan(s, kTeamGd, every, plan), teamed = false;
   while (true) {
     const bool team = teams;
     if (team) {
-      if (run_team(s, kTeamGd, plan, &fp, s->small_steps)) {
+      const int st = run_team(s, kTeamGd, plan, &fp, s->small_steps);
+      if (!(st & kTeamAbsent)) teamed = true;
+      if (st) {
         teams = false;
         leave_team(s);
       }
@@ -1799,9 +1801,12 @@ int sc_gd_steps(sc_system* s, int nmax, double emin, int* steps_done) {
   for (auto& S : s->scal) done = std::max(done, S.iters);
   if (steps_done) *steps_done = done;
   // positions are final; leave forces, energy and stress of the final state
-  // (the updates skip finished packings: fill every packing's cells first)
+  // (the updates skip finished packings: fill every packing's cells first; the
+  // force passes skip them too, and with them the rebuild that a team which gave
+  // up asked for: ask again)
   s->cur_buf = 0;
   bin_all_sized(s, 0, 0);
+  if (teamed) force_rebuild(s);
   force_pass(s, true, 0);
   return check_errors(s);
   API_END
@@ -1918,7 +1923,7 @@ int sc_fire_minimize(sc_system* s, const double* params, double switch_frms, int
   // report SC_ERR_LIST_OVERFLOW.
   std::vector<int> active;
   for (int k = 0; k < s->npack; ++k) active.push_back(k);
-  bool teams = true, was_team = false;
+  bool teams = true, was_team = false, teamed = false;
   TeamPlan plan;
   while (true) {
     const bool team = teams && team_plan(s, kTeamFire, active, plan);
@@ -1937,6 +1942,7 @@ int sc_fire_minimize(sc_system* s, const double* params, double switch_frms, int
       else if (active.size() > 1 && plan.shape == 2) steps = std::min(steps, 1024);
       const int st = run_team(s, kTeamFire, plan, &fp, steps);
       if (st & (kTeamAbsent | kTeamOver)) teams = false;
+      if (!(st & kTeamAbsent)) teamed = true;
     } else if (graph) {
       if (!g.exec) g.capture([&]() { iterations(chunk); });
       g.launch();
@@ -1995,11 +2001,14 @@ int sc_fire_minimize(sc_system* s, const double* params, double switch_frms, int
     if (s->scal[k].converged != 1) status = SC_ERR_NOT_CONVERGED;
   }
   // forces / energy / stress of the final state in FP64; the updates skip
-  // finished packings, so the cells of every packing are filled again first
+  // finished packings, so the cells of every packing are filled again first.
+  // The force passes skip them too, and with them the rebuild that followed a
+  // team or a re-sort while others went on: ask again.
   set_prec_all(s, kFP64);
   upload_scal(s);
   s->cur_buf = 0;
   bin_all_sized(s, 0, 0);
+  if (teamed || !graph) force_rebuild(s);
   force_pass(s, true, 0);
   int e = check_errors(s);
   download_scal(s);

@@ -329,3 +329,71 @@ def test_fire_autotuner_tries_shapes_by_launches():
         assert s.team_info() == (4, 0)
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_packings_that_finished_before_another_gave_up(precision):
+    """Of a batch only one packing runs out of room; the others finish in the
+    team, the launches per step then pass them over, and the final evaluation,
+    and the steps after it, are theirs too."""
+    packs = [_packing(300, 4), _packing(1000, 1, discs=2, radius=3.0), _packing(100, 5),
+             _packing(700, 6)]
+    params = native.fire_params(dt0=0.05, dt_max=0.5, max_move=0.02, ftol=1e-12, max_iter=60)
+    side = np.concatenate([np.full(p.n, p.L) for p in packs])
+    for name in ("fire", "descent"):
+        out = []
+        for small in (256, 0):
+            print("finished before,", name, precision, small, flush=True)
+            s = _system(packs, small)
+            try:
+                s.set_precision(precision)
+                s.set_dynamics(step=0.05)
+                if name == "fire":
+                    s.fire(params, check=False)
+                else:
+                    s.gd_steps(60)
+                assert s.team_info() == ((1, native.SC_TEAM_NO_ROOM) if small else (0, 0))
+                box = [s.box(k) for k in range(s.npack)]
+                out.append((s.positions(), s.forces(), box))
+                s.set_dynamics(strain_rate=1e-3, step=0.01)
+                s.strain_steps(3)
+                out.append((s.positions(), s.forces(), box))
+            finally:
+                s.close()
+        tol = TOL if precision == "fp64" else 1e-5  # (FP32 pairs: 6e-8 of a force a step)
+        for a, b in ((out[0], out[2]), (out[1], out[3])):
+            _same(a, b, side, tol)
+            for p, q in zip(a[2], b[2]):
+                assert q["ncontacts"] > 50 and p["ncontacts"] == pytest.approx(q["ncontacts"], abs=2)
+                assert p["E"] == pytest.approx(q["E"], rel=1e-3)
+
+
+def test_packings_that_finished_before_a_resort():
+    """Without graphs the launches per step re-sort the bank every 240
+    iterations; packings that had finished (two of these jammed discs', whose
+    descent has moved them far from their cells in the bank) keep their forces."""
+    packs = []
+    for n, phi, seed in ((60, 1.0, 1), (200, 1.1, 4), (400, 0.9, 6), (300, 0.88, 7)):
+        R, A = configs.bidisperse(n, aspect=1.0)
+        packs.append(configs.make_packing(R, A, phi, seed, f"N={n} phi {phi}"))
+    params = native.fire_params(dt0=0.05, dt_max=0.5, max_move=0.02, ftol=1e-4, max_iter=2000)
+    out = []
+    for graphs in (False, True):
+        print("re-sort", graphs, flush=True)
+        s = _system(packs, 0)
+        try:
+            s.set_graphs(graphs)
+            s.set_dynamics(step=0.1)
+            s.gd_steps(500)
+            it, _, _ = s.fire(params, check=False)
+            out.append((it, s.positions(), s.forces(), [s.box(k) for k in range(4)]))
+        finally:
+            s.close()
+    it = out[1][0]
+    assert it[0] < 240 and it[1] < 240 and it[2] > 270 and it[3] > 270
+    n = packs[0].n + packs[1].n  # (the re-sorted others' sums run in another order)
+    np.testing.assert_array_equal(out[0][0][:2], it[:2])
+    side = np.concatenate([np.full(p.n, p.L) for p in packs[:2]])
+    _same(*[([v[:n] for v in o[1]], [v[:n] for v in o[2]]) for o in out], side, 1e-7)
+    for p, q in zip(out[0][3][:2], out[1][3][:2]):
+        assert q["ncontacts"] > 100 and p["ncontacts"] == q["ncontacts"]
