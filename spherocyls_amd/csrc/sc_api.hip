@@ -43,7 +43,7 @@ size_t tile_lds_bytes(int cap, int groups, int nthr);
 template <int MODE, bool TWO_POINT, bool MIXED, int SHAPE>
 __global__ void k_team(TeamArgs a);
 __global__ void k_team_clear(TeamArgs a);
-__global__ void k_team_records(TeamArgs a, int team, double* out);
+__global__ void k_team_records(TeamArgs a, int team, double* out, double* pack_sum);
 size_t team_lds_bytes(int shape, int cell_words);
 constexpr int kExport = 64;
 }  // namespace sc
@@ -1040,7 +1040,8 @@ int run_team(sc_system* s, int mode, const TeamPlan& plan, const FireParams* fp,
     if (nrec > 0)
       hipLaunchKernelGGL(k_team_records, dim3(nrec), dim3(256), 0, s->stream, a, nseats,
                          s->d_se_ring + ((size_t)(step0 + se_every - 1) / se_every -
-                                         (step0 > 0 ? 1 : 0)) * kNSe);
+                                         (step0 > 0 ? 1 : 0)) * kNSe,
+                         s->d_pack_sum);
     HIPCK(hipMemcpyAsync(words, s->d_err, sizeof(words), hipMemcpyDeviceToHost, s->stream));
     HIPCK(hipMemcpyAsync(s->scal.data(), s->d_scal[s->cur_scal], sizeof(PackScal) * s->npack,
                          hipMemcpyDeviceToHost, s->stream));

@@ -176,7 +176,10 @@ __global__ void k_team_clear(TeamArgs a) {
 // a 28th of the members' loads (9 records of 256 members: 45 us by nine threads
 // alone, now 5.8).
 constexpr int kRecordRuns = 28;
-__global__ void __launch_bounds__(256) k_team_records(TeamArgs a, int team, double* out) {
+// pack_sum keeps the last record of a state that the launch has left behind (of
+// the state it ended at the host goes on to record, or to take again).
+__global__ void __launch_bounds__(256)
+    k_team_records(TeamArgs a, int team, double* out, double* pack_sum) {
   __shared__ double s_run[kRecordRuns * kNSe];
   const int r = blockIdx.x, t = threadIdx.x;
   const int run = t / kNSe, i = t - run * kNSe, per = (team + kRecordRuns - 1) / kRecordRuns;
@@ -195,6 +198,8 @@ __global__ void __launch_bounds__(256) k_team_records(TeamArgs a, int team, doub
   if (t == kSeE) v *= P.inv_2n;
   else if (t != kSeNc) v /= S.Lx * S.Ly;
   out[(size_t)r * kNSe + t] = v;
+  const int at = ((a.step0 + a.se_every - a.se_first) / a.se_every + r) * a.se_every;
+  if (at < S.step && at + a.se_every >= S.step) pack_sum[t] = v;
 }
 
 // MODE kTeamFire / kTeamGd: minimiser iterations (force pass, sums and

@@ -397,3 +397,27 @@ def test_packings_that_finished_before_a_resort():
     _same(*[([v[:n] for v in o[1]], [v[:n] for v in o[2]]) for o in out], side, 1e-7)
     for p, q in zip(out[0][3][:2], out[1][3][:2]):
         assert q["ncontacts"] > 100 and p["ncontacts"] == q["ncontacts"]
+
+
+@pytest.mark.parametrize("n,steps,every", [
+    (100, 50, 20), (700, 50, 50), (700, 50, 7), (700, 4100, 1900), (4096, 60, 59)])
+def test_the_box_keeps_the_last_record(n, steps, every):
+    """Energy and stress of the box after sheared steps are those of the last
+    recorded state (here of several launches, too)."""
+    pk = _packing(n, 8, phi=0.84)
+    out = []
+    for small in (256, 0):
+        print("last record", n, steps, every, small, flush=True)
+        s = _system(pk, 0)
+        try:
+            s.fire(native.fire_params(dt0=0.05, dt_max=0.5, max_move=0.02, max_iter=200), check=False)
+            s.set_small_fire(small)
+            s.set_dynamics(strain_rate=1e-4, step=0.01)
+            se = s.strain_steps(steps, every)
+            assert s.team_steps() == (steps if small else 0)
+            box = s.box(0)
+            out.append([box[k] for k in native.SE_FIELDS])
+            np.testing.assert_array_equal(out[-1], se[-1, 0])
+        finally:
+            s.close()
+    np.testing.assert_allclose(out[0], out[1], rtol=0, atol=1e-7 * np.abs(out[1][:-1]).max())
