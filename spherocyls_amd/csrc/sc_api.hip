@@ -1584,8 +1584,10 @@ int sc_strain_steps(sc_system* s, int nsteps, int se_every, double* se_out) {
   // 200 at 60 thousand.  Launches and team, us: 5 steps of 512 282 and 288, of
   // 16384 298 and 317; 7 steps 345 and 308, 363 and 334; 10 steps of 32700 446 and
   // 454, 15 598 and 534; 15 steps of 60001 617 and 679, 20 779 and 784, 30 1101
-  // and 1002.
-  if (s->npack == 1 && !s->timing && nsteps >= 6 + s->ntot / 4000 &&
+  // and 1002.  The line lies above those, where random overlapping packings, whose
+  // rows hold for a few steps only, are no slower either (10 steps of 16384 859
+  // and 902, 20 of 33000 1368 and 1452).
+  if (s->npack == 1 && !s->timing && nsteps >= 8 + s->ntot / 2500 &&
       !(se && s->prec == SC_PREC_MIXED) && team_plan(s, mode, only, plan)) {
     while (st < nsteps) {
       const int upto = std::min(nsteps, st + 2 * resort_every);

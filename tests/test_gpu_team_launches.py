@@ -269,7 +269,7 @@ def test_steps_before_one_that_outran_the_rows_stay(n, rate, gamma, every):
         assert out[0][3][key] == pytest.approx(out[1][3][key], abs=1e-13)
 
 
-@pytest.mark.parametrize("n,least", [(100, 6), (700, 6), (16384, 10), (60001, 21)])
+@pytest.mark.parametrize("n,least", [(100, 8), (700, 8), (16384, 14), (60001, 32)])
 def test_short_sheared_calls_are_launched_step_by_step(n, least):
     """A team's coming and going costs more than the first few steps save; calls
     below the line are the launches per step, bit for bit."""
