@@ -1943,6 +1943,8 @@ int sc_fire_minimize(sc_system* s, const double* params, double switch_frms, int
       int steps = s->small_steps;
       if (active.size() > 1 && plan.exchange) steps = std::min(steps, 128);
       else if (active.size() > 1 && plan.shape == 2) steps = std::min(steps, 1024);
+      else if (active.size() > 1)  // (about 60 ms: another thread's team waits 0.2 s for its CUs)
+        steps = std::min(steps, std::max(128, 8192 / (int)(1 + plan.seats.size() / 512)));
       const int st = run_team(s, kTeamFire, plan, &fp, steps);
       if (st & (kTeamAbsent | kTeamOver)) teams = false;
       if (!(st & kTeamAbsent)) teamed = true;
